@@ -188,6 +188,120 @@ __global__ void __launch_bounds__(256) index_scores_kernel(const float* __restri
     scores[row * score_stride + place] = g < limit ? rounded_product(total, scale) : -INFINITY;
 }
 
+// The same scores on the matrix cores, 128 columns: v_mfma_f32_32x32x2_f32 adds its two columns to the accumulator one after the
+// other, each as a fused multiply-add rounded to FP32 (denormals kept), so 64 of them in a row ARE the canonical chain, bit for bit
+// -- at 139 TFLOP/s measured for the instruction alone, against the 79 TFLOP/s of the vector units' FP32 FMAs without packing.
+//
+// A wave owns one row's queries (A operands, heads as the rows of the product; 64 registers a tile of 32 heads, held for all its
+// groups) and works 64 groups at a time: two tiles of 32 as B operands, whose lane takes the even columns of a key (lanes 0-31) or
+// the odd ones (32-63).  Four independent products are always in flight, so none waits for its accumulator.  The products leave a
+// lane half of a group's heads, in runs of four (C layout: head 8 (r / 4) + 4 (lane / 32) + r % 4); one exchange of half-waves a pair of
+// registers gives every lane all heads of one group, and the terms are formed and added in head order there: 0.2 of a percent of
+// the time.  What bounds it is the products: 256 rows x 8256 groups x 64 heads take 312 us (111 TFLOP/s) where the chains on the
+// vector units took 917; a decode row over 16250 groups 13 us where it took 94.
+typedef float floatx16 __attribute__((ext_vector_type(16)));
+template<int HT, bool BF16>
+__global__ void __launch_bounds__(64, 2) index_scores_matrix_kernel(const float* __restrict__ q, const void* __restrict__ keys, size_t key_batch_stride,
+                                                                     const float* __restrict__ weights, const int32_t* __restrict__ visible,
+                                                                     size_t groups, int heads, float scale, float* __restrict__ scores, size_t score_stride,
+                                                                     const int32_t* __restrict__ candidates, size_t blocks, size_t block, unsigned tiles) {
+    constexpr int DIM = 128, COLUMNS = BF16 ? 16 : 8, CHUNKS = DIM / COLUMNS;      // two 16-byte pieces of a key at a time
+    const size_t row = blockIdx.y;
+    const unsigned lane = threadIdx.x;
+    const int j = lane % 32, half = lane / 32;
+    const uint32_t odd = half ? 0xffffffffu : 0u, picked = half ? 0x07060c0cu : 0x05040c0cu;       // the lane's column of a pair: as a mask, as bytes of a word
+    const size_t scored = candidates ? blocks * block : groups;
+    const size_t first = size_t(blockIdx.x) * tiles * 64;
+    const int32_t* row_candidates = candidates ? candidates + row * blocks : nullptr;
+    const int32_t seen = visible[row];
+    const size_t limit = min(groups, size_t(seen > 0 ? seen : 0));
+    float qf[HT][DIM / 2], weight[HT];      // weight: lane i (and i + 32) holds head 32 ht + i's
+    #pragma unroll
+    for (int ht = 0; ht < HT; ++ht) {
+        const int head = 32 * ht + j;
+        const uint32_t real = head < heads ? 0xffffffffu : 0u;      // (a mask and no condition: every load is asked for before the first is waited for)
+        const uint4* from = reinterpret_cast<const uint4*>(q + (row * heads + min(head, heads - 1)) * DIM);
+        const uint32_t first_of_pair = real & ~odd, second_of_pair = real & odd;
+        #pragma unroll
+        for (int c = 0; c < DIM / 4; ++c) {
+            const uint4 x = from[c];
+            qf[ht][2 * c] = __uint_as_float((x.x & first_of_pair) | (x.y & second_of_pair));
+            qf[ht][2 * c + 1] = __uint_as_float((x.z & first_of_pair) | (x.w & second_of_pair));
+        }
+        weight[ht] = __uint_as_float(__float_as_uint(weights[row * heads + min(head, heads - 1)]) & real);
+    }
+    for (unsigned tile = 0; tile < tiles; ++tile) {
+        const size_t base = first + size_t(tile) * 64, place = base + lane;
+        if (base >= scored) break;
+        if (!row_candidates && base >= limit) {        // nothing of this tile is visible
+            if (place < scored) scores[row * score_stride + place] = -INFINITY;
+            continue;
+        }
+        const uint4* from[2];
+        #pragma unroll
+        for (int t = 0; t < 2; ++t) {
+            const size_t p = min(base + 32 * t + j, scored - 1);
+            const size_t g = min(row_candidates ? CandidateMap{row_candidates, block, groups}.group_at(p) : p, groups - 1);
+            from[t] = reinterpret_cast<const uint4*>(static_cast<const uint8_t*>(keys) + (row * key_batch_stride + g * DIM) * (BF16 ? 2 : 4));
+        }
+        floatx16 acc[HT][2];
+        #pragma unroll
+        for (int ht = 0; ht < HT; ++ht)
+            #pragma unroll
+            for (int t = 0; t < 2; ++t)
+                #pragma unroll
+                for (int r = 0; r < 16; ++r) acc[ht][t][r] = 0.0f;
+        uint4 piece[2][2];
+        #pragma unroll
+        for (int t = 0; t < 2; ++t) { piece[t][0] = from[t][0]; piece[t][1] = from[t][1]; }
+        #pragma unroll
+        for (int c = 0; c < CHUNKS; ++c) {
+            float k[2][COLUMNS / 2];                    // the lane's half of the chunk's columns
+            #pragma unroll
+            for (int t = 0; t < 2; ++t) {
+                const uint32_t words[8] = {piece[t][0].x, piece[t][0].y, piece[t][0].z, piece[t][0].w, piece[t][1].x, piece[t][1].y, piece[t][1].z, piece[t][1].w};
+                #pragma unroll
+                for (int i = 0; i < COLUMNS / 2; ++i)
+                    k[t][i] = __uint_as_float(BF16 ? __builtin_amdgcn_perm(words[i], 0u, picked) : (words[(2 * i) % 8] & ~odd) | (words[(2 * i + 1) % 8] & odd));
+            }
+            if (c + 1 < CHUNKS) {
+                #pragma unroll
+                for (int t = 0; t < 2; ++t) { piece[t][0] = from[t][2 * c + 2]; piece[t][1] = from[t][2 * c + 3]; }
+            }
+            #pragma unroll
+            for (int i = 0; i < COLUMNS / 2; ++i)
+                #pragma unroll
+                for (int ht = 0; ht < HT; ++ht)
+                    #pragma unroll
+                    for (int t = 0; t < 2; ++t)
+                        acc[ht][t] = __builtin_amdgcn_mfma_f32_32x32x2f32(qf[ht][c * (COLUMNS / 2) + i], k[t][i], acc[ht][t], 0, 0, 0);
+        }
+        float total = 0.0f;
+        #pragma unroll
+        for (int ht = 0; ht < HT; ++ht)
+            #pragma unroll
+            for (int run = 0; run < 4; ++run) {
+                float dots[8];
+                #pragma unroll
+                for (int i = 0; i < 4; ++i) {
+                    // lanes 0-31 take group tile 0, lanes 32-63 tile 1: the first result is heads 0-3 of the run, the second heads 4-7
+                    const auto swapped = __builtin_amdgcn_permlane32_swap(__float_as_uint(acc[ht][0][4 * run + i]), __float_as_uint(acc[ht][1][4 * run + i]), false, false);
+                    dots[i] = __uint_as_float(swapped[0]);
+                    dots[4 + i] = __uint_as_float(swapped[1]);
+                }
+                #pragma unroll
+                for (int i = 0; i < 8; ++i) {
+                    const float w = __uint_as_float(__builtin_amdgcn_readlane(__float_as_uint(weight[ht]), 8 * run + i));
+                    total = add_rounded_product(total, fmaxf(dots[i], 0.0f), w);
+                }
+            }
+        if (place < scored) {
+            const size_t g = row_candidates ? CandidateMap{row_candidates, block, groups}.group_at(place) : place;
+            scores[row * score_stride + place] = g < limit ? rounded_product(total, scale) : -INFINITY;
+        }
+    }
+}
+
 // ---- top-k -------------------------------------------------------------------------------------------------
 
 // A score as an unsigned key of the same order (the rule of reference gpu/ops.hpp:1766-1769): both zeros are one key, a
@@ -910,6 +1024,26 @@ void launch_scores(Device& d, const float* q, const void* keys, bool bf16, size_
                    size_t rows, size_t groups, size_t heads, size_t dim, float scale, float* scores, size_t score_stride,
                    const int32_t* candidates, size_t blocks, size_t block) {
     const size_t scored = candidates ? blocks * block : groups;
+    if (dim == 128 && (uintptr_t(q) | uintptr_t(keys)) % 16 == 0) {
+        // Waves are single workgroups, two a SIMD (eight a compute unit) at once.  A row's tiles of 64 groups are cut into equal runs,
+        // one a wave, so that the waves fill whole rounds of the card; a run costs its tiles and about one more for the row's queries.
+        // (256 rows x 129 tiles: runs of 17, one round, 312 us; 8, two and a bit, 364 us; 1, 401 us.)
+        const size_t row_tiles = (scored + 63) / 64, slots = 8 * size_t(d.compute_units);
+        size_t tiles = row_tiles, cost = SIZE_MAX;
+        for (size_t rounds = 1; rounds <= 8; ++rounds) {
+            const size_t runs = std::min(row_tiles, std::max<size_t>(1, rounds * slots / rows)), each = (row_tiles + runs - 1) / runs;
+            const size_t waited = (rows * ((row_tiles + each - 1) / each) + slots - 1) / slots * (each + 1);
+            if (waited < cost) { cost = waited; tiles = each; }
+        }
+        const dim3 grid(checked_blocks((row_tiles + tiles - 1) / tiles, 1), unsigned(rows));
+#define SD_SCORES(H, B) index_scores_matrix_kernel<H, B><<<grid, 64, 0, d.stream>>>(q, keys, key_batch_stride, weights, visible, groups, int(heads), scale, \
+                                                                                            scores, score_stride, candidates, blocks, block, unsigned(tiles))
+        if (heads <= 32) { if (bf16) SD_SCORES(1, true); else SD_SCORES(1, false); }
+        else { if (bf16) SD_SCORES(2, true); else SD_SCORES(2, false); }
+#undef SD_SCORES
+        SD_CHECK(hipGetLastError());
+        return;
+    }
     const dim3 grid(checked_blocks(scored), unsigned(rows));
 #define SD_SCORES(H, B) index_scores_kernel<H, B><<<grid, 256, 0, d.stream>>>(q, keys, key_batch_stride, weights, visible, groups, heads, dim, scale, \
                                                                               scores, score_stride, candidates, blocks, block)

@@ -610,3 +610,30 @@ def test_sparse_path_operands_off_16_byte_boundaries(gpu, oracle):
         close_enough(result[b], want[0], f"sequence {b}")
     for b in (qb, kb, wb, vb, indices, ab, lb, out):
         gpu.release(b)
+
+
+@pytest.mark.parametrize("heads,groups,rows", [(1, 1, 1), (31, 63, 2), (32, 64, 1), (33, 65, 3), (64, 300, 2), (64, 16500, 1), (32, 1030, 40), (64, 8200, 70)])
+def test_matrix_core_chains_are_the_canonical_scores(gpu, oracle, heads, groups, rows):
+    # 128 columns go through the FP32 matrix instruction: the same bits at the edges of its tiles (32 heads, 64 groups, several tiles a
+    # wave), with values whose products are denormal among them, nothing or everything visible, FP32 and BF16 keys
+    from straydog_amd.backend import tagged_bf16
+    rng = np.random.default_rng(heads * 100000 + groups)
+    q = (rng.standard_normal((rows, heads, 128)) * 2).astype(np.float32)
+    keys = rng.standard_normal((groups, 128)).astype(np.float32)
+    keys[::7] *= np.float32(2.0 ** -126)
+    keys[::5, ::3] = 0.0
+    key_bits, key_values = _bf16_round(oracle, keys)
+    weights = rng.standard_normal((rows, heads)).astype(np.float32)
+    visible = rng.integers(0, groups + 1, size=rows).astype(np.int32)
+    visible[0] = groups
+    if rows > 2:
+        visible[1:3] = (0, -3)
+    some = sorted(set(rng.integers(0, rows, size=3)) | {0, min(1, rows - 1)})        # rows the oracle restates
+    qb, wb, vb, kb, hb, out = gpu.upload(q), gpu.upload(weights), gpu.upload(visible), gpu.upload(keys), gpu.upload(key_bits), gpu.buffer(rows * groups * 4)
+    for pointer, values in ((kb.base(), keys), (tagged_bf16(hb.base()), key_values)):
+        gpu.index_scores(qb.base(), pointer, wb.base(), vb.base(), rows, groups, heads, 128, 0.0625, out.base())
+        got = _read(gpu, out, np.uint32, rows * groups).reshape(rows, groups)
+        want = oracle.index_scores(q[some], values, weights[some], visible[some], 0.0625)
+        assert np.array_equal(got[some], want.view(np.uint32))
+    for b in (qb, wb, vb, kb, hb, out):
+        gpu.release(b)
