@@ -131,6 +131,15 @@ void* workspace(Device& d, size_t bytes) {
     return d.workspace;
 }
 
+void* workspace_or_null(Device& d, size_t bytes) {
+    if (bytes > d.workspace_bytes) {
+        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+        SD_CHECK(hipStreamIsCapturing(d.stream, &capturing));
+        if (capturing != hipStreamCaptureStatusNone) return nullptr;
+    }
+    return workspace(d, bytes);
+}
+
 void op_span(Device& d, const void* pointer, size_t bytes, const char* what) {
     const uint8_t* at = static_cast<const uint8_t*>(pointer);
     std::lock_guard<std::mutex> lock(d.mutex);

@@ -142,6 +142,8 @@ void upload(Device& d, void* target, const void* data, size_t bytes);     // cal
 void download(Device& d, void* output, const void* source, size_t bytes);  // device -> caller memory, waits
 // A workspace of at least `bytes` that lives with the device; grows only outside graph capture.
 void* workspace(Device& d, size_t bytes);
+// The same, or null where it would have to grow while a graph is recorded: for ops that can also do without.
+void* workspace_or_null(Device& d, size_t bytes);
 // Recorded graphs hold the addresses of the library's own buffers: when one of them moves, the graphs recorded so far go.
 void drop_recorded_graphs(Device& d);
 

@@ -17,6 +17,11 @@ bool latent_gather_supported(uint64_t kdim, uint64_t vdim);
 uint64_t latent_gather_scratch(uint64_t batch, uint64_t k, uint64_t heads, uint64_t vdim);
 void latent_gather(Device& d, const void* q, const void* latents, const int32_t* selected, uint64_t batch, uint64_t groups, uint64_t k,
                    uint64_t heads, float scale, float* out, float* partial);
+bool latent_rows_supported(uint64_t dim, uint64_t raw_rows, uint64_t window, uint64_t compressed_rows, uint64_t selections, const void* q, const void* raw,
+                           const void* compressed, const void* out);
+void latent_rows(Device& d, const float* q, const float* raw, uint64_t raw_rows, const int32_t* positions, uint64_t window, const void* compressed, bool bf16,
+                 uint64_t compressed_rows, const int32_t* selected, uint64_t selections, const float* sinks, uint64_t rows, uint64_t heads, float scale,
+                 uint64_t pairs, const float* frequencies, const double2* turns, float* out);
 }
 
 namespace {
@@ -323,6 +328,12 @@ int sd_op_sparse_attention(void* handle, const float* q, const float* raw, uint6
         args.inverse = value.turns + value.turns_rows * value.turns_pairs;
     }
     value.turns_ready = false;
+    // rows of 512 columns: the matrix-core kernel (latent_rows.hip); the general one takes every other shape
+    if (latent_rows_supported(dim, raw_rows, window, compressed_rows, selections, q, raw, args.compressed, out)) {
+        latent_rows(value, q, raw, raw_rows, positions, window, args.compressed, state_bf16(compressed), compressed_rows, selected, selections, sinks, rows, heads, scale,
+                    args.pairs, frequencies, args.forward, out);
+        return 0;
+    }
     launch(value, args, size_t(rows), size_t(window + selections), state_bf16(compressed));
     SD_OP_END
 }

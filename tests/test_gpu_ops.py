@@ -637,3 +637,40 @@ def test_matrix_core_chains_are_the_canonical_scores(gpu, oracle, heads, groups,
         assert np.array_equal(got[some], want.view(np.uint32))
     for b in (qb, wb, vb, kb, hb, out):
         gpu.release(b)
+
+
+@pytest.mark.parametrize("rows,heads,window,raw_rows,selections,compressed,rope_dims", [
+    (1, 64, 128, 128, 512, 900, 64), (1, 16, 5, 8, 0, 0, 0), (2, 33, 31, 40, 33, 50, 128), (7, 64, 33, 300, 1, 1, 2), (3, 80, 128, 200, 100, 64, 64),
+    (200, 64, 128, 384, 70, 500, 64), (270, 20, 16, 300, 31, 40, 0)])
+def test_latent_rows_on_the_matrix_cores(gpu, oracle, rows, heads, window, raw_rows, selections, compressed, rope_dims):
+    # rows of 512 columns: runs of steps merged and outputs finished in place, ragged heads, windows that have not filled yet or wrap, no
+    # selection at all, entries that name no row; the bound is FP32's: 512-column chains and sums of up to 640 weights of order one
+    # (the general kernel's difference from the oracle on these is 2e-6)
+    from straydog_amd.backend import tagged_bf16
+    rng = np.random.default_rng(rows * 1000 + heads)
+    dim = 512
+    q = rng.standard_normal((rows, heads, dim)).astype(np.float32) * 2
+    raw = rng.standard_normal((raw_rows, dim)).astype(np.float32)
+    bits, values = _bf16_round(oracle, rng.standard_normal((max(compressed, 1), dim)).astype(np.float32))
+    wide = rng.standard_normal((max(compressed, 1), dim)).astype(np.float32)
+    positions = (rng.integers(0, 3, size=rows) * 200 + np.arange(rows)).astype(np.int32)
+    selected = rng.integers(-2, max(compressed, 1), size=(rows, max(selections, 1))).astype(np.int32)
+    sinks = (rng.standard_normal(heads) * 3).astype(np.float32)
+    freqs = (1.6e5 ** (-(2.0 * np.arange(max(rope_dims // 2, 1))) / max(rope_dims, 1))).astype(np.float32)
+    scale = float(1.0 / np.sqrt(dim))
+    qb, rb, pb, sb, kb, fb = (gpu.upload(x) for x in (q, raw, positions, selected, sinks, freqs))
+    hb, vb, wb = gpu.upload(bits), gpu.upload(values), gpu.upload(wide)
+    out = gpu.buffer(q.size * 4)
+    results = []
+    for pointer in (tagged_bf16(hb.base()), vb.base(), wb.base()):
+        gpu.sparse_attention(qb.base(), rb.base(), raw_rows, pb.base(), window, pointer, compressed, sb.base(), selections, kb.base(), rows, heads, dim, scale,
+                             rope_dims, fb.base() if rope_dims else None, None, out.base())
+        results.append(_read(gpu, out, np.float32, q.size).reshape(q.shape))
+    assert np.array_equal(results[0].view(np.uint32), results[1].view(np.uint32)), "BF16 rows and their FP32 values differ"
+    some = sorted(set(rng.integers(0, rows, size=6)) | {0, rows - 1})
+    for got, table in ((results[0], values), (results[2], wide)):
+        chosen = np.where(selected[some] < 0, -1, selected[some]) if selections else np.zeros((len(some), 0), np.int32)
+        _, want = oracle.latent_attention(q[some], raw, positions[some], window, table, chosen, sinks, dim, scale, rope_dims, freqs if rope_dims else None, wide=True)
+        assert np.abs(got[some] - want).max() < 1e-5
+    for b in (qb, rb, pb, sb, kb, fb, hb, vb, wb, out):
+        gpu.release(b)
