@@ -14,15 +14,17 @@
 //     keys; two waves share 16 heads, each with half of the 512 columns: it multiplies its half of the queries (96 registers of terms)
 //     with its half of the keys, the two add their partial scores through LDS, both form the weights, and each sums its half of the
 //     value columns (64 registers).  That fits two waves a SIMD, which a wave with all 512 columns (320 registers) does not;
-//   * a wave brings in whole rows (32 / waves of them a step, 1 KiB an instruction, the row's address the wave's), splits FP32
-//     rows into planes of terms, and stores them to a padded tile that every wave reads without bank conflicts; the next step's rows
-//     are fetched into registers before this step is multiplied, and no barrier waits for them;
+//   * a wave brings in whole rows (32 / waves of them a step, the row's address the wave's): BF16 rows go from memory to a padded tile
+//     in LDS by themselves, a step ahead, their numbers in the selection read another step ahead (fetched through registers they left
+//     51 registers to spill, and each number waited for the row before it: 128 us, then 109, now 97); FP32 rows are split into three
+//     planes of terms on their way;
 //   * the scores S^T = K . Q^T leave the weights in the B-operand layout of O^T += V^T . P^T; a lane's place in a value operand
 //     stands for eight neighbouring columns in eight products, so nothing is transposed (as in latent_gather.hip).
 // Many rows (a prompt) give every compute unit a workgroup that finishes its outputs; few rows are cut into runs of steps whose
 // (maximum, sum, unnormalised outputs) latent_rows_merge_kernel puts together.
-// Measured at 64 heads, a window of 128 and 512 selected BF16 rows: 256 rows in 128 us where the general kernel (FP32 on the vector
-// units, a key row read once for eight heads) took 1400; one row in 17.5 + 4.6 us where it took 447.  The differences from 64-bit
+// Measured at 64 heads, a window of 128 and 512 selected BF16 rows: 256 rows in 97 us where the general kernel (FP32 on the vector
+// units, a key row read once for eight heads) took 1400; one row in 14 + 4.6 us where it took 447.  Of the 97 us the
+// queries and outputs take 13 (67 MB); a step of BF16 rows takes 3.3 us, of which its products are 1.4 and its LDS reads, in phase with them, 0.9.  The differences from 64-bit
 // arithmetic are as large as before, 1e-6 at outputs of order one.
 #include "paged_rows.hpp"
 
@@ -71,6 +73,8 @@ __device__ __forceinline__ void split_pair(float x, float y, uint32_t& high, uin
     x -= __uint_as_float(middle << 16); y -= __uint_as_float(middle & 0xffff0000u);
     low = to_bf16_pair(x, y);
 }
+// every load of the wave, those to LDS included
+__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 struct Terms { uint4 high, middle, low; };       // eight values
 __device__ __forceinline__ Terms split_eight(const float (&x)[8]) {
     Terms t;
@@ -90,23 +94,31 @@ __device__ __forceinline__ void turn(float& x, float& y, double2 t) {
     y = float(a * t.y + b * t.x);
 }
 
-// A step's eight value columns c of the wave's columns 8 * li.., as operands: rows {4g..4g+3, 16+4g..16+4g+3} of the tile.
-__device__ __forceinline__ void value_operands(const uint8_t* from, bf16x8 (&out)[8]) {
+// O^T += V^T . P^T for eight products: place li of product c's operand is value column c of the lane's eight from `from` on, its k-slots
+// the tile's rows {4g..4g+3, 16+4g..16+4g+3}; the N weight operands follow one another, two columns in turn.
+template<int N>
+__device__ __forceinline__ void value_products(const uint8_t* from, const bf16x8 (&weights)[N], floatx4* acc) {
     uint4 rows8[8];
     #pragma unroll
     for (int e = 0; e < 8; ++e) rows8[e] = *reinterpret_cast<const uint4*>(from + (e < 4 ? e : 12 + e) * PITCH);
     #pragma unroll
-    for (int c = 0; c < 8; ++c) {
-        const uint32_t sel = (c & 1) ? 0x07060302u : 0x05040100u;
-        uint32_t words[4];
+    for (int c = 0; c < 8; c += 2) {
+        bf16x8 v[2];
         #pragma unroll
-        for (int w = 0; w < 4; ++w) {
-            const uint4 &low = rows8[2 * w], &high = rows8[2 * w + 1];
-            const uint32_t lo = c / 2 == 0 ? low.x : c / 2 == 1 ? low.y : c / 2 == 2 ? low.z : low.w;
-            const uint32_t hi = c / 2 == 0 ? high.x : c / 2 == 1 ? high.y : c / 2 == 2 ? high.z : high.w;
-            words[w] = byte_perm(hi, lo, sel);
+        for (int i = 0; i < 2; ++i) {
+            uint32_t words[4];
+            #pragma unroll
+            for (int w = 0; w < 4; ++w) {
+                const uint4 &low = rows8[2 * w], &high = rows8[2 * w + 1];
+                const uint32_t lo = c == 0 ? low.x : c == 2 ? low.y : c == 4 ? low.z : low.w, hi = c == 0 ? high.x : c == 2 ? high.y : c == 4 ? high.z : high.w;
+                words[w] = byte_perm(hi, lo, i ? 0x07060302u : 0x05040100u);
+            }
+            v[i] = operand(uint4{words[0], words[1], words[2], words[3]});
         }
-        out[c] = operand(uint4{words[0], words[1], words[2], words[3]});
+        #pragma unroll
+        for (int n = 0; n < N; ++n)
+            #pragma unroll
+            for (int i = 0; i < 2; ++i) acc[c + i] = product(v[i], weights[n], acc[c + i]);
     }
 }
 
@@ -139,36 +151,34 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         else sincos(double(p) * double(a.frequencies[thread]), &t.y, &t.x);
         turns[thread] = t;
     }
-    // the rows of a step: whether it is FP32 rows, and their addresses (a row that does not exist is read from the ring's first)
-    uint4 fetched[MINE][2];
-    uint32_t present = 0;
-    const auto fetch = [&](unsigned step) {
-        present = 0;
-        if (step < raw_steps) {
-            #pragma unroll
-            for (int j = 0; j < MINE; ++j) {
-                const unsigned index = step * STEP + wave + WAVES_HERE * j;
-                const bool exists = index < raw_count;
-                const uint4* from = reinterpret_cast<const uint4*>(a.raw + size_t(exists ? unsigned(first + index) % a.raw_rows : 0u) * DIM) + 2 * lane;
-                fetched[j][0] = from[0]; fetched[j][1] = from[1];
-                present |= exists ? 1u << j : 0u;
-            }
-        } else {
-            #pragma unroll
-            for (int j = 0; j < MINE; ++j) {
-                const unsigned index = (step - raw_steps) * STEP + wave + WAVES_HERE * j;
-                const uint32_t at = uint32_t(selected[min(index, a.selections - 1)]);
-                const bool exists = index < a.selections && at < a.compressed_rows;         // (a negative entry is a large unsigned one)
-                if (BF16) fetched[j][0] = *(reinterpret_cast<const uint4*>(exists ? static_cast<const uint16_t*>(a.compressed) + size_t(at) * DIM : reinterpret_cast<const uint16_t*>(a.raw)) + lane);
-                else {
-                    const uint4* from = reinterpret_cast<const uint4*>(exists ? static_cast<const float*>(a.compressed) + size_t(at) * DIM : a.raw) + 2 * lane;
-                    fetched[j][0] = from[0]; fetched[j][1] = from[1];
-                }
-                present |= exists ? 1u << j : 0u;
-            }
-        }
+    // A step's rows.  BF16 rows go straight to their plane of the tile, a row an instruction, asked for a step ahead; FP32 rows come
+    // through registers, where they are split.  A row that does not exist is read from the ring's first and zeroed afterwards.  The
+    // selection's entries are read another step ahead, the wave's MINE rows in as many lanes: asked for where they are needed, each
+    // would wait for the row before it.
+    int32_t names = -1;
+    const auto read_names = [&](unsigned step) {
+        const unsigned index = (step - raw_steps) * STEP + wave + WAVES_HERE * (lane % MINE);
+        const int32_t entry = selected[min(index, a.selections - 1)];
+        names = index < a.selections ? entry : -1;
     };
-    if (begin < end) fetch(begin);
+    const auto named_row = [&](int j, bool& exists) -> const uint8_t* {
+        const uint32_t at = uint32_t(__builtin_amdgcn_readlane(names, j));
+        exists = at < a.compressed_rows;                                                    // (a negative entry is a large unsigned one)
+        return exists ? static_cast<const uint8_t*>(a.compressed) + size_t(at) * DIM * (BF16 ? 2 : 4) : reinterpret_cast<const uint8_t*>(a.raw);
+    };
+    uint32_t present = 0;                    // bit j: the wave's j-th row of the step asked for ahead exists
+    const auto ask = [&](unsigned step) {
+        present = 0;
+        #pragma unroll
+        for (int j = 0; j < MINE; ++j) {
+            bool exists;
+            const uint8_t* from = named_row(j, exists);
+            load_run_to_lds<false, 1>(from, lds_address(tiles + (step & 1) * PLANE + (wave + WAVES_HERE * j) * PITCH), 16 * lane);
+            present |= exists ? 1u << j : 0u;
+        }
+        if (step + 1 < end) read_names(step + 1);
+    };
+    if (end > raw_steps) read_names(max(begin, raw_steps));
 
     // queries: the wave's half of its heads' columns as three terms
     uint4 qh[KSTEPS], qm[KSTEPS], ql[KSTEPS];
@@ -180,11 +190,13 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         for (int b = 0; b < KSTEPS; ++b) {
             const float4 x0 = *reinterpret_cast<const float4*>(from + 32 * b), x1 = *reinterpret_cast<const float4*>(from + 32 * b + 4);
             float x[8] = {x0.x, x0.y, x0.z, x0.w, x1.x, x1.y, x1.z, x1.w};
-            if (b >= KSTEPS / 2 && half) {             // (at most 128 columns are turned)
+            if (b >= KSTEPS / 2 && half && HALF + 32 * b + 32 > rotated) {             // (at most 128 columns are turned)
                 #pragma unroll
                 for (int i = 0; i < 8; i += 2) {
                     const int column = HALF + 32 * b + 8 * g + i;
-                    if (column >= rotated) turn(x[i], x[i + 1], turns[(column - rotated) / 2]);
+                    float u = x[i], v = x[i + 1];
+                    turn(u, v, turns[max(column - rotated, 0) / 2]);
+                    x[i] = column >= rotated ? u : x[i]; x[i + 1] = column >= rotated ? v : x[i + 1];
                 }
             }
             const Terms t = split_eight(x);
@@ -201,24 +213,46 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         const unsigned turn_of = step & 1;
         uint8_t* tile = tiles + (wide ? 0u : turn_of * PLANE);
         uint32_t* here = seen + turn_of * STEP;
-        #pragma unroll
-        for (int j = 0; j < MINE; ++j) {
-            const int r = wave + WAVES_HERE * j;
-            if (!((present >> j) & 1u)) fetched[j][0] = fetched[j][1] = uint4{0u, 0u, 0u, 0u};       // (its weights are zero, and zero times anything finite adds nothing)
-            uint8_t* to = tile + r * PITCH + 16 * lane;
-            if (wide) {
-                const uint4 u = fetched[j][0], v = fetched[j][1];
-                const float x[8] = {__uint_as_float(u.x), __uint_as_float(u.y), __uint_as_float(u.z), __uint_as_float(u.w),
-                                    __uint_as_float(v.x), __uint_as_float(v.y), __uint_as_float(v.z), __uint_as_float(v.w)};
-                const Terms t = split_eight(x);
+        if (wide) {
+            float4 pieces[MINE][2];
+            present = 0;
+            #pragma unroll
+            for (int j = 0; j < MINE; ++j) {
+                bool exists;
+                const uint8_t* from;
+                if (BF16 || step < raw_steps) {
+                    const unsigned index = step * STEP + wave + WAVES_HERE * j;
+                    exists = index < raw_count;
+                    from = reinterpret_cast<const uint8_t*>(a.raw + size_t(exists ? unsigned(first + index) % a.raw_rows : 0u) * DIM);
+                } else from = named_row(j, exists);
+                pieces[j][0] = reinterpret_cast<const float4*>(from)[2 * lane]; pieces[j][1] = reinterpret_cast<const float4*>(from)[2 * lane + 1];
+                present |= exists ? 1u << j : 0u;
+            }
+            if (!BF16 && step >= raw_steps && step + 1 < end) read_names(step + 1);
+            #pragma unroll
+            for (int j = 0; j < MINE; ++j) {
+                const float4 u = pieces[j][0], v = pieces[j][1];
+                const float x[8] = {u.x, u.y, u.z, u.w, v.x, v.y, v.z, v.w};
+                Terms t = split_eight(x);
+                if (!((present >> j) & 1u)) t.high = t.middle = t.low = uint4{0u, 0u, 0u, 0u};             // (its weights are zero, and zero times anything finite adds nothing)
+                uint8_t* to = tile + (wave + WAVES_HERE * j) * PITCH + 16 * lane;
                 *reinterpret_cast<uint4*>(to) = t.high;
                 *reinterpret_cast<uint4*>(to + PLANE) = t.middle;
                 *reinterpret_cast<uint4*>(to + 2 * PLANE) = t.low;
-            } else *reinterpret_cast<uint4*>(to) = fetched[j][0];
-            if (lane == 0) here[r] = (present >> j) & 1u;
+                if (lane == 0) here[wave + WAVES_HERE * j] = (present >> j) & 1u;
+            }
+        } else {
+            if (step == begin || step == raw_steps) ask(step);
+            wait_loads();
+            #pragma unroll
+            for (int j = 0; j < MINE; ++j) {
+                const int r = wave + WAVES_HERE * j;
+                if (!((present >> j) & 1u)) *reinterpret_cast<uint4*>(tile + r * PITCH + 16 * lane) = uint4{0u, 0u, 0u, 0u};
+                if (lane == 0) here[r] = (present >> j) & 1u;
+            }
         }
-        if (step + 1 < end) fetch(step + 1);
         ring_barrier();
+        if (!wide && step + 1 < end) ask(step + 1);
         // S^T over the wave's columns: keys (4 a lane group) x heads (lane li), one accumulator an order of magnitude
         floatx4 s[2];
         {
@@ -287,24 +321,11 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         #pragma unroll
         for (int q = 0; q < TILES / 8; ++q) {
             const uint8_t* from = tile + 4 * g * PITCH + 2 * (HALF * half + 128 * q + 8 * li);
-            bf16x8 v[8];
             if (wide) {
-                value_operands(from + 2 * PLANE, v);
-                #pragma unroll
-                for (int c = 0; c < 8; ++c) acc[8 * q + c] = product(v[c], wh, acc[8 * q + c]);
-                value_operands(from + PLANE, v);
-                #pragma unroll
-                for (int c = 0; c < 8; ++c) acc[8 * q + c] = product(v[c], wm, acc[8 * q + c]);
-                #pragma unroll
-                for (int c = 0; c < 8; ++c) acc[8 * q + c] = product(v[c], wh, acc[8 * q + c]);
+                value_products<1>(from + 2 * PLANE, {wh}, acc + 8 * q);
+                value_products<2>(from + PLANE, {wm, wh}, acc + 8 * q);
             }
-            value_operands(from, v);
-            #pragma unroll
-            for (int c = 0; c < 8; ++c) acc[8 * q + c] = product(v[c], wl, acc[8 * q + c]);
-            #pragma unroll
-            for (int c = 0; c < 8; ++c) acc[8 * q + c] = product(v[c], wm, acc[8 * q + c]);
-            #pragma unroll
-            for (int c = 0; c < 8; ++c) acc[8 * q + c] = product(v[c], wh, acc[8 * q + c]);
+            value_products<3>(from, {wl, wm, wh}, acc + 8 * q);
         }
         if (wide) ring_barrier();          // the planes are written again by the next step
     }
