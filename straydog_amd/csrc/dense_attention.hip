@@ -12,6 +12,13 @@
 
 using namespace sd;
 
+namespace sd {
+bool dense_matrix_supported(uint64_t context, uint64_t rows, uint64_t heads, uint64_t kv_heads, uint64_t dim, const float* q, const float* keys, const float* values,
+                            const float* gate, const float* out);
+void dense_matrix(Device& d, const float* q, const float* keys, const float* values, uint64_t context, const int32_t* positions, uint64_t rows, uint64_t heads,
+                  uint64_t kv_heads, uint64_t dim, float scale, const float* gate, float* scratch, uint64_t scratch_splits, float* out);
+}
+
 namespace {
 
 constexpr int TILE = 64, SLICE = 32, THREADS = 256, MAX_GROUP = 16, MAX_COLS = 4;
@@ -223,6 +230,11 @@ int sd_op_attention(void* handle, const float* q, const float* keys, const float
     if (!scratch || scratch_bytes < partial_bytes) throw std::runtime_error("Straydog attention scratch too small");
     op_span(value, scratch, partial_bytes, "attention scratch");
     if (attention_lds(size_t(heads / kv_heads), size_t(dim)) > 160 * 1024 - 64) throw std::runtime_error("invalid Straydog attention shape");
+    // 128 or 256 columns: the matrix-core kernel (dense_matrix.hip); the one here takes every other shape
+    if (dense_matrix_supported(context, rows, heads, kv_heads, dim, q, keys, values, gate, out)) {
+        dense_matrix(value, q, keys, values, context, positions, rows, heads, kv_heads, dim, scale, gate, scratch, splits, out);
+        return 0;
+    }
     const DenseSource source{keys, values, positions, size_t(context), size_t(kv_heads), size_t(dim)};
     launch(value, source, q, size_t(rows), size_t(heads), size_t(kv_heads), size_t(dim), scale, splits, scratch, gate, out);
     SD_OP_END

@@ -674,3 +674,42 @@ def test_latent_rows_on_the_matrix_cores(gpu, oracle, rows, heads, window, raw_r
         assert np.abs(got[some] - want).max() < 1e-5
     for b in (qb, rb, pb, sb, kb, fb, hb, vb, wb, out):
         gpu.release(b)
+
+
+@pytest.mark.parametrize("rows,heads,kv_heads,dim,context", [(1, 16, 2, 256, 4200), (1, 4, 4, 128, 33), (2, 16, 1, 128, 1000), (5, 24, 2, 256, 96), (33, 16, 2, 128, 700),
+                                                             (70, 16, 2, 256, 300), (300, 16, 4, 128, 400), (1, 1, 1, 256, 1)])
+def test_dense_attention_on_the_matrix_cores(gpu, oracle, rows, heads, kv_heads, dim, context):
+    # 128 and 256 columns: one and two tiles of 32 query rows, runs of keys merged or one run finished in place, rows that see one key and
+    # rows past the cache's end, what lies past every row's position never used; the scratch of the reference's contract, and graphs that
+    # find no larger workspace
+    rng = np.random.default_rng(rows * 1000 + context)
+    q = rng.standard_normal((rows, heads, dim)).astype(np.float32) * 2
+    keys = rng.standard_normal((context, kv_heads, dim)).astype(np.float32)
+    values = rng.standard_normal((context, kv_heads, dim)).astype(np.float32)
+    positions = rng.integers(0, context, size=rows).astype(np.int32)
+    positions[-1] = context + 3 if rows > 1 else context - 1
+    if rows > 5:
+        positions[:3] = (0, context // 2, 31)
+    gate = rng.standard_normal(q.shape).astype(np.float32)
+    qs, ks, vs, gs, ps = (gpu.upload(x) for x in (q, keys, values, gate, positions))
+    pairs = rows * heads
+    scratch, out = gpu.buffer(pairs * min(64, max(1, 256 // pairs)) * (dim + 2) * 4), gpu.buffer(q.size * 4)
+    for gated in (False, True):
+        gpu.attention(qs.base(), ks.base(), vs.base(), context, ps.base(), rows, heads, kv_heads, dim, float(dim ** -0.5), gs.base() if gated else None, scratch,
+                      out.base())
+        got = _read(gpu, out, np.float32, q.size).reshape(q.shape)
+        want, bound = oracle.op_attention_f64(q, keys, values, positions, float(np.float32(dim ** -0.5)), gate if gated else None)
+        assert np.all(np.isfinite(got)) and np.abs((got - want) / bound).max() <= 1.0
+    with backend(1 << 30) as other:         # nothing run on this handle yet: its workspace is empty
+        copies = [other.upload(x) for x in (q, keys, values, positions)]
+        room, result = other.buffer(scratch.size), other.buffer(q.size * 4)
+        other.graph_begin()
+        other.attention(*[b.base() for b in copies[:3]], context, copies[3].base(), rows, heads, kv_heads, dim, float(dim ** -0.5), None, room, result.base())
+        other.graph_end(1)
+        for _ in range(3):
+            assert other.graph_run(1)
+            got = _read(other, result, np.float32, q.size).reshape(q.shape)
+            want, bound = oracle.op_attention_f64(q, keys, values, positions, float(np.float32(dim ** -0.5)), None)
+            assert np.abs((got - want) / bound).max() <= 1.0
+    for b in (qs, ks, vs, gs, ps, scratch, out):
+        gpu.release(b)
