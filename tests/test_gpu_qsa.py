@@ -642,3 +642,44 @@ def test_prompt_chunk_stage_in_one_call_equals_its_parts(gpu, oracle, row_bytes,
         gpu.qsa_prefill_attend(state, one["projections"].base(), stride, most, first, gpu.buffer(4096), one["attended"].base())
     with pytest.raises(RuntimeError, match="inside the context"):
         gpu.qsa_prefill_attend(state, one["projections"].base(), stride, most, context - 1, scratch, one["attended"].base())
+
+
+@pytest.mark.parametrize("row_bytes,paged,rows,f16", [(272, True, 33, False), (272, False, 70, True), (512, True, 64, True), (512, False, 35, False)])
+def test_prompt_rows_have_the_bits_of_single_rows(gpu, oracle, row_bytes, paged, rows, f16):
+    # enough rows for a workgroup each over their whole lists: the same bits as every row alone, whose chunks are workgroups; lists of
+    # no entry, one, a unit's edges, a chunk's edges and everything, entries that do not count among them, with the gate and without
+    rng = np.random.default_rng(rows)
+    heads, kv_heads, context, selected = 24, 2, 3072, 2052
+    page_tokens = 256 if paged else context
+    pages = context // page_tokens
+    pool, pool_buffer = gpu.kv_pool(pages, page_tokens, kv_heads, 256, row_bytes)
+    table = gpu.upload(rng.permutation(pages).astype(np.int32))
+    kb = gpu.upload(rng.standard_normal((context, kv_heads, 256)).astype(np.float32))
+    vb = gpu.upload(rng.standard_normal((context, kv_heads, 256)).astype(np.float32))
+    gpu.kv_write(pool, table.base(), pages, gpu.upload(np.zeros(1, np.int32)).base(), kb.base(), vb.base(), False, 1, context)
+    base = context - rows
+    indices = np.full((rows, selected), 7.0, dtype=np.float32)
+    counts = np.zeros(rows, dtype=np.float32)
+    for r in range(rows):
+        counts[r] = (0, 1, 31, 32, 33, 127, 128, 129, 2052)[r % 9] if r < 18 else rng.integers(1, selected + 1)
+        indices[r, :int(counts[r])] = np.sort(rng.permutation(base + r + 1)[:int(counts[r])]).astype(np.float32)
+    indices[5, 3], indices[20, 0], indices[21, 40:90] = -1.0, float(context - 1), float(context + 5)
+    q = rng.standard_normal((rows, heads, 256)).astype(np.float16 if f16 else np.float32)
+    gate = rng.standard_normal((rows, heads, 512)).astype(np.float32)
+    ib, cb, qb, gb = (gpu.upload(x) for x in (indices, counts, q, gate))
+    size = 2 if f16 else 4
+    out, scratch = gpu.buffer(q.size * size), gpu.buffer(gpu.selected_attention_scratch(rows, kv_heads, selected))
+    for gated in (False, True):
+        def run(first, count):
+            gpu.selected_attention(pool, table.base() if paged else None, context, base + first, ib.at(first * selected * 4), selected, cb.at(first * 4),
+                                   qb.at(first * heads * 256 * size), f16, count, heads, 0.0625, out.at(first * heads * 256 * size), f16, scratch,
+                                   gate=gb.at(first * heads * 512 * 4) if gated else None, gate_stride=512 if gated else 0)
+        run(0, rows)
+        together = _read(gpu, out, np.uint16 if f16 else np.uint32, q.size).reshape(rows, -1)
+        gpu.write_buffer(out, 0, np.zeros(q.size * size, np.uint8))
+        for r in range(rows):
+            run(r, 1)
+        alone = _read(gpu, out, np.uint16 if f16 else np.uint32, q.size).reshape(rows, -1)
+        assert np.array_equal(together, alone) and not together[0].any() and together[8].any()
+    for b in (pool_buffer, table, kb, vb, ib, cb, qb, gb, out, scratch):
+        gpu.release(b)
