@@ -77,10 +77,9 @@ __device__ __forceinline__ size_t entry_row(const SelectedArgs& a, float raw, si
     return (page * 2 * a.kv_heads + kvh) * a.page_tokens + in_page;
 }
 
-// 32 entries' scores, weights and value sums, from nothing.
+// 32 entries' weights for the group's heads under their own maximum m; l: the lane's share of their sum.
 template<bool Q8>
-__device__ __forceinline__ void unit_attention(const SelectedArgs& a, const RowLoad<DIM, Q8>& current, const half8 (&qf)[DIM / 32], uint32_t usable, int g, float& m, float& l,
-                                               floatx4 (&acc)[DIM / 16]) {
+__device__ __forceinline__ half8 unit_weights(const SelectedArgs& a, const RowLoad<DIM, Q8>& current, const half8 (&qf)[DIM / 32], uint32_t usable, int g, float& m, float& l) {
     floatx4 s[2];
     #pragma unroll
     for (int t = 0; t < 2; ++t) {
@@ -104,16 +103,24 @@ __device__ __forceinline__ void unit_attention(const SelectedArgs& a, const RowL
             l += w;
             p[4 * t + r] = (_Float16)w;
         }
-    ValueScales<DIM> vs;
-    value_scales<DIM>(current, vs);
-    #pragma unroll
-    for (int jj = 0; jj < DIM / 16; ++jj)
-        acc[jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(value_operand<DIM>(current, vs, jj), p, floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
+    return p;
+}
+// The weighted sum of the unit's values for output tile jj, from nothing.
+template<bool Q8>
+__device__ __forceinline__ floatx4 unit_values(const RowLoad<DIM, Q8>& current, const ValueScales<DIM>& vs, const half8& p, int jj) {
+    return __builtin_amdgcn_mfma_f32_16x16x32_f16(value_operand<DIM>(current, vs, jj), p, floatx4{0.0f, 0.0f, 0.0f, 0.0f}, 0, 0, 0);
 }
 
-// The order in which a row's entries are put together is the same however its chunks are spread over workgroups, so a row has the
-// same bits alone and among the rows of a prompt: a chunk's four units under their common maximum, in order; then the chunks in
-// order, the sums so far scaled down where a chunk raises the maximum.
+// The order in which a row's entries are put together is the same however its chunks are spread over waves and workgroups, so a row
+// has the same bits alone and among the rows of a prompt: a chunk's four units under their common maximum, in order; the chunks of
+// each quarter of the list in order, the sums so far scaled down where a chunk raises the maximum; the quarters in order likewise.
+constexpr unsigned QUARTERS = 4;
+// a unit's maximum in exponent units, rounded (not contracted with a difference that follows)
+__device__ __forceinline__ float exponent_of(float m, float scale_log2) {
+    #pragma clang fp contract(off)
+    return m * scale_log2;
+}
+__device__ __forceinline__ unsigned quarter_begin(unsigned chunks, unsigned quarter) { return chunks * quarter / QUARTERS; }
 struct Running { float top, sum; };
 __device__ __forceinline__ void chunk_factors(Running& so_far, float top, float sum, float& keep, float& take) {
     const float higher = fmaxf(so_far.top, top);
@@ -170,7 +177,11 @@ __global__ void __launch_bounds__(WAVES * 64) selected_attention_kernel(Selected
         __builtin_amdgcn_s_waitcnt(0x0f70);             // vmcnt(0): the gathered rows have landed
         RowLoad<DIM, Q8> current;
         load_step<DIM>(current, stage, stage + SLAB, li, g);
-        unit_attention<Q8>(a, current, qf, uint32_t(usable), g, m, l, acc);
+        const half8 p = unit_weights<Q8>(a, current, qf, uint32_t(usable), g, m, l);
+        ValueScales<DIM> vs;
+        value_scales<DIM>(current, vs);
+        #pragma unroll
+        for (int jj = 0; jj < TILES; ++jj) acc[jj] = unit_values<Q8>(current, vs, p, jj);
     }
 
     // Merge the waves through LDS: per wave and query head the maximum, the sum and the unnormalised output.
@@ -178,7 +189,7 @@ __global__ void __launch_bounds__(WAVES * 64) selected_attention_kernel(Selected
     {
         const float sum = row_sum(l);
         float* mine = lds + (size_t(wave) * 16 + li) * STRIDE;
-        if (g == 0) { mine[DIM] = m * a.scale_log2; mine[DIM + 1] = sum; }      // maxima leave in exponent units
+        if (g == 0) { mine[DIM] = exponent_of(m, a.scale_log2); mine[DIM + 1] = sum; }      // maxima leave in exponent units
         #pragma unroll
         for (int jj = 0; jj < TILES; ++jj)
             #pragma unroll
@@ -211,12 +222,20 @@ __global__ void __launch_bounds__(DIM) selected_merge_kernel(SelectedArgs a) {
     constexpr int STRIDE = DIM + 2;
     const size_t row = blockIdx.x / a.heads;
     const unsigned head = blockIdx.x % a.heads, kvh = head / a.group, col = threadIdx.x;
-    const unsigned used = (list_length(a, row) + CHUNK - 1) / CHUNK;
+    const unsigned used = __builtin_amdgcn_readfirstlane((list_length(a, row) + CHUNK - 1) / CHUNK);
     const float* base = a.partial + ((row * a.kv_heads + kvh) * a.chunks) * 16 * STRIDE + size_t(head % a.group) * STRIDE;
-    // the chunks' pieces are asked for eight at a time: eight loads in flight, not one after the other
-    constexpr unsigned AT_ONCE = 8;
-    Running so_far{NEG_BIG, 0.0f};
-    float value = 0.0f;
+    // the chunks' pieces are asked for twenty at a time (a list of 2052 has 17): as many loads in flight, not one after the other
+    constexpr unsigned AT_ONCE = 20;
+    Running so_far{NEG_BIG, 0.0f}, quarter{NEG_BIG, 0.0f};
+    float value = 0.0f, quarter_value = 0.0f, keep, take;
+    unsigned quarters = 0;                             // those closed
+    const auto close = [&] {
+        chunk_factors(so_far, quarter.top, quarter.sum, keep, take);
+        value = chunk_added(value, quarter_value, keep, take);
+        quarter = Running{NEG_BIG, 0.0f};
+        quarter_value = 0.0f;
+        ++quarters;
+    };
     for (unsigned c0 = 0; c0 < used; c0 += AT_ONCE) {
         float tops[AT_ONCE], sums[AT_ONCE], values[AT_ONCE];
         #pragma unroll
@@ -225,13 +244,16 @@ __global__ void __launch_bounds__(DIM) selected_merge_kernel(SelectedArgs a) {
             tops[i] = part[DIM]; sums[i] = part[DIM + 1]; values[i] = part[col];
         }
         #pragma unroll
+        for (unsigned i = 0; i < AT_ONCE; ++i) asm volatile("" : "+v"(values[i]), "+v"(tops[i]), "+v"(sums[i]));      // (here, not one by one behind the branches below)
+        #pragma unroll
         for (unsigned i = 0; i < AT_ONCE; ++i) {
-            // (a place past the last chunk: nothing is taken and everything kept)
-            float keep, take;
-            chunk_factors(so_far, c0 + i < used ? tops[i] : NEG_BIG, c0 + i < used ? sums[i] : 0.0f, keep, take);
-            value = chunk_added(value, c0 + i < used ? values[i] : 0.0f, keep, take);
+            if (c0 + i >= used) break;
+            while (c0 + i >= quarter_begin(used, quarters + 1)) close();
+            chunk_factors(quarter, tops[i], sums[i], keep, take);
+            quarter_value = chunk_added(quarter_value, values[i], keep, take);
         }
     }
+    while (quarters < QUARTERS) close();
     value = finished(value, so_far.sum);
     if (a.gate) value = gated(value, a.gate[row * a.gate_row_stride + head * a.gate_stride + col]);
     const size_t at = (row * a.heads + head) * DIM + col;
@@ -239,111 +261,225 @@ __global__ void __launch_bounds__(DIM) selected_merge_kernel(SelectedArgs a) {
     else static_cast<float*>(a.out)[at] = value;
 }
 
-// The rows of a prompt chunk: a workgroup works a row's whole list for one K/V head, chunk after chunk, and stores the finished
-// outputs -- no partial results, which for 1024 rows were 0.43 GB written and read again.
-//   * The list is turned into pool rows once, in LDS.  A unit's rows are gathered into the wave's stage while the unit before is
-//     multiplied: its operands are in registers by then.
-//   * A chunk's four units meet through LDS lane to lane: wave w takes the value tiles 4 w .. 4 w + 3 of all four (16 registers of
-//     running sums a wave), with FP16 rows over the value slabs, whose next rows are then asked for afterwards.
+// The rows of a prompt chunk: a workgroup works a row's whole list for one K/V head, a wave a quarter of it, and stores the finished
+// outputs.
+//   * The list is turned into places of the pool once, in LDS.  From there on the waves are on their own: each gathers slabs of 32
+//     rows (K or V) into a ring of two, asks for the next but one as soon as a slab's operands are in registers, and meets the others
+//     only when its quarter is done.
+//   * A chunk's four units give their weights first and are then summed, in the order that chunks as workgroups have.
+//   * Q8_0 rows lie in a slab as 256 bytes of values and, behind all of them, 16 of scales; the 16-byte piece a lane brings is the one that
+//     belongs at its place turned by the row's number, so operands are read without bank conflicts and a row's address costs a lane
+//     two instructions (an LDS word, shifted and added).
+//   * 77 KB of LDS (Q8_0, a list of 2052) and 256 registers: two workgroups a compute unit, so each SIMD has a second wave while one waits or multiplies.
+//     (Units exchanged through LDS chunk by chunk, with 142 KB and one wave a SIMD, took 552 us below.)
 //   * Workgroups that run together on one die have neighbouring rows and the same K/V head: their selections overlap, and the die's
 //     L2 serves a row to all of them.
-// Bound by vector instructions (turning Q8_0 bytes into FP16 operands is 384 of a unit's ~600).  Measured, 1024 rows of 2052 entries, 24
-// heads over 2: PROMPT_AFTER us where chunks as workgroups and their merge took 741 + 112.
+// Bound by vector instructions (turning Q8_0 bytes into FP16 operands is 384 of a unit's ~700).  Measured, 1024 rows of 2052 Q8_0
+// entries, 24 heads over 2: 276 us where chunks as workgroups and their merge take 741 + 112; FP16 rows, the whole stage: 626 us for 1943.
 constexpr unsigned LIST_MAX = 4096;
 template<bool Q8> struct ListShape {
-    static constexpr int ROW = Q8 ? DIM + DIM / 16 : 2 * DIM, SLAB = STEP * ROW, STAGES = WAVES * 2 * SLAB, EXCHANGE = WAVES * WAVES * 4 * 1024;
-    static constexpr int BYTES = STAGES + (Q8 ? EXCHANGE : 0) + WAVES * 16 * 8 + LIST_MAX / 8;      // the list follows
+    static constexpr int ROW = Q8 ? DIM + DIM / 16 : 2 * DIM, PIECES = ROW / 16, SLAB = STEP * ROW, STAGES = WAVES * 2 * SLAB, LOADS = Q8 ? 9 : 16;
+    static constexpr int BYTES = STAGES + WAVES * 16 * 8 + LIST_MAX / 8;      // the list follows
+    static_assert(STAGES >= WAVES * WAVES * 4 * 1024, "the waves' sums meet over the stages");
 };
+// The same number, in a way the compiler cannot see through: the addresses formed from it inside a loop are formed there and do not
+// sit in registers through it.
+__device__ __forceinline__ int fresh(int x) { asm volatile("" : "+v"(x)); return x; }
+template<int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+// Four global->LDS loads to `to` and the three KiB after it, from four addresses a lane.
+__device__ __forceinline__ void load_four_to_lds(const uint8_t* const (&from)[4], uint32_t to) {
+    uint32_t keep;
+#define SD_NEXT_LOAD "s_add_u32 m0, m0, 0x400\n\ts_nop 0\n\t"
+    asm volatile("s_mov_b32 %0, m0\n\ts_mov_b32 m0, %1\n\ts_nop 0\n\tglobal_load_lds_dwordx4 %2, off\n\t" SD_NEXT_LOAD "global_load_lds_dwordx4 %3, off\n\t"
+                 SD_NEXT_LOAD "global_load_lds_dwordx4 %4, off\n\t" SD_NEXT_LOAD "global_load_lds_dwordx4 %5, off\n\ts_mov_b32 m0, %0"
+                 : "=&s"(keep) : "s"(to), "v"(from[0]), "v"(from[1]), "v"(from[2]), "v"(from[3]) : "memory", "scc");
+#undef SD_NEXT_LOAD
+}
+// A slab's rows, asked for; list: the places (in 16-byte pieces of the plane) of its 32 rows.
+template<bool Q8>
+__device__ __forceinline__ void gather_slab(const uint8_t* plane, const uint32_t* list, uint8_t* slab, int thread) {
+    const int lane = fresh(thread) & 63;
+    const uint32_t to = __builtin_amdgcn_readfirstlane(lds_address(slab));
+    const auto place = [&](uint32_t row_at, uint32_t piece) { return plane + (uint64_t(row_at + piece) << 4); };
+    constexpr int SPAN = Q8 ? 16 : 32, ROWS = 64 / SPAN;                 // a lane's piece is one of SPAN; rows a load
+    const uint32_t* from = list + lane / SPAN;
+    const uint32_t turned = (lane % SPAN) ^ (lane / SPAN);               // (row % 16 = (ROWS * j) % 16 + lane / SPAN, the two without a common bit)
+    #pragma unroll
+    for (int j = 0; j < SPAN / 2; j += 4) {
+        const uint8_t* at[4];
+        #pragma unroll
+        for (int i = 0; i < 4; ++i) at[i] = place(from[ROWS * (j + i)], turned ^ ((ROWS * (j + i)) % 16));
+        load_four_to_lds(at, to + 1024 * j);
+    }
+    if (Q8 && lane < STEP) load_to_lds<false>(place(list[lane], 16), slab + STEP * DIM);
+}
+// A slab's operands as paged_rows.hpp takes them: the K side, the V side.
+__device__ __forceinline__ void slab_keys(RowLoad<DIM, true>& r, const uint8_t* slab, int thread) {
+    const int lane = fresh(thread), li = lane & 15, g = lane >> 4 & 3;
+    #pragma unroll
+    for (int t = 0; t < 2; ++t) {
+        const uint32_t row = (16 * t + li) * DIM + 16 * (g / 2 ^ li) + 8 * (g & 1);
+        #pragma unroll
+        for (int b = 0; b < DIM / 32; ++b) r.k[t][b] = *reinterpret_cast<const uint2*>(slab + (row ^ 32 * b));
+        const uint4 scales = *reinterpret_cast<const uint4*>(slab + STEP * DIM + 16 * (16 * t + li));
+        r.kscale[t][0] = scales.x; r.kscale[t][1] = scales.y; r.kscale[t][2] = scales.z; r.kscale[t][3] = scales.w;
+    }
+}
+__device__ __forceinline__ void slab_values(RowLoad<DIM, true>& r, const uint8_t* slab, int thread) {
+    const int lane = fresh(thread), li = lane & 15, g = lane >> 4 & 3;
+    #pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int token = 4 * g + (e < 4 ? e : 12 + e);
+        const uint4 words = *reinterpret_cast<const uint4*>(slab + token * DIM + 16 * (li ^ (token & 15)));
+        r.v[e][0] = words.x; r.v[e][1] = words.y; r.v[e][2] = words.z; r.v[e][3] = words.w;
+        r.vscale[e] = *reinterpret_cast<const uint16_t*>(slab + STEP * DIM + 16 * token + 2 * (li / 2));
+    }
+}
+__device__ __forceinline__ void slab_keys(RowLoad<DIM, false>& r, const uint8_t* slab, int thread) {
+    const int lane = fresh(thread), li = lane & 15, g = lane >> 4 & 3;
+    #pragma unroll
+    for (int t = 0; t < 2; ++t)
+        #pragma unroll
+        for (int b = 0; b < DIM / 32; ++b) r.k[t][b] = *reinterpret_cast<const half8*>(slab + (16 * t + li) * 2 * DIM + 16 * ((4 * b + g) ^ li));
+}
+__device__ __forceinline__ void slab_values(RowLoad<DIM, false>& r, const uint8_t* slab, int thread) {
+    const int lane = fresh(thread), li = lane & 15, g = lane >> 4 & 3;
+    #pragma unroll
+    for (int e = 0; e < 8; ++e) {
+        const int token = 4 * g + (e < 4 ? e : 12 + e);
+        #pragma unroll
+        for (int h = 0; h < 2; ++h) {
+            const uint4 words = *reinterpret_cast<const uint4*>(slab + token * 2 * DIM + 16 * ((2 * li + h) ^ (token & 15)));
+            r.v[e][4 * h] = words.x; r.v[e][4 * h + 1] = words.y; r.v[e][4 * h + 2] = words.z; r.v[e][4 * h + 3] = words.w;
+        }
+    }
+}
 template<bool Q8, bool F16_OUT>
-__global__ void __launch_bounds__(WAVES * 64) selected_list_kernel(SelectedArgs a, unsigned rows) {
+__global__ void __launch_bounds__(WAVES * 64, Q8 ? 2 : 1) selected_list_kernel(SelectedArgs a, unsigned rows) {
     using Shape = ListShape<Q8>;
-    constexpr int ROW = Shape::ROW, SLAB = Shape::SLAB, PIECES = ROW / 16, UNITS = (STEP * PIECES + 63) / 64, TILES = DIM / 16;
+    constexpr int TILES = DIM / 16, UNITS = CHUNK / STEP;
     const unsigned items = rows * a.kv_heads, per_die = (items + 7) / 8, item = blockIdx.x % 8 * per_die + blockIdx.x / 8;
     if (item >= items || blockIdx.x / 8 >= per_die) return;
     const unsigned kvh = item / rows;
     const size_t row = item % rows, position = (a.dynamic_base ? size_t(*a.dynamic_base) : a.base) + row;
     const int thread = threadIdx.x, lane = thread & 63, wave = __builtin_amdgcn_readfirstlane(thread >> 6), li = lane & 15, g = lane >> 4;
-    const unsigned count = list_length(a, row), chunks = (count + CHUNK - 1) / CHUNK;
+    const unsigned count = __builtin_amdgcn_readfirstlane(list_length(a, row)), units = (count + STEP - 1) / STEP, chunks = (count + CHUNK - 1) / CHUNK;
     extern __shared__ uint8_t bytes[];
-    uint8_t *const kstage = bytes + wave * SLAB, *const vstage = bytes + (WAVES + wave) * SLAB;
-    floatx4* const exchange = reinterpret_cast<floatx4*>(bytes + (Q8 ? Shape::STAGES : WAVES * SLAB));       // [to][from][4][64]
-    float2* const stats = reinterpret_cast<float2*>(bytes + Shape::STAGES + (Q8 ? Shape::EXCHANGE : 0));     // [wave][16]: (maximum, sum)
+    uint8_t* const ring = bytes + wave * 2 * Shape::SLAB;
+    float2* const stats = reinterpret_cast<float2*>(bytes + Shape::STAGES);                                  // [wave][16]: (maximum, sum)
     uint32_t* const usable = reinterpret_cast<uint32_t*>(stats + WAVES * 16);                                // [unit]
     uint32_t* const list = usable + LIST_MAX / 32;
 
     for (unsigned e = thread; e < chunks * CHUNK; e += WAVES * 64) {
         bool counts_in;
-        list[e] = uint32_t(entry_row(a, e < count ? a.indices[row * a.selected + e] : -1.0f, position, kvh, counts_in));
+        list[e] = uint32_t(entry_row(a, e < count ? a.indices[row * a.selected + e] : -1.0f, position, kvh, counts_in)) * Shape::PIECES;
         const uint64_t these = __ballot(counts_in);
         if (lane == 0) { usable[e / STEP] = uint32_t(these); usable[e / STEP + 1] = uint32_t(these >> 32); }
     }
     half8 qf[DIM / 32];
     load_queries(a, row, kvh, li, g, qf);
-    const size_t value_plane = size_t(a.kv_heads) * a.page_tokens * ROW;
-    const auto gather = [&](unsigned unit, uint8_t* to, size_t plane) {
-        #pragma unroll
-        for (int j = 0; j < UNITS; ++j) {
-            const int piece = 64 * j + lane, entry = piece / PIECES, within = piece % PIECES;
-            if (64 * j + 64 <= STEP * PIECES || piece < STEP * PIECES)
-                load_to_lds<false>(a.pages + plane + size_t(list[unit * STEP + entry]) * ROW + 16 * within, to + 1024 * j);
-        }
-    };
     settle_loads();
     ring_barrier();
-    if (wave * STEP < count) { gather(wave, kstage, 0); gather(wave, vstage, value_plane); }
+    // The wave's slabs in order: of every chunk of its quarter the units' keys, then their values.
+    const uint8_t* const value_plane = a.pages + size_t(a.kv_heads) * a.page_tokens * Shape::ROW;
+    const unsigned begin = quarter_begin(chunks, wave), end = quarter_begin(chunks, wave + 1);
+    unsigned ahead_chunk = begin, ahead_slab = 0, asked = 0, taken = 0;
+    const auto units_of = [&](unsigned chunk) { return min(units - chunk * UNITS, unsigned(UNITS)); };
+    const auto ask = [&] {
+        if (ahead_chunk >= end) return;
+        const unsigned n = units_of(ahead_chunk), unit = ahead_chunk * UNITS + (ahead_slab < n ? ahead_slab : ahead_slab - n);
+        gather_slab<Q8>(ahead_slab < n ? a.pages : value_plane, list + unit * STEP, ring + (asked & 1) * Shape::SLAB, thread);
+        ++asked;
+        if (++ahead_slab == 2 * n) { ahead_slab = 0; ++ahead_chunk; }
+    };
+    const auto landed = [&] {                               // the next slab, complete
+        if (asked - taken > 1) wait_loads<Shape::LOADS>(); else wait_loads<0>();
+        return ring + (taken++ & 1) * Shape::SLAB;
+    };
+    const auto read = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };       // its operands are in registers: it may be overwritten
+    ask();
+    ask();
     Running so_far{NEG_BIG, 0.0f};
-    floatx4 total[4];
+    floatx4 total[TILES];
     #pragma unroll
-    for (int t = 0; t < 4; ++t) total[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
-    for (unsigned chunk = 0; chunk < chunks; ++chunk) {
-        const unsigned unit = chunk * WAVES + wave;
-        const bool more = (unit + WAVES) * STEP < count;
-        floatx4 acc[TILES];
-        float m = NEG_BIG, l = 0.0f;
-        if (unit * STEP < count) {
-            __builtin_amdgcn_s_waitcnt(0x0f70);             // the gathered rows have landed
-            RowLoad<DIM, Q8> current;
-            load_step<DIM>(current, kstage, vstage, li, g);
-            const uint32_t mask = usable[unit];
-            __builtin_amdgcn_s_waitcnt(0xc07f);             // the operands are in registers: the stage is free
-            asm volatile("" ::: "memory");
-            if (more) { gather(unit + WAVES, kstage, 0); if (Q8) gather(unit + WAVES, vstage, value_plane); }
-            unit_attention<Q8>(a, current, qf, mask, g, m, l, acc);
-        } else {
-            #pragma unroll
-            for (int jj = 0; jj < TILES; ++jj) acc[jj] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (int jj = 0; jj < TILES; ++jj) total[jj] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    for (unsigned chunk = begin; chunk < end; ++chunk) {
+        const unsigned n = units_of(chunk);
+        half8 p[UNITS];
+        float tops[UNITS], weight[UNITS], top = NEG_BIG, chunk_sum = 0.0f;
+        #pragma unroll
+        for (int u = 0; u < UNITS; ++u) {
+            float m = NEG_BIG, l = 0.0f;
+            if (u < int(n)) {
+                const uint8_t* slab = landed();
+                RowLoad<DIM, Q8> current;
+                slab_keys(current, slab, thread);
+                const uint32_t mask = usable[chunk * UNITS + u];
+                read();
+                ask();
+                p[u] = unit_weights<Q8>(a, current, qf, mask, g, m, l);
+            }
+            tops[u] = exponent_of(m, a.scale_log2);
+            top = fmaxf(top, tops[u]);
+            weight[u] = row_sum(l);
         }
-        const float sum = row_sum(l);
-        ring_barrier();                                     // the units of the chunk before have been taken (and, with FP16 rows, every wave has its values)
-        if (g == 0) stats[wave * 16 + li] = float2{m * a.scale_log2, sum};
         #pragma unroll
-        for (int jj = 0; jj < TILES; ++jj) exchange[((jj / 4 * WAVES + wave) * 4 + jj % 4) * 64 + lane] = acc[jj];
-        ring_barrier();
-        float2 unit_stats[WAVES];
-        float top = NEG_BIG;
+        for (int u = 0; u < UNITS; ++u) {
+            const float sum = weight[u];
+            weight[u] = __builtin_amdgcn_exp2f(tops[u] - top);
+            chunk_sum = fmaf(sum, weight[u], chunk_sum);
+        }
+        floatx4 value[TILES];
         #pragma unroll
-        for (int w = 0; w < WAVES; ++w) { unit_stats[w] = stats[w * 16 + li]; top = fmaxf(top, unit_stats[w].x); }
-        float weight[WAVES], chunk_sum = 0.0f;
+        for (int jj = 0; jj < TILES; ++jj) value[jj] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
         #pragma unroll
-        for (int w = 0; w < WAVES; ++w) { weight[w] = __builtin_amdgcn_exp2f(unit_stats[w].x - top); chunk_sum = fmaf(unit_stats[w].y, weight[w], chunk_sum); }
+        for (int u = 0; u < UNITS; ++u)
+            if (u < int(n)) {
+                const uint8_t* slab = landed();
+                RowLoad<DIM, Q8> current;
+                slab_values(current, slab, thread);
+                read();
+                ask();
+                ValueScales<DIM> vs;
+                value_scales<DIM>(current, vs);
+                #pragma unroll
+                for (int jj = 0; jj < TILES; jj += 2) {
+                    const floatx4 part[2] = {unit_values<Q8>(current, vs, p[u], jj), unit_values<Q8>(current, vs, p[u], jj + 1)};
+                    #pragma unroll
+                    for (int i = 0; i < 2; ++i)
+                        #pragma unroll
+                        for (int r = 0; r < 4; ++r) value[jj + i][r] = fmaf(part[i][r], weight[u], value[jj + i][r]);
+                    __builtin_amdgcn_sched_barrier(0);      // (more tiles in flight and the registers spill)
+                }
+            }
         float keep, take;
         chunk_factors(so_far, top, chunk_sum, keep, take);
         #pragma unroll
+        for (int jj = 0; jj < TILES; ++jj)
+            #pragma unroll
+            for (int r = 0; r < 4; ++r) total[jj][r] = chunk_added(total[jj][r], value[jj][r], keep, take);
+    }
+    // The quarters meet over the stages, lane to lane: wave w takes the value tiles 4 w .. 4 w + 3 of all four.
+    ring_barrier();
+    floatx4* const exchange = reinterpret_cast<floatx4*>(bytes);                                             // [to][from][4][64]
+    if (g == 0) stats[wave * 16 + li] = float2{so_far.top, so_far.sum};
+    #pragma unroll
+    for (int jj = 0; jj < TILES; ++jj) exchange[((jj / 4 * WAVES + wave) * 4 + jj % 4) * 64 + lane] = total[jj];
+    ring_barrier();
+    so_far = Running{NEG_BIG, 0.0f};
+    floatx4 sums[4];
+    #pragma unroll
+    for (int t = 0; t < 4; ++t) sums[t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    #pragma unroll
+    for (int w = 0; w < WAVES; ++w) {
+        const float2 quarter = stats[w * 16 + li];
+        float keep, take;
+        chunk_factors(so_far, quarter.x, quarter.y, keep, take);
+        #pragma unroll
         for (int t = 0; t < 4; ++t) {
-            floatx4 part[WAVES];
+            const floatx4 part = exchange[((wave * WAVES + w) * 4 + t) * 64 + lane];
             #pragma unroll
-            for (int w = 0; w < WAVES; ++w) part[w] = exchange[((wave * WAVES + w) * 4 + t) * 64 + lane];
-            #pragma unroll
-            for (int r = 0; r < 4; ++r) {
-                float value = 0.0f;
-                #pragma unroll
-                for (int w = 0; w < WAVES; ++w) value = fmaf(part[w][r], weight[w], value);
-                total[t][r] = chunk_added(total[t][r], value, keep, take);
-            }
-        }
-        if (!Q8 && chunk + 1 < chunks) {
-            ring_barrier();                                 // the exchange lay over the value slabs
-            if (more) gather(unit + WAVES, vstage, value_plane);
+            for (int r = 0; r < 4; ++r) sums[t][r] = chunk_added(sums[t][r], part[r], keep, take);
         }
     }
     if (li >= int(a.group)) return;
@@ -354,7 +490,7 @@ __global__ void __launch_bounds__(WAVES * 64) selected_list_kernel(SelectedArgs 
         const unsigned column = 16 * (4 * g + r) + 4 * wave;
         float value[4];
         #pragma unroll
-        for (int t = 0; t < 4; ++t) value[t] = finished(total[t][r], so_far.sum);
+        for (int t = 0; t < 4; ++t) value[t] = finished(sums[t][r], so_far.sum);
         if (a.gate) {
             const float4 x = *reinterpret_cast<const float4*>(a.gate + row * a.gate_row_stride + head * a.gate_stride + column);
             value[0] = gated(value[0], x.x); value[1] = gated(value[1], x.y); value[2] = gated(value[2], x.z); value[3] = gated(value[3], x.w);
@@ -366,6 +502,7 @@ __global__ void __launch_bounds__(WAVES * 64) selected_list_kernel(SelectedArgs 
         } else *reinterpret_cast<float4*>(static_cast<float*>(a.out) + at) = float4{value[0], value[1], value[2], value[3]};
     }
 }
+static_assert(WAVES == QUARTERS, "a wave a quarter");
 
 uint64_t scratch_bytes_for(uint64_t rows, uint64_t kv_heads, uint64_t selected) {
     return checked_floats({rows, kv_heads, (selected + CHUNK - 1) / CHUNK, 16, uint64_t(DIM) + 2});
@@ -432,9 +569,11 @@ int sdx_selected_attention(void* handle, const sdx_kv_pool* pool, const int32_t*
     args.chunks = unsigned((selected + CHUNK - 1) / CHUNK);
     args.gate = gate; args.gate_stride = size_t(gate_stride); args.gate_row_stride = size_t(gate_row_stride); args.out = out;
     const bool q8 = pool->row_bytes != 2 * pool->dim;
-    // A workgroup a row and K/V head once there are enough of them: LISTS_RULE
-    const bool lists = rows * pool->kv_heads * 4 >= value.compute_units && args.chunks * CHUNK <= LIST_MAX &&
-                       checked_product({pool->page_count, 2, pool->kv_heads, pool->page_tokens}) <= (uint64_t(1) << 32) && rows * pool->kv_heads < (uint64_t(1) << 31) &&
+    // A workgroup a row and K/V head once there are enough of them.  The stage of a chunk, lists of 2052 over two K/V heads, chunks as
+    // workgroups / lists: Q8_0 32 rows 108 / 127 us, 48: 123 / 132, 64: 138 / 134, 256: 304 / 175; FP16, whose chunks fill a compute unit's
+    // LDS, 16 rows 106 / 115, 24: 122 / 118, 64: 185 / 125.
+    const bool lists = rows * pool->kv_heads * (q8 ? 2 : 6) >= value.compute_units && args.chunks * CHUNK <= LIST_MAX &&
+                       checked_product({pool->page_count, 2, pool->kv_heads, pool->page_tokens, pool->row_bytes / 16}) <= (uint64_t(1) << 32) && rows * pool->kv_heads < (uint64_t(1) << 31) &&
                        (uintptr_t(out) | uintptr_t(gate)) % 16 == 0 && (gate_stride | gate_row_stride) % 4 == 0;
     if (q8) { if (out_f16) launch<true, true>(value, args, rows, lists); else launch<true, false>(value, args, rows, lists); }
     else { if (out_f16) launch<false, true>(value, args, rows, lists); else launch<false, false>(value, args, rows, lists); }

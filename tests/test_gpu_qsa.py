@@ -644,7 +644,7 @@ def test_prompt_chunk_stage_in_one_call_equals_its_parts(gpu, oracle, row_bytes,
         gpu.qsa_prefill_attend(state, one["projections"].base(), stride, most, context - 1, scratch, one["attended"].base())
 
 
-@pytest.mark.parametrize("row_bytes,paged,rows,f16", [(272, True, 33, False), (272, False, 70, True), (512, True, 64, True), (512, False, 35, False)])
+@pytest.mark.parametrize("row_bytes,paged,rows,f16", [(272, True, 65, False), (272, False, 70, True), (512, True, 64, True), (512, False, 35, False)])
 def test_prompt_rows_have_the_bits_of_single_rows(gpu, oracle, row_bytes, paged, rows, f16):
     # enough rows for a workgroup each over their whole lists: the same bits as every row alone, whose chunks are workgroups; lists of
     # no entry, one, a unit's edges, a chunk's edges and everything, entries that do not count among them, with the gate and without
