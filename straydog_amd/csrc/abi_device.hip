@@ -40,11 +40,12 @@ static std::string budget_exceeded(const Device& d, size_t bytes) {
            std::to_string(d.budget >> 20) + " MiB left)";
 }
 
-void* allocate(Device& d, size_t bytes, bool zero) {
-    const size_t available = d.budget > d.used ? d.budget - d.used : 0;
-    if (!bytes || bytes > available || allocation_tail > available - bytes) throw std::runtime_error(budget_exceeded(d, bytes));
+// Null when the card has no room.
+static void* try_allocate(Device& d, size_t bytes, bool zero) {
     void* pointer = nullptr;
-    SD_CHECK(hipMalloc(&pointer, bytes + allocation_tail));
+    const hipError_t error = hipMalloc(&pointer, bytes + allocation_tail);
+    if (error == hipErrorOutOfMemory) { (void)hipGetLastError(); return nullptr; }
+    SD_CHECK(error);
     {
         std::lock_guard<std::mutex> lock(d.mutex);
         d.allocations.emplace(static_cast<const uint8_t*>(pointer), bytes);
@@ -52,6 +53,25 @@ void* allocate(Device& d, size_t bytes, bool zero) {
     }
     if (zero) SD_CHECK(hipMemsetAsync(pointer, 0, bytes + allocation_tail, d.stream));
     else SD_CHECK(hipMemsetAsync(static_cast<uint8_t*>(pointer) + bytes, 0, allocation_tail, d.stream));
+    return pointer;
+}
+
+// The optional workspaces back to the budget; false: there were none (or a graph is being recorded, which may hold them).
+static bool give_back_optional_spaces(Device& d) {
+    if (d.optional_spaces.empty() || d.recording) return false;
+    drop_recorded_graphs(d);
+    for (const auto& space : d.optional_spaces) release(d, space.first);
+    d.optional_spaces.clear();
+    return true;
+}
+
+void* allocate(Device& d, size_t bytes, bool zero) {
+    const auto available = [&] { return d.budget > d.used ? d.budget - d.used : 0; };
+    const auto over = [&] { return !bytes || bytes > available() || allocation_tail > available() - bytes; };
+    if (over() && (!bytes || !give_back_optional_spaces(d) || over())) throw std::runtime_error(budget_exceeded(d, bytes));
+    void* pointer = try_allocate(d, bytes, zero);
+    if (!pointer && give_back_optional_spaces(d)) pointer = try_allocate(d, bytes, zero);
+    if (!pointer) SD_CHECK(hipErrorOutOfMemory);
     return pointer;
 }
 
@@ -131,13 +151,19 @@ void* workspace(Device& d, size_t bytes) {
     return d.workspace;
 }
 
-void* workspace_or_null(Device& d, size_t bytes) {
-    if (bytes > d.workspace_bytes) {
-        hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
-        SD_CHECK(hipStreamIsCapturing(d.stream, &capturing));
-        if (capturing != hipStreamCaptureStatusNone) return nullptr;
-    }
-    return workspace(d, bytes);
+void* optional_space(Device& d, size_t bytes) {
+    const size_t held = d.optional_spaces.empty() ? 0 : d.optional_spaces.back().second;
+    if (bytes <= held) return held ? d.optional_spaces.back().first : nullptr;
+    hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
+    SD_CHECK(hipStreamIsCapturing(d.stream, &capturing));
+    if (bytes > optional_space_most || capturing != hipStreamCaptureStatusNone) return nullptr;
+    const size_t rounded = std::min(optional_space_most, std::max((bytes + (size_t(4) << 20) - 1) & ~((size_t(4) << 20) - 1), 2 * held));
+    // (what is held already is not given back for this)
+    const size_t available = d.budget > d.used ? d.budget - d.used : 0;
+    if (rounded > available || allocation_tail > available - rounded) return nullptr;
+    void* space = try_allocate(d, rounded, false);
+    if (space) d.optional_spaces.emplace_back(space, rounded);
+    return space;
 }
 
 void op_span(Device& d, const void* pointer, size_t bytes, const char* what) {
