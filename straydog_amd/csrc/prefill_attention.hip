@@ -15,7 +15,9 @@
 //     operands without bank conflicts, multiplies and exponentiates, every wave's stream pipelined by hand.  A workgroup
 //     owns two runs of 128 rows, one from the end of the span and its mirror image from the start, so every workgroup does
 //     about the same work, and writes its outputs normalised, with no merge (details at the kernels);
-//   * prefill_attention_kernel (256 columns): 4 x QT x 16 rows per workgroup; every wave builds its own operands from the
+//   * prefill_operands_kernel (256 columns): the same idea with tiles of 32 keys that hold the products' operands as the lanes take
+//     them, 128 rows a workgroup, two workgroups a compute unit, walks cut into shares of keys where there are few of them;
+//   * prefill_attention_kernel (256 columns, many sequences with few rows each, and the union walk): 4 x QT x 16 rows per workgroup; every wave builds its own operands from the
 //     raw rows in the stage (paged_rows.hpp); a quarter of the rows belongs to a pair of waves, one taking the first 32
 //     keys of every step and one the last 32, each with its own online softmax, merged through LDS at the end; the
 //     workgroups with the longest walks are dispatched first.
@@ -48,7 +50,7 @@ struct PrefillArgs {
     const void* q;
     int q_f16;
     float scale_log2;      // softmax scale * log2(e): scores live in the base-2 domain
-    unsigned rows;         // span * group: query rows per K/V head
+    unsigned rows, seqs;   // span * group: query rows per K/V head
     int max_context;       // positions[s] + span is clipped to this
     unsigned page_last;    // the pool's last page (table entries outside the pool are taken as the nearest page of it)
     void* out;
@@ -1078,6 +1080,260 @@ __global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_e
     if (!early_leaves) deliver(1);
 }
 
+// ---- the form for 256 columns: K/V unpacked once per call into the products' operands ----------------------------------------
+// A pass before the attention turns the cached rows of every (sequence, K/V head) into tiles of 32 keys, 32 KiB of FP16 each: 16
+// operands of S^T = K . Q^T and 16 of O^T += V^T . P^T, every one 1 KiB in the order of the wave's lanes.  The attention kernel copies
+// a tile into LDS and reads an operand at a constant distance from the lane's own place: no conversion, no address and no bank
+// conflict in its loop.  K operand (t, b): lane (li, g) has columns 32 b + 8 g .. + 7 of key 16 t + li.  V operand j: lane (li, g) has
+// keys {4 g .., 16 + 4 g ..} of column 32 (j / 2) + 8 (li / 4) + 4 (j % 2) + li % 4, so that the results of two operands are eight
+// neighbouring columns of a lane's query row.
+constexpr int WIDE = 256, WIDE_BLOCKS = WIDE / 32, WIDE_TILES = WIDE / 16, WIDE_TILE = 2 * STEP * WIDE * 2, WIDE_ROWS = 32, WIDE_GROUP = GROUPS * WIDE_ROWS;
+// A workgroup builds a tile's K operands or its V operands.
+template<bool Q8>
+__global__ void __launch_bounds__(256) unpack_operands_kernel(PrefillArgs args, uint8_t* tiles_out, unsigned tiles_per_seq) {
+    constexpr int ROW = Q8 ? WIDE + WIDE / 16 : 2 * WIDE, PIECES = ROW / 16, ALL = STEP * PIECES;
+    const int tile = blockIdx.x / 2, value = blockIdx.x % 2, kvh = blockIdx.y, seq = blockIdx.z, thread = threadIdx.x;
+    const int position = first_position(args.positions, unsigned(seq), args.max_context);
+    const int cached = min(position + int(args.span), args.max_context);
+    if (tile * STEP >= cached) return;
+    const int32_t* table = args.page_table + size_t(seq) * args.table_stride;
+    const size_t plane_bytes = size_t(args.page_tokens) * ROW;
+    __shared__ __attribute__((aligned(16))) uint8_t raw[STEP][ROW];
+    // rows past the sequence's end are never read: they are zeros
+    #pragma unroll
+    for (int first = 0; first < ALL; first += 256) {
+        const int at = first + thread, piece = at % PIECES, row = at / PIECES, token = tile * STEP + row;
+        if (at >= ALL) break;
+        uint4 bytes = {0u, 0u, 0u, 0u};
+        if (token < cached)
+            bytes = *reinterpret_cast<const uint4*>(args.pages + (size_t(pool_page(table[token / int(args.page_tokens)], args.page_last)) * 2 * args.kv_heads +
+                                                                  (value ? args.kv_heads : 0) + kvh) * plane_bytes + size_t(token % int(args.page_tokens)) * ROW + 16 * piece);
+        *reinterpret_cast<uint4*>(&raw[row][16 * piece]) = bytes;
+    }
+    __syncthreads();
+    const int lane = thread & 63, li = lane & 15, g = lane >> 4;
+    uint8_t* out = tiles_out + ((size_t(seq) * args.kv_heads + kvh) * tiles_per_seq + tile) * WIDE_TILE + 1024 * 2 * WIDE_BLOCKS * value + 16 * lane;
+    #pragma unroll
+    for (int n = 0; n < 4; ++n) {
+        const int operand = thread / 64 + 4 * n;
+        half8 x;
+        if (!value) {
+            const int b = operand % WIDE_BLOCKS;
+            const uint8_t* row = raw[16 * (operand / WIDE_BLOCKS) + li];
+            if (Q8) {
+                const uint2 bytes = *reinterpret_cast<const uint2*>(row + 32 * b + 8 * g);
+                const _Float16 scale = *reinterpret_cast<const _Float16*>(row + WIDE + 2 * b);
+                #pragma unroll
+                for (int i = 0; i < 8; ++i) x[i] = (_Float16)float(int8_t((i < 4 ? bytes.x : bytes.y) >> (8 * (i & 3)))) * scale;
+            } else x = *reinterpret_cast<const half8*>(row + 64 * b + 16 * g);
+        } else {
+            const int column = 32 * (operand / 2) + 8 * (li / 4) + 4 * (operand % 2) + li % 4;
+            #pragma unroll
+            for (int e = 0; e < 8; ++e) {
+                const uint8_t* row = raw[4 * g + (e < 4 ? e : 12 + e)];
+                if (Q8) x[e] = (_Float16)float(int8_t(row[column])) * *reinterpret_cast<const _Float16*>(row + WIDE + 2 * (column / 32));
+                else x[e] = *reinterpret_cast<const _Float16*>(row + 2 * column);
+            }
+        }
+        *reinterpret_cast<half8*>(out + 1024 * operand) = x;
+    }
+}
+
+// 128 query rows a workgroup, 32 a wave (two tiles of 16: 128 registers of outputs, 64 of queries), a step of 32 keys at a time,
+// the next tile on its way while this one is multiplied; one meeting a step.  64 KB of LDS and 256 registers: two workgroups a compute
+// unit, so that one multiplies while the other forms its weights.  A step is 64 products a wave (1024 cycles) and 32 reads of LDS: the
+// LDS (160 bytes a cycle asked of its 128 with the tiles' arrival) bounds it ahead of the products.
+// Measured, 2 x 1531 tokens of 24 heads over 2 (57.6 GFLOP): 73 us (0.78 PFLOP/s) where the kernel that converts in its loop takes 205.
+__global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_operands_kernel(PrefillArgs args, const uint8_t* tiles_in,
+                                                                                                             unsigned tiles_per_seq, unsigned first_round, unsigned splits, float* partial) {
+    // The workgroups in the order of their walks, the longest first, as many as there are compute units; then, as the second of each
+    // compute unit, from the shortest of the next as many upwards; then the rest.
+    const unsigned pairs = args.kv_heads * args.seqs, runs = (args.rows + WIDE_GROUP - 1) / WIDE_GROUP, at = blockIdx.x;
+    const unsigned second_end = min(gridDim.x, 2 * first_round), index = at < first_round || at >= second_end ? at : second_end - 1 - (at - first_round);
+    const unsigned item = index / splits, split = index % splits;
+    const int run = int(runs - 1 - item / pairs), kvh = int(item % pairs % args.kv_heads), seq = int(item % pairs / args.kv_heads);
+    const int thread = threadIdx.x, lane = thread & 63, wave = __builtin_amdgcn_readfirstlane(thread >> 6), li = lane & 15, g = lane >> 4;
+    const int position = first_position(args.positions, unsigned(seq), args.max_context);
+    const int cached = min(position + int(args.span), args.max_context);
+    const int row0 = run * WIDE_GROUP + wave * WIDE_ROWS, group_last = min(int(args.rows), (run + 1) * WIDE_GROUP) - 1;
+    const int keys = min(position + group_last / int(args.group) + 1, cached), steps = (keys + STEP - 1) / STEP;
+    const int begin = int(unsigned(steps) * split / splits), end = int(unsigned(steps) * (split + 1) / splits);
+    const bool idle = row0 >= int(args.rows);                   // a wave past the last row only helps copying
+    const int wave_first = position + row0 / int(args.group);
+    const int wave_steps = idle ? 0 : min(position + (min(int(args.rows), row0 + WIDE_ROWS) - 1) / int(args.group), keys - 1) / STEP + 1;
+    extern __shared__ __attribute__((aligned(16))) uint8_t stages[];
+    const uint8_t* const source = tiles_in + (size_t(seq) * args.kv_heads + kvh) * tiles_per_seq * WIDE_TILE;
+    const uint32_t stage0 = __builtin_amdgcn_readfirstlane(lds_address(stages));
+    const auto ask = [&](int step) {
+        const uint8_t* from = source + size_t(step) * WIDE_TILE + 8192 * wave;
+        const uint32_t to = stage0 + (step & 1) * WIDE_TILE + 8192 * wave;
+        load_run_to_lds<false, 4>(from, to, 16 * lane);
+        load_run_to_lds<false, 4>(from + 4096, to + 4096, 16 * lane);
+    };
+    half8 qf[2][WIDE_BLOCKS];
+    int limit[2];
+    #pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+        const int row = row0 + 16 * qt + li;
+        const bool real = row < int(args.rows);
+        const int span_row = real ? row / int(args.group) : 0, head = kvh * int(args.group) + (real ? row % int(args.group) : 0);
+        limit[qt] = min(real ? position + span_row : 0x7fffffff, cached - 1);
+        const size_t first = ((size_t(seq) * args.span + span_row) * args.heads + head) * WIDE;
+        #pragma unroll
+        for (int b = 0; b < WIDE_BLOCKS; ++b) {
+            half8 value = {};
+            if (real) {
+                if (args.q_f16) value = *reinterpret_cast<const half8*>(static_cast<const _Float16*>(args.q) + first + 32 * b + 8 * g);
+                else {
+                    const float* from = static_cast<const float*>(args.q) + first + 32 * b + 8 * g;
+                    #pragma unroll
+                    for (int i = 0; i < 8; ++i) value[i] = (_Float16)from[i];
+                }
+            }
+            qf[qt][b] = value;
+        }
+    }
+    floatx4 acc[2][WIDE_TILES];
+    float ref[2] = {NEG_BIG, NEG_BIG}, l[2] = {0.0f, 0.0f};           // the rows' reference maxima (base-2 exponents), the lane's share of their sums
+    #pragma unroll
+    for (int qt = 0; qt < 2; ++qt)
+        #pragma unroll
+        for (int jj = 0; jj < WIDE_TILES; ++jj) acc[qt][jj] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+    settle_loads();
+    if (begin < end) ask(begin);
+    for (int step = begin; step < end; ++step) {
+        wait_loads<0>();
+        ring_barrier();
+        if (step + 1 < end) ask(step + 1);
+        if (step >= wave_steps) continue;
+        const uint8_t* const tile = stages + (step & 1) * WIDE_TILE + 16 * lane;
+        const auto operand = [&](int n) { return *reinterpret_cast<const half8*>(tile + 1024 * n); };
+        floatx4 s[2][2];
+        #pragma unroll
+        for (int qt = 0; qt < 2; ++qt)
+            #pragma unroll
+            for (int t = 0; t < 2; ++t) s[qt][t] = floatx4{0.0f, 0.0f, 0.0f, 0.0f};
+        constexpr int AHEAD = 2;
+        half8 k[AHEAD + 1][2];
+        #pragma unroll
+        for (int b = 0; b < AHEAD; ++b) { k[b][0] = operand(b); k[b][1] = operand(WIDE_BLOCKS + b); }
+        #pragma unroll
+        for (int b = 0; b < WIDE_BLOCKS; ++b) {
+            if (b + AHEAD < WIDE_BLOCKS) { k[(b + AHEAD) % (AHEAD + 1)][0] = operand(b + AHEAD); k[(b + AHEAD) % (AHEAD + 1)][1] = operand(WIDE_BLOCKS + b + AHEAD); }
+            __builtin_amdgcn_sched_barrier(0);
+            #pragma unroll
+            for (int t = 0; t < 2; ++t)
+                #pragma unroll
+                for (int qt = 0; qt < 2; ++qt) s[qt][t] = __builtin_amdgcn_mfma_f32_16x16x32_f16(k[b % (AHEAD + 1)][t], qf[qt][b], s[qt][t], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+        constexpr int VALUES_AHEAD = 4;
+        half8 v[VALUES_AHEAD + 1];
+        #pragma unroll
+        for (int jj = 0; jj < VALUES_AHEAD; ++jj) v[jj] = operand(2 * WIDE_BLOCKS + jj);
+        if (step * STEP + STEP - 1 > wave_first) {
+            #pragma unroll
+            for (int qt = 0; qt < 2; ++qt)
+                #pragma unroll
+                for (int t = 0; t < 2; ++t)
+                    #pragma unroll
+                    for (int r = 0; r < 4; ++r)
+                        if (step * STEP + 16 * t + 4 * g + r > limit[qt]) s[qt][t][r] = -INFINITY;
+        }
+        half8 p[2];
+        #pragma unroll
+        for (int qt = 0; qt < 2; ++qt) {
+            const float top = fmaxf(fmaxf(fmaxf(s[qt][0][0], s[qt][0][1]), fmaxf(s[qt][0][2], s[qt][0][3])), fmaxf(fmaxf(s[qt][1][0], s[qt][1][1]), fmaxf(s[qt][1][2], s[qt][1][3])));
+            // (from the first step on: nothing has been seen yet; a row that sees none of a share's keys keeps that)
+            if (__any(fmaf(top, args.scale_log2, -ref[qt]) > SLACK)) {
+                asm volatile("; new reference maxima" ::: "memory");
+                const float higher = fmaxf(ref[qt], row_max(top) * args.scale_log2), alpha = __builtin_amdgcn_exp2f(ref[qt] - higher);
+                ref[qt] = higher;
+                l[qt] *= alpha;
+                #pragma unroll
+                for (int jj = 0; jj < WIDE_TILES; ++jj) acc[qt][jj] *= alpha;
+            }
+            #pragma unroll
+            for (int t = 0; t < 2; ++t)
+                #pragma unroll
+                for (int r = 0; r < 4; ++r) {
+                    const float w = __builtin_amdgcn_exp2f(fmaf(s[qt][t][r], args.scale_log2, -ref[qt]));
+                    l[qt] += w;
+                    p[qt][4 * t + r] = (_Float16)w;
+                }
+        }
+        #pragma unroll
+        for (int jj = 0; jj < WIDE_TILES; ++jj) {
+            if (jj + VALUES_AHEAD < WIDE_TILES) v[(jj + VALUES_AHEAD) % (VALUES_AHEAD + 1)] = operand(2 * WIDE_BLOCKS + jj + VALUES_AHEAD);
+            __builtin_amdgcn_sched_barrier(0);
+            #pragma unroll
+            for (int qt = 0; qt < 2; ++qt) acc[qt][jj] = __builtin_amdgcn_mfma_f32_16x16x32_f16(v[jj % (VALUES_AHEAD + 1)], p[qt], acc[qt][jj], 0, 0, 0);
+            __builtin_amdgcn_sched_barrier(0);
+        }
+    }
+    #pragma unroll
+    for (int qt = 0; qt < 2; ++qt) {
+        const int row = row0 + 16 * qt + li;
+        const float sum = row_sum(l[qt]);
+        if (row >= int(args.rows)) continue;
+        if (splits > 1) {
+            const size_t at = (size_t(item) * splits + split) * WIDE_GROUP + (row - run * WIDE_GROUP), all = size_t(gridDim.x) * WIDE_GROUP;
+            #pragma unroll
+            for (int jj = 0; jj < WIDE_TILES; ++jj) *reinterpret_cast<floatx4*>(partial + at * WIDE + 32 * (jj / 2) + 8 * g + 4 * (jj % 2)) = acc[qt][jj];
+            if (g == 0) *reinterpret_cast<float2*>(partial + all * WIDE + 2 * at) = float2{ref[qt], sum};
+            continue;
+        }
+        const float inverse = 1.0f / sum;
+        const int span_row = row / int(args.group), head = kvh * int(args.group) + row % int(args.group);
+        const size_t first = ((size_t(seq) * args.span + span_row) * args.heads + head) * WIDE + 8 * g;
+        #pragma unroll
+        for (int jj = 0; jj < WIDE_TILES; jj += 2) {
+            const floatx4 low = acc[qt][jj] * inverse, high = acc[qt][jj + 1] * inverse;
+            if (args.out_f16)
+                *reinterpret_cast<half8*>(static_cast<_Float16*>(args.out) + first + 16 * jj) =
+                    half8{(_Float16)low[0], (_Float16)low[1], (_Float16)low[2], (_Float16)low[3], (_Float16)high[0], (_Float16)high[1], (_Float16)high[2], (_Float16)high[3]};
+            else {
+                float* to = static_cast<float*>(args.out) + first + 16 * jj;
+                *reinterpret_cast<floatx4*>(to) = low; *reinterpret_cast<floatx4*>(to + 4) = high;
+            }
+        }
+    }
+}
+
+// A wave a query row: the shares of its keys under their common maximum, normalised.
+__global__ void __launch_bounds__(256) merge_shares_kernel(PrefillArgs args, const float* partial, unsigned splits) {
+    const unsigned pairs = args.kv_heads * args.seqs, runs = (args.rows + WIDE_GROUP - 1) / WIDE_GROUP, lane = threadIdx.x % 64;
+    const unsigned item = blockIdx.x / (WIDE_GROUP / 4), in_run = blockIdx.x % (WIDE_GROUP / 4) * 4 + threadIdx.x / 64;
+    const unsigned run = runs - 1 - item / pairs, kvh = item % pairs % args.kv_heads, seq = item % pairs / args.kv_heads, row = run * WIDE_GROUP + in_run;
+    if (row >= args.rows) return;
+    const size_t first = size_t(item) * splits * WIDE_GROUP + in_run;
+    const float2* const stats = reinterpret_cast<const float2*>(partial + size_t(pairs) * runs * splits * WIDE_GROUP * WIDE);
+    constexpr unsigned MOST = 16;
+    floatx4 values[MOST];
+    float2 stat[MOST];
+    #pragma unroll
+    for (unsigned i = 0; i < MOST; ++i) {
+        const size_t at = first + size_t(min(i, splits - 1)) * WIDE_GROUP;
+        if (i < splits) { values[i] = *reinterpret_cast<const floatx4*>(partial + at * WIDE + 4 * lane); stat[i] = stats[at]; }
+        else { values[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f}; stat[i] = float2{NEG_BIG, 0.0f}; }
+    }
+    float top = NEG_BIG, sum = 0.0f;
+    #pragma unroll
+    for (unsigned i = 0; i < MOST; ++i) top = fmaxf(top, stat[i].x);
+    floatx4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+    #pragma unroll
+    for (unsigned i = 0; i < MOST; ++i) {
+        const float weight = __builtin_amdgcn_exp2f(stat[i].x - top);
+        sum += stat[i].y * weight;
+        x += values[i] * weight;
+    }
+    x *= 1.0f / sum;
+    const size_t out = ((size_t(seq) * args.span + row / args.group) * args.heads + kvh * args.group + row % args.group) * WIDE + 4 * lane;
+    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+    if (args.out_f16) *reinterpret_cast<half4*>(static_cast<_Float16*>(args.out) + out) = half4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
+    else *reinterpret_cast<floatx4*>(static_cast<float*>(args.out) + out) = x;
+}
+
 // `tiles`: where the cached rows' FP16 tiles go -- the device's workspace, rebuilt whole on every call, or a buffer the caller
 // keeps between the chunks of a prompt (then `append` may carry the chunk's new rows and the count of positions still valid).
 template<int DIM, int QT, bool Q8>
@@ -1095,6 +1351,34 @@ void launch_dense(Device& d, const PrefillArgs& args, unsigned seqs, uint8_t* ti
         raise_shared_limit(d, reinterpret_cast<const void*>(&prefill_dense64_kernel<DIM>), shared);
         timed_launch(d, &prefill_dense64_kernel<DIM>, dim3((runs + 1) / 2, args.kv_heads, seqs), dim3(GROUPS * 64), shared, args, tiles, tiles_per_seq);
     } else timed_launch(d, &prefill_dense_kernel<DIM, QT>, dim3((runs + 1) / 2, args.kv_heads, seqs), dim3(TEAM * 64), shared, args, tiles, tiles_per_seq);
+}
+
+// 256 columns.  False: there is no room for the operands.
+template<bool Q8>
+bool launch_operands(Device& d, const PrefillArgs& args) {
+    const unsigned tiles_per_seq = unsigned((args.max_context + STEP - 1) / STEP);
+    const unsigned runs = (args.rows + WIDE_GROUP - 1) / WIDE_GROUP, items = runs * args.kv_heads * args.seqs;
+    // Where the walks are too few for the card they are cut into up to 16 shares of keys: a share costs its steps (about 1 us each) and
+    // a sixteenth of a step a workgroup for its sums' way through memory.
+    unsigned splits = 1, cost = 16 * tiles_per_seq;
+    for (unsigned s = 2; s <= 16 && items * s <= 2 * d.compute_units; ++s) {
+        const unsigned this_cost = 16 * ((tiles_per_seq + s - 1) / s) + items * s;
+        if (this_cost < cost) { cost = this_cost; splits = s; }
+    }
+    const uint64_t tile_bytes = checked_product({args.seqs, args.kv_heads, tiles_per_seq, uint64_t(WIDE_TILE)});
+    const uint64_t partial_bytes = splits > 1 ? uint64_t(items) * splits * WIDE_GROUP * (WIDE + 2) * 4 : 0;
+    uint8_t* tiles = static_cast<uint8_t*>(optional_space(d, tile_bytes + partial_bytes));
+    if (!tiles) return false;
+    float* partial = reinterpret_cast<float*>(tiles + tile_bytes);
+    unpack_operands_kernel<Q8><<<dim3(2 * tiles_per_seq, args.kv_heads, args.seqs), 256, 0, d.stream>>>(args, tiles, tiles_per_seq);
+    SD_CHECK(hipGetLastError());
+    raise_shared_limit(d, reinterpret_cast<const void*>(&prefill_operands_kernel), 2 * WIDE_TILE);
+    timed_launch(d, &prefill_operands_kernel, dim3(items * splits), dim3(GROUPS * 64), 2 * WIDE_TILE, args, static_cast<const uint8_t*>(tiles), tiles_per_seq, d.compute_units, splits, partial);
+    if (splits > 1) {
+        SD_CHECK(hipGetLastError());
+        merge_shares_kernel<<<items * (WIDE_GROUP / 4), 256, 0, d.stream>>>(args, partial, splits);
+    }
+    return true;
 }
 
 template<int DIM, int QT, bool Q8, int OCC>
@@ -1123,13 +1407,22 @@ void prefill_attention(Device& d, const sdx_kv_pool* pool, const int32_t* page_t
     args.group = unsigned(heads / pool->kv_heads); args.span = unsigned(span);
     args.page_table = page_table; args.table_stride = size_t(table_stride); args.positions = positions;
     args.q = q; args.q_f16 = q_f16; args.scale_log2 = scale * 1.44269504088896341f;
-    args.rows = unsigned(span * args.group); args.max_context = int(max_context);
+    args.rows = unsigned(span * args.group); args.seqs = unsigned(seqs); args.max_context = int(max_context);
     args.page_last = unsigned(std::min<uint64_t>(pool->page_count - 1, 0x7fffffffu));
     args.out = out; args.out_f16 = out_f16;
     const bool q8 = pool->row_bytes != 2 * pool->dim;
     if (pool->dim == 128) {
         if (q8) launch_dense<128, 2, true>(d, args, unsigned(seqs), nullptr, AppendArgs{}, 0); else launch_dense<128, 2, false>(d, args, unsigned(seqs), nullptr, AppendArgs{}, 0);
-    } else { if (q8) launch<256, 1, true, 2>(d, args, unsigned(seqs)); else launch<256, 1, false, 2>(d, args, unsigned(seqs)); }
+        return;
+    }
+    // Operands unpacked first (2 x 512 B a key and K/V head, written and read again) or the kernel that converts in its loop, a workgroup 64
+    // rows.  The second is the better one only for up to 128 rows a K/V head where these alone fill the card (24 heads over 2, Q8_0, first /
+    // second: 64 sequences of 8192 keys, spans of 8: 547 / 419 us, of 16: 650 / 830; 32 sequences, of 8: 293 / 412; 8 of 16384: 147 / 746;
+    // one of 2000: 24 / 96; whole prompts of 2 x 1531 tokens 89 / 226).
+    const uint64_t filled = seqs * pool->kv_heads * ((args.rows + GROUPS * 16 - 1) / (GROUPS * 16)), groups = seqs * pool->kv_heads * ((args.rows + WIDE_GROUP - 1) / WIDE_GROUP);
+    const bool converting = args.rows <= WIDE_GROUP && filled * 4 > uint64_t(d.compute_units) * 3;
+    if (!converting && (uintptr_t(q) | uintptr_t(out)) % 16 == 0 && groups < (uint64_t(1) << 24) && (q8 ? launch_operands<true>(d, args) : launch_operands<false>(d, args))) return;
+    if (q8) launch<256, 1, true, 2>(d, args, unsigned(seqs)); else launch<256, 1, false, 2>(d, args, unsigned(seqs));
 }
 
 // A prompt chunk in one call: the chunk's K/V rows appended (when given) and its queries attended, the cached rows' tiles kept in

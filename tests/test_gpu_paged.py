@@ -606,3 +606,51 @@ def test_paged_stream_probe_reads_the_whole_pool(gpu, pages, page_tokens, kv_hea
     gpu.synchronize()
     assert np.array_equal(gpu.read_buffer(buffer, 0, np.uint8, size), before)
     gpu.release(buffer)
+
+
+@pytest.mark.parametrize("fmt,span,heads,kv_heads,contexts", [("q8", 6, 24, 2, [0, 1000]), ("f16", 11, 24, 2, [0, 37, 700]), ("q8", 129, 1, 1, [2000]), ("f16", 64, 6, 3, [31]),
+                                                              ("q8", 33, 16, 1, [5, 1030]), ("q8", 6, 24, 2, [7 * i for i in range(40)]), ("q8", 8, 16, 2, [3 * i for i in range(100)])])
+def test_rows_of_256_columns_over_unpacked_operands(gpu, oracle, fmt, span, heads, kv_heads, contexts):
+    # The operands' kernel at the edges of its workgroups (128 rows) and steps (32 keys), its walks whole and in shares, and the converting
+    # kernel where many sequences fill the card or q and out are off 16-byte boundaries; a recording that finds no room for the
+    # operands, and one that does, replayed.
+    rng = np.random.default_rng(span * 100 + len(contexts))
+    dim, page_tokens = 256, 32
+    row_bytes = 272 if fmt == "q8" else 512
+    pool, buffer, host, table, tb = make_pool(gpu, oracle, rng, [c + span for c in contexts], kv_heads, dim, page_tokens, row_bytes,
+                                              dtype=np.float32 if fmt == "q8" else np.float16)
+    q = rng.standard_normal((len(contexts), span, heads, dim)).astype(np.float16).astype(np.float32)
+    scale = 1.0 / np.sqrt(dim)
+    some = sorted({0, len(contexts) // 2, len(contexts) - 1})
+    want = oracle.paged_attention(host, row_bytes, page_tokens, kv_heads, dim, table[some], np.array(contexts, np.int32)[some], q[some], scale)
+    for q_f16, out_f16 in ((True, False), (False, True)):
+        got = _run(gpu, pool, table, tb, contexts, q, span, heads, scale, q_f16, out_f16)[some]
+        assert np.abs(got - want).max() <= 2e-3 + (2.0 ** -11 * np.abs(want).max() if out_f16 else 0)
+    most = max(contexts) + span
+
+    def attend(handle, pool_at, table_at, position_at, q_at, out_at, scratch):
+        handle.paged_attention(pool_at, table_at, table.shape[1], position_at, most, q_at, False, len(contexts), span, heads, float(scale), out_at, False, scratch)
+    pb, qb, out = gpu.upload(np.array(contexts, np.int32)), gpu.upload(np.concatenate([np.zeros(2, np.float32), q.ravel()])), gpu.buffer(q.size * 4 + 8)
+    scratch = gpu.buffer(max(16, gpu.paged_attention_scratch(len(contexts), span, heads, dim, most)))
+    attend(gpu, pool, tb.base(), pb.base(), qb.at(8), out.at(8), scratch)
+    raw = gpu.read_buffer(out, 0, np.float32, q.size + 2)
+    assert np.abs(raw[2:].reshape(q.shape)[some] - want).max() <= 2e-3
+    with backend(1 << 30) as other:         # nothing run on this handle yet
+        pages = pool.page_count
+        other_pool, pages_at = other.kv_pool(pages, page_tokens, kv_heads, dim, row_bytes)
+        other.write_buffer(pages_at, 0, host)
+        tables, positions, queries, result = other.upload(table), other.upload(np.array(contexts, np.int32)), other.upload(q), other.buffer(q.size * 4)
+        room = other.buffer(scratch.size)
+        for key in (1, 2):
+            if key == 2:
+                attend(other, other_pool, tables.base(), positions.base(), queries.base(), result.base(), room)
+            other.graph_begin()
+            attend(other, other_pool, tables.base(), positions.base(), queries.base(), result.base(), room)
+            other.graph_end(key)
+        for key in (1, 2, 1, 2):
+            other.write_buffer(result, 0, np.zeros(q.size, np.float32))
+            assert other.graph_run(key)
+            raw = other.read_buffer(result, 0, np.float32, q.size)
+            assert np.abs(raw.reshape(q.shape)[some] - want).max() <= 2e-3
+    for b in (buffer, tb, pb, qb, out, scratch):
+        gpu.release(b)
