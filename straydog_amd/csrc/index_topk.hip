@@ -430,18 +430,95 @@ __device__ void top_k_row(Score score, Index index, size_t places, size_t k, int
     for (size_t i = slot + t; i < k; i += TOPK_THREADS) out[i] = -1;
 }
 
+// The same for rows of up to KEYS x 1024 places, which are read once and held: thread t has the places t, t + 1024, ...  Three passes of
+// 11, 11 and 10 bits (the first digit takes in two bits of the mantissa: scores of one order of magnitude then meet in a few
+// bins instead of one, where their additions wait for each other); the ordered pass is a ballot for each 64 neighbouring places
+// and one scan over their counts.  Bound by latency: a workgroup a row.  Measured (the call): a row of 16250 scores 15 us where
+// the passes above take 35 (five sweeps over memory, 8-bit digits), 32768 25 / 64, 500 5 / 6; 256 rows of 8256 13 / 25, 700 of 16250 49 / 117.
+template<int KEYS, class Score, class Index>
+__device__ void top_k_held_row(Score score, Index index, size_t places, size_t k, int32_t* out) {
+    constexpr int BINS = 2048, RUNS = KEYS * TOPK_WAVES;
+    static_assert(RUNS <= TOPK_THREADS, "a thread a run of 64 places");
+    __shared__ uint32_t bins[BINS], run_greater[RUNS], run_ties[RUNS];
+    __shared__ uint32_t wave_sums[TOPK_WAVES];
+    __shared__ uint32_t picked_bin, picked_rank;
+    const unsigned t = threadIdx.x, lane = t % 64, wave = t / 64;
+    const uint32_t floor = top_k_key(-INFINITY);
+    uint32_t keys[KEYS];
+    #pragma unroll
+    for (int i = 0; i < KEYS; ++i) {
+        const size_t place = t + size_t(i) * TOPK_THREADS;
+        keys[i] = place < places ? max(top_k_key(score(place)), floor) : floor;       // (what lies below minus infinity does not count either)
+    }
+    uint32_t prefix = 0, rank = uint32_t(k);
+    bool all = false;
+    #pragma unroll
+    for (int level = 0; level < 3; ++level) {
+        const int shift = level == 0 ? 21 : level == 1 ? 10 : 0, above_digit = level == 1 ? 21 : 10;
+        const uint32_t digits = level == 2 ? 1023u : 2047u;
+        bins[t] = 0; bins[t + TOPK_THREADS] = 0;
+        __syncthreads();
+        #pragma unroll
+        for (int i = 0; i < KEYS; ++i)
+            if (keys[i] > floor && (level == 0 || (keys[i] >> above_digit) == (prefix >> above_digit))) atomicAdd(&bins[(keys[i] >> shift) & digits], 1u);
+        __syncthreads();
+        // thread t holds the bins 2047 - 2 t and 2046 - 2 t: the scan counts keys in higher bins
+        const uint32_t high = bins[BINS - 1 - 2 * t], low = bins[BINS - 2 - 2 * t];
+        uint32_t live;
+        const uint32_t above = block_scan(high + low, wave_sums, live);
+        if (level == 0 && live <= k) { all = true; break; }
+        if (above < rank && above + high + low >= rank) {
+            const bool second = above + high < rank;
+            picked_bin = BINS - 1 - 2 * t - second;
+            picked_rank = rank - above - (second ? high : 0u);
+        }
+        __syncthreads();
+        prefix |= picked_bin << shift;
+        rank = picked_rank;
+    }
+    const uint32_t threshold = all ? floor : prefix, need = all ? 0u : rank;
+    #pragma unroll
+    for (int i = 0; i < KEYS; ++i) {
+        const uint64_t greater = __ballot(keys[i] > threshold), ties = __ballot(!all && keys[i] == threshold);
+        if (lane == 0) { run_greater[i * TOPK_WAVES + wave] = __popcll(greater); run_ties[i * TOPK_WAVES + wave] = __popcll(ties); }
+    }
+    __syncthreads();
+    uint32_t kept, all_ties;
+    const uint32_t greater_before = block_scan(t < RUNS ? run_greater[t] : 0u, wave_sums, kept);
+    const uint32_t ties_before = block_scan(t < RUNS ? run_ties[t] : 0u, wave_sums, all_ties);
+    if (t < RUNS) { run_greater[t] = greater_before; run_ties[t] = ties_before; }
+    __syncthreads();
+    #pragma unroll
+    for (int i = 0; i < KEYS; ++i) {
+        const bool greater = keys[i] > threshold, tie = !all && keys[i] == threshold;
+        const uint64_t below = (uint64_t(1) << lane) - 1;
+        const uint32_t ties = run_ties[i * TOPK_WAVES + wave] + __popcll(__ballot(tie) & below);
+        const uint32_t slot = run_greater[i * TOPK_WAVES + wave] + __popcll(__ballot(greater) & below) + min(ties, need);
+        if (greater || (tie && ties < need)) out[slot] = index(t + size_t(i) * TOPK_THREADS);
+    }
+    for (size_t i = kept + min(all_ties, need) + t; i < k; i += TOPK_THREADS) out[i] = -1;
+}
+
+// KEYS 0: a row of any length, read in every pass
+template<int KEYS>
 __global__ void __launch_bounds__(TOPK_THREADS) top_k_kernel(const float* scores, size_t groups, size_t score_stride, size_t k, int32_t* out) {
     const float* s = scores + size_t(blockIdx.x) * score_stride;
-    top_k_row([s](size_t g) { return s[g]; }, [](size_t g) { return int32_t(g); }, groups, k, out + size_t(blockIdx.x) * k);
+    const auto score = [s](size_t g) { return s[g]; };
+    const auto index = [](size_t g) { return int32_t(g); };
+    if constexpr (KEYS == 0) top_k_row(score, index, groups, k, out + size_t(blockIdx.x) * k);
+    else top_k_held_row<KEYS>(score, index, groups, k, out + size_t(blockIdx.x) * k);
 }
 
 // Top-k over a row's candidate groups: scores are stored in candidate order (sd_op_index_select with candidates).
+template<int KEYS>
 __global__ void __launch_bounds__(TOPK_THREADS) top_k_candidates_kernel(const float* scores, size_t score_stride, size_t groups, const int32_t* candidates,
                                                                         size_t blocks, size_t block, size_t k, int32_t* out) {
     const float* s = scores + size_t(blockIdx.x) * score_stride;
     const CandidateMap map{candidates + size_t(blockIdx.x) * blocks, block, groups};
-    top_k_row([=](size_t place) { return map.group_at(place) < groups ? s[place] : -INFINITY; },
-              [=](size_t place) { return int32_t(map.group_at(place)); }, blocks * block, k, out + size_t(blockIdx.x) * k);
+    const auto score = [=](size_t place) { return map.group_at(place) < groups ? s[place] : -INFINITY; };
+    const auto index = [=](size_t place) { return int32_t(map.group_at(place)); };
+    if constexpr (KEYS == 0) top_k_row(score, index, blocks * block, k, out + size_t(blockIdx.x) * k);
+    else top_k_held_row<KEYS>(score, index, blocks * block, k, out + size_t(blockIdx.x) * k);
 }
 
 // What the candidate pick ranks blocks by (reference gpu/ops.hpp:1952-1965): a block's highest score, and +inf for the block
@@ -1020,6 +1097,11 @@ void widen_bf16(Device& d, const void* from, float* to, size_t count) {
     SD_CHECK(hipGetLastError());
 }
 
+void launch_top_k(Device& d, const float* scores, size_t rows, size_t places, size_t stride, size_t k, int32_t* out) {
+    const auto kernel = places <= 8 * TOPK_THREADS ? top_k_kernel<8> : places <= 16 * TOPK_THREADS ? top_k_kernel<16> : places <= 32 * TOPK_THREADS ? top_k_kernel<32> : top_k_kernel<0>;
+    kernel<<<unsigned(rows), TOPK_THREADS, 0, d.stream>>>(scores, places, stride, k, out);
+}
+
 void launch_scores(Device& d, const float* q, const void* keys, bool bf16, size_t key_batch_stride, const float* weights, const int32_t* visible,
                    size_t rows, size_t groups, size_t heads, size_t dim, float scale, float* scores, size_t score_stride,
                    const int32_t* candidates, size_t blocks, size_t block) {
@@ -1236,11 +1318,12 @@ void index_select_launch(Device& value, const float* q, const float* keys, const
     const size_t stride = candidates ? size_t(scored) : size_t(groups);
     launch_scores(value, rotated, state_base(keys), state_bf16(keys), 0, weights, visible, size_t(rows), size_t(groups), size_t(heads), size_t(dim),
                   scale, scores, stride, candidates, size_t(blocks), size_t(block ? block : 1));
-    if (candidates)
-        top_k_candidates_kernel<<<unsigned(rows), TOPK_THREADS, 0, value.stream>>>(scores, stride, size_t(groups), candidates, size_t(blocks),
-                                                                                   size_t(block), size_t(k), out);
-    else
-        top_k_kernel<<<unsigned(rows), TOPK_THREADS, 0, value.stream>>>(scores, size_t(groups), stride, size_t(k), out);
+    if (candidates) {
+        const size_t places = size_t(blocks) * size_t(block);
+        const auto kernel = places <= 8 * TOPK_THREADS ? top_k_candidates_kernel<8> : places <= 16 * TOPK_THREADS ? top_k_candidates_kernel<16> :
+                            top_k_candidates_kernel<0>;                    // (with 32 and the map's arithmetic the registers spill)
+        kernel<<<unsigned(rows), TOPK_THREADS, 0, value.stream>>>(scores, stride, size_t(groups), candidates, size_t(blocks), size_t(block), size_t(k), out);
+    } else launch_top_k(value, scores, size_t(rows), size_t(groups), stride, size_t(k), out);
     SD_CHECK(hipGetLastError());
 }
 
@@ -1314,7 +1397,7 @@ int sd_op_top_k(void* handle, const float* scores, uint64_t rows, uint64_t group
     if (!rows || rows > 0x7fffffffu || !groups || !k || groups > (uint64_t(1) << 31) || k > (uint64_t(1) << 31)) throw std::runtime_error("invalid Straydog top-k shape");
     op_span(value, scores, checked_floats({rows, groups}), "scores");
     op_span(value, out, checked_floats({rows, k}), "top-k indices");
-    top_k_kernel<<<unsigned(rows), TOPK_THREADS, 0, value.stream>>>(scores, size_t(groups), size_t(groups), size_t(k), out);
+    launch_top_k(value, scores, size_t(rows), size_t(groups), size_t(groups), size_t(k), out);
     SD_OP_END
 }
 
@@ -1332,7 +1415,7 @@ int sd_op_index_candidates(void* handle, const float* scores, const int32_t* vis
     block_tops_kernel<<<dim3(checked_blocks(size_t(count), 4), unsigned(rows)), 256, 0, value.stream>>>(scores, visible, size_t(groups), size_t(block),
                                                                                                  size_t(count), scratch);
     SD_CHECK(hipGetLastError());
-    top_k_kernel<<<unsigned(rows), TOPK_THREADS, 0, value.stream>>>(scratch, size_t(count), size_t(count), size_t(blocks), out);
+    launch_top_k(value, scratch, size_t(rows), size_t(count), size_t(count), size_t(blocks), out);
     SD_OP_END
 }
 
@@ -1400,7 +1483,7 @@ int sdx_index_top_k(void* handle, const void* q_index, const void* keys, const f
     widen_bf16(value, q_index, wide_q, size_t(batch * heads * dim));
     launch_scores(value, wide_q, keys, true, size_t(groups * dim), weights, visible, size_t(batch), size_t(groups), size_t(heads), size_t(dim), scale,
                   row_scores, size_t(groups), nullptr, 0, 1);
-    top_k_kernel<<<unsigned(batch), TOPK_THREADS, 0, value.stream>>>(row_scores, size_t(groups), size_t(groups), size_t(k), indices);
+    launch_top_k(value, row_scores, size_t(batch), size_t(groups), size_t(groups), size_t(k), indices);
     SD_OP_END
 }
 

@@ -147,6 +147,22 @@ def test_top_k_matches_its_reference_with_many_ties(gpu, oracle, groups):
     gpu.release(sb); gpu.release(out)
 
 
+@pytest.mark.parametrize("groups", [1, 1023, 8192, 8193, 16384, 16385, 32768, 32769])
+def test_top_k_of_rows_that_are_held(gpu, oracle, groups):
+    # the lengths at which a thread holds 8, 16 and 32 places or the row is swept: ties at the cut, everything kept, almost nothing live
+    rng = np.random.default_rng(groups)
+    scores = np.stack([np.maximum(rng.standard_normal(groups), 0), rng.integers(0, 5, groups), np.full(groups, -np.inf), rng.standard_normal(groups) * 1e-40]).astype(np.float32)
+    scores[2, groups // 2] = -3.0
+    scores[3, ::3] = np.array([0.0, -0.0, np.inf], np.float32)[rng.integers(0, 3, len(scores[3, ::3]))]
+    sb = gpu.upload(scores)
+    for k in (1, 512, max(1, groups - 1), groups + 5):
+        out = gpu.buffer(scores.shape[0] * k * 4)
+        gpu.top_k(sb.base(), scores.shape[0], groups, k, out.base())
+        assert np.array_equal(_read(gpu, out, np.int32, scores.shape[0] * k).reshape(-1, k), oracle.top_k(scores, k)), k
+        gpu.release(out)
+    gpu.release(sb)
+
+
 def test_top_k_edge_cases(gpu, oracle):
     cases = [np.array([[1.0, 1.0, 1.0, 2.0, -np.inf, 1.0]], np.float32), np.full((1, 700), -np.inf, np.float32),
              np.zeros((3, 9000), np.float32), np.array([[0.0, -0.0, -1.0, np.inf]], np.float32)]
