@@ -407,7 +407,9 @@ __global__ void __launch_bounds__(256) interval_threshold_kernel(const float* __
 
 // ---- the selection of a row ----------------------------------------------------------------------------------------------------
 constexpr int SELECT = 512;         // threads of a row's selection
-__global__ void __launch_bounds__(SELECT) interval_select_kernel(const float* __restrict__ queries, size_t stride, const float* __restrict__ blocks, size_t pool,
+// Short phases bound by latency: two workgroups a compute unit (128 registers, 62 KB of LDS) overlap them, 1024 rows 69 us where one
+// (162 registers) takes 85; 256 rows, one a compute unit either way, 24.
+__global__ void __launch_bounds__(SELECT, 4) interval_select_kernel(const float* __restrict__ queries, size_t stride, const float* __restrict__ blocks, size_t pool,
                                                               size_t base, size_t selected, const float* __restrict__ scores, const float* __restrict__ copy,
                                                               const float2* __restrict__ key_stats, const float4* __restrict__ info,
                                                               const uint64_t* __restrict__ kept, const uint64_t* __restrict__ sure, unsigned words,
@@ -491,16 +493,21 @@ __global__ void __launch_bounds__(SELECT) interval_select_kernel(const float* __
         const unsigned head = t % 4;
         float dot = 0.0f;
         if (i < band) {
-            // (all of the block's 512 bytes asked for at once: one trip to memory, then the chain)
+            // (half of the block's 512 bytes asked for at once, the other half as its chain goes on: all of them would be 162 registers and
+            // one workgroup a compute unit instead of two)
             const float4* key = reinterpret_cast<const float4*>(copy + size_t(block_of[band_of[i]]) * COLUMNS);
             const float* q = query + head * COLUMNS;
-            float4 four[COLUMNS / 4];
+            constexpr unsigned PIECES = COLUMNS / 4, AHEAD = PIECES / 2;
+            float4 four[AHEAD];
             #pragma unroll
-            for (unsigned c = 0; c < COLUMNS / 4; ++c) four[c] = key[c];
+            for (unsigned c = 0; c < AHEAD; ++c) four[c] = key[c];
             #pragma unroll
-            for (unsigned c = 0; c < COLUMNS / 4; ++c) {
-                dot = fmaf(four[c].x, q[4 * c], dot); dot = fmaf(four[c].y, q[4 * c + 1], dot);
-                dot = fmaf(four[c].z, q[4 * c + 2], dot); dot = fmaf(four[c].w, q[4 * c + 3], dot);
+            for (unsigned c = 0; c < PIECES; ++c) {
+                const float4 x = four[c % AHEAD];
+                if (c + AHEAD < PIECES) four[c % AHEAD] = key[c + AHEAD];
+                dot = fmaf(x.x, q[4 * c], dot); dot = fmaf(x.y, q[4 * c + 1], dot);
+                dot = fmaf(x.z, q[4 * c + 2], dot); dot = fmaf(x.w, q[4 * c + 3], dot);
+                if (c % 4 == 3) __builtin_amdgcn_sched_barrier(0);      // (the query's reads stay behind it)
             }
         }
         const unsigned lane = t % 64, first = lane & ~3u;
