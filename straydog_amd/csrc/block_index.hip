@@ -27,10 +27,12 @@ namespace {
 
 constexpr int HEADS = 4, COLUMNS = 128, KEEP = 512, RING = 16;
 
+__device__ __forceinline__ float turn_angle(unsigned column, size_t position) { return float(position) / powf(1e7f, float(column % 32) / 32.0f); }
+__device__ __forceinline__ float turned(float own, float partner, unsigned column, float cosine, float sine) { return own * cosine + (column < 32 ? -partner : partner) * sine; }
 __device__ __forceinline__ float turn(float own, float partner, unsigned column, size_t position) {
     if (column >= 64) return own;
-    const float angle = float(position) / powf(1e7f, float(column % 32) / 32.0f);
-    return own * cosf(angle) + (column < 32 ? -partner : partner) * sinf(angle);
+    const float angle = turn_angle(column, position);
+    return turned(own, partner, column, cosf(angle), sinf(angle));
 }
 
 // A vector of `width` values (128 or 256), one per thread c < width: x * norm / sqrt(mean(x^2) + 1e-6), the first 64 columns turned
@@ -590,7 +592,7 @@ struct StageArgs {
     size_t stride;
     const float *q_norm, *k_norm, *index_q_norm, *index_k_norm;
     unsigned heads, kv_heads, steps;
-    const uint32_t *positions, *ropes;   // device-resident positions of the rows, or null: row r is at base + r
+    const uint32_t *positions, *ropes;   // device-resident positions of the rows (stage_prepare_kernel)
     size_t base;
     uint8_t* pages;
     unsigned page_tokens, row_bytes;
@@ -605,7 +607,7 @@ __global__ void __launch_bounds__(256) stage_prepare_kernel(StageArgs a) {
     __shared__ float values[256], sums[256];
     __shared__ __align__(16) float key[256];
     const unsigned block = blockIdx.x, c = threadIdx.x;
-    const size_t row = blockIdx.y, pos = a.positions ? a.positions[row] : a.base + row, rope = a.ropes ? a.ropes[row] : a.base + row;
+    const size_t row = blockIdx.y, pos = a.positions[row], rope = a.ropes[row];
     float* own = a.projections + row * a.stride;
     const size_t keys_at = size_t(a.heads) * 512, values_at = keys_at + size_t(a.kv_heads) * 256, index_at = keys_at + size_t(a.kv_heads) * 512;
     if (block < a.heads) {
@@ -643,6 +645,76 @@ __global__ void __launch_bounds__(256) stage_prepare_kernel(StageArgs a) {
                 const float value = normalized(x, a.index_k_norm, COLUMNS, size_t(a.ropes[r]) - 3, values, sums);
                 if (c < COLUMNS) a.blocks[c * a.pool + at / 4] = value;
             }
+        }
+    }
+}
+
+// The same vectors of a prompt chunk's rows (row r is at base + r), a wave a vector at a time: the sum of squares is formed lane by lane
+// in the halving tree's order, so there is no barrier, and a row's angles are formed once for the vectors a wave has, which
+// are all asked for before the first is summed.  Measured, 1024 rows of 24 + 2 + 4 vectors, eight a wave: 22 us (57 MB read, 29 written) where a workgroup a
+// vector takes 43 (an angle's power, cosine and sine are a third of a vector's instructions, its barriers most of its time).
+constexpr int STAGE_WAVES = 4;
+__device__ __forceinline__ float tree_of_four(const float (&x)[4], bool wide) {
+    #pragma clang fp contract(off)
+    const float first = x[0] * x[0], second = x[1] * x[1];
+    float sum = wide ? (first + x[2] * x[2]) + (second + x[3] * x[3]) : first + second;
+    #pragma unroll
+    for (unsigned offset = 32; offset; offset /= 2) sum += __shfl_down(sum, offset);
+    return __shfl(sum, 0);
+}
+template<int STAGE_EACH>
+__global__ void __launch_bounds__(64 * STAGE_WAVES) stage_rows_kernel(StageArgs a) {
+    __shared__ __align__(16) float keys[STAGE_WAVES][256];
+    const unsigned lane = threadIdx.x % 64, wave = __builtin_amdgcn_readfirstlane(threadIdx.x / 64), vectors = a.heads + a.kv_heads + HEADS;
+    const size_t row = blockIdx.y, pos = a.base + row;
+    float* own = a.projections + row * a.stride;
+    const size_t keys_at = size_t(a.heads) * 512, values_at = keys_at + size_t(a.kv_heads) * 256, index_at = keys_at + size_t(a.kv_heads) * 512;
+    const auto vector_of = [&](int i) { return (blockIdx.x * STAGE_EACH + i) * STAGE_WAVES + wave; };
+    const auto place_of = [&](unsigned v) {
+        return v < a.heads ? size_t(v) * 512 : v < a.heads + a.kv_heads ? keys_at + size_t(v - a.heads) * 256 : index_at + size_t(v - a.heads - a.kv_heads) * COLUMNS;
+    };
+    float x[STAGE_EACH][4];
+    #pragma unroll
+    for (int i = 0; i < STAGE_EACH; ++i) {
+        const unsigned v = min(vector_of(i), vectors - 1);
+        const float* from = own + place_of(v) + lane;
+        x[i][0] = from[0]; x[i][1] = from[64];
+        x[i][2] = x[i][3] = 0.0f;
+        if (v < a.heads + a.kv_heads) { x[i][2] = from[128]; x[i][3] = from[192]; }
+    }
+    const float angle = turn_angle(lane, pos), cosine = cosf(angle), sine = sinf(angle);
+    #pragma unroll
+    for (int i = 0; i < STAGE_EACH; ++i) {
+        const unsigned v = vector_of(i);
+        if (v >= vectors) return;
+        const bool wide = v < a.heads + a.kv_heads;
+        const float* norm = (v < a.heads ? a.q_norm : wide ? a.k_norm : a.index_q_norm) + lane;
+        const float denominator = sqrtf(tree_of_four(x[i], wide) / float(wide ? 256 : COLUMNS) + 1e-6f);
+        float value[4];
+        value[0] = x[i][0] * norm[0] / denominator; value[1] = x[i][1] * norm[64] / denominator;
+        if (wide) { value[2] = x[i][2] * norm[128] / denominator; value[3] = x[i][3] * norm[192] / denominator; }
+        value[0] = turned(value[0], __shfl_xor(value[0], 32), lane, cosine, sine);
+        if (v < a.heads) {
+            float* to = a.queries + (row * a.heads + v) * 256 + lane;
+            to[0] = value[0]; to[64] = value[1]; to[128] = value[2]; to[192] = value[3];
+        } else if (!wide) {
+            float* to = own + place_of(v) + lane;
+            to[0] = value[0]; to[64] = value[1];
+        } else {
+            const unsigned head = v - a.heads;
+            const long long entry = pos >= a.context ? -1 : a.page_table ? a.page_table[pos / a.page_tokens] : 0;
+            if (entry < 0 || size_t(entry) >= a.page_count) continue;      // a position outside the cache, or an entry that names no page of the pool, writes no row
+            const size_t page = size_t(entry), in_page = a.page_table ? pos % a.page_tokens : pos;
+            #pragma unroll
+            for (int j = 0; j < 4; ++j) keys[wave][lane + 64 * j] = value[j];
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // (the wave's own stretch)
+            uint8_t* target = a.pages + ((page * 2 * a.kv_heads + head) * a.page_tokens + in_page) * a.row_bytes;
+            const float4 k = *reinterpret_cast<const float4*>(&keys[wave][4 * lane]);
+            const float* from = own + values_at + size_t(head) * 256 + 4 * lane;
+            const float key4[4] = {k.x, k.y, k.z, k.w}, value4[4] = {from[0], from[1], from[2], from[3]};
+            kv_store_quad(target, lane, 256, a.row_bytes != 512, key4, true);
+            kv_store_quad(target + size_t(a.kv_heads) * a.page_tokens * a.row_bytes, lane, 256, a.row_bytes != 512, value4, true);
+            asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory");             // (read before the next key head's are written)
         }
     }
 }
@@ -894,8 +966,12 @@ int sdx_qsa_prefill_attend(void* handle, const sdx_qsa_state* state, float* proj
         args.heads = unsigned(heads); args.kv_heads = kv.kv_heads; args.steps = unsigned(steps); args.positions = nullptr; args.ropes = nullptr; args.base = size_t(base);
         args.pages = static_cast<uint8_t*>(kv.pages); args.page_tokens = kv.page_tokens; args.row_bytes = kv.row_bytes; args.page_table = state->page_table; args.page_count = size_t(kv.page_count);
         args.context = context; args.queries = static_cast<float*>(scratch); args.blocks = state->blocks; args.history = state->history; args.pool = pool;
-        // 1. rows normalised and turned, K/V rows appended (no workgroup of the grid pools: the span's blocks are pooled at once below)
-        stage_prepare_kernel<<<dim3(unsigned(heads + kv.kv_heads + HEADS), unsigned(steps)), 256, 0, value.stream>>>(args);
+        // 1. rows normalised and turned, K/V rows appended
+        // vectors a wave: as many as leave the card waves enough (the whole stage: 9 rows one 83 us, eight 92; 256 rows two 167, eight 176)
+        const auto launch_stage = [&](auto kernel, unsigned each) {
+            kernel<<<dim3(unsigned((heads + kv.kv_heads + HEADS + STAGE_WAVES * each - 1) / (STAGE_WAVES * each)), unsigned(steps)), 64 * STAGE_WAVES, 0, value.stream>>>(args);
+        };
+        if (steps >= 512) launch_stage(stage_rows_kernel<8>, 8); else if (steps >= 128) launch_stage(stage_rows_kernel<2>, 2); else launch_stage(stage_rows_kernel<1>, 1);
         SD_CHECK(hipGetLastError());
         // 2. the blocks the span completes, and the ring's newest rows
         index_at = heads * 512 + size_t(kv.kv_heads) * 512;
