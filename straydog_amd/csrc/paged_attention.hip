@@ -111,7 +111,7 @@ template<int N> __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_
 // A step's K and V slabs (32 contiguous rows each) are copied by fully coalesced 16-byte global->LDS loads into the wave's
 // own LDS stage; operands are then read from LDS in MFMA layout while the next step's copy is in flight.  OCC = the waves per
 // SIMD the variant is compiled for (its register budget).
-template<int DIM, int QT, bool Q8, int OCC>
+template<int DIM, int QT, bool Q8, int OCC, bool PARTED = false>
 __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu(OCC, OCC))) paged_attention_kernel(PagedArgs given) {
     constexpr int ROW = Q8 ? DIM + DIM / 16 : 2 * DIM, BLOCKS = DIM / 32, W = DIM / 16, TILES = DIM / 16;
     const int wave = __builtin_amdgcn_readfirstlane(threadIdx.x >> 6);
@@ -203,12 +203,12 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
         advance();
     }
     // Query rows of this K/V head: row = span_row * group + head_in_group; a lane holds row qt*16 + li as B operands.
-    // A row past the last real one holds zeros (its scores are never stored).
+    // A row past the last real one holds zeros (its scores are never stored).  (PARTED: the rows from 32 blockIdx.y on)
     half8 qf[QT][BLOCKS];
     int limit[QT];
     #pragma unroll
     for (int qt = 0; qt < QT; ++qt) {
-        const int row = qt * 16 + li;
+        const int row = (PARTED ? 32 * int(blockIdx.y) : 0) + qt * 16 + li;
         const bool real = row < int(args.rows);
         const int span_row = real ? row / int(args.group) : 0, head = kvh * int(args.group) + (real ? row % int(args.group) : 0);
         limit[qt] = real ? position + span_row : 0x7fffffff;
@@ -374,7 +374,7 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
         #pragma unroll
         for (int qt = 0; qt < QT; ++qt) {
             const float sum = SUMS_BY_PRODUCT ? l[qt] : row_sum(l[qt]);       // (a sum formed by products is whole in each of the row's lanes)
-            const int row = qt * 16 + li_after;
+            const int row = (PARTED ? 32 * int(blockIdx.y) : 0) + qt * 16 + li_after;
             if (row < int(args.rows)) {
                 float* to = out + size_t(row) * STRIDE;
                 if (g_after == 0) *reinterpret_cast<float2*>(to + DIM) = make_float2(m[qt] * args.scale_log2, sum);
@@ -472,13 +472,13 @@ uint64_t most_groups(uint64_t seqs, uint64_t kv_heads, uint64_t max_context) {
     return seqs * kv_heads * ((max_context + smallest_share * UNIT - 1) / (smallest_share * UNIT));
 }
 
-template<int DIM, int QT, bool Q8, int OCC>
+template<int DIM, int QT, bool Q8, int OCC, bool PARTED = false>
 void launch(Device& d, const PagedArgs& args, dim3 grid) {
     constexpr int slab = STEP * (Q8 ? DIM + DIM / 16 : 2 * DIM);
     const size_t shared = std::max(size_t(2) * QT * (DIM / 16 * 4 + 2) * 64 * 4, size_t(WAVES) * stages_per_wave(slab, OCC) * 2 * slab);
     if (shared > 160 * 1024) throw std::runtime_error("Straydog paged attention: too many query rows per K/V head for the decode kernel");
-    if (shared > 64 * 1024) raise_shared_limit(d, reinterpret_cast<const void*>(&paged_attention_kernel<DIM, QT, Q8, OCC>), shared);
-    timed_launch(d, &paged_attention_kernel<DIM, QT, Q8, OCC>, grid, dim3(WAVES * 64), shared, args);
+    if (shared > 64 * 1024) raise_shared_limit(d, reinterpret_cast<const void*>(&paged_attention_kernel<DIM, QT, Q8, OCC, PARTED>), shared);
+    timed_launch(d, &paged_attention_kernel<DIM, QT, Q8, OCC, PARTED>, grid, dim3(WAVES * 64), shared, args);
 }
 
 // The variants that exist: (columns, query tiles, format) -> waves per SIMD the kernel is compiled for.  One query tile is
@@ -511,6 +511,11 @@ unsigned resident_slots(const Device& d, unsigned dim, bool q8, unsigned query_t
 constexpr size_t static_scratch_bytes = size_t(16) << 20;
 static __device__ __align__(256) float scratch[static_scratch_bytes / 4];
 
+// Whether the caller's area lies in an allocation of the device (where it need not: the call can also do without).
+bool holds(Device& d, const void* at, size_t bytes) {
+    try { op_span(d, at, bytes, "attention scratch"); return true; } catch (const std::exception&) { return false; }
+}
+
 // What both entry points do once their partial-result area is known.  `timed`: the main kernel may go through the extended
 // launch when the handle is being profiled (that creates events, which the entry point that allocates nothing must not).
 void paged_attention(Device& value, const sdx_kv_pool* pool, const int32_t* page_table, uint64_t table_stride, const int32_t* positions,
@@ -526,7 +531,24 @@ void paged_attention(Device& value, const sdx_kv_pool* pool, const int32_t* page
     op_span(value, positions, checked_floats({seqs}), "query positions");
     op_span(value, q, checked_product({seqs, span, heads, pool->dim, q_f16 ? 2u : 4u}), "attention queries");
     op_span(value, out, checked_product({seqs, span, heads, pool->dim, out_f16 ? 2u : 4u}), "an attention output");
-    if (query_tiles > (pool->dim == 128 ? 4u : 2u)) {
+    // Up to 32 rows a K/V head at 256 columns (64 at 128) are one workgroup's.  At 256 columns up to 64 rows, over Q8_0 up to 128, can be
+    // runs of 32 rows that walk the same shares side by side (their keys come from memory about once, and are converted once a run),
+    // instead of a prompt's kernels, which unpack every key: the better way for batches that give each compute unit 128 keys, and
+    // with more than two runs, or over FP16 rows where the prompt's converting kernel has work for half the card, for long sequences.  (24 heads over 2, Q8_0, here / there: 36 rows, 16 sequences of 8192 keys 66 / 139 us, 64
+    // of 8192 190 / 537, one of 16384 37 / 55, one of 2000 26 / 23; 72 rows, 16 of 8192 104 / 147, 16 of 2000 55 / 47.  FP16 rows: 36 rows,
+    // 16 of 8192 103 / 166, 64 of 1500 89 / 73, 64 of 8192 347 / 347, 60 rows 354 / 402; 72 rows 571 / 434.)  The caller's scratch has to hold the partial results.
+    unsigned parts = 1;
+    if (pool->dim == 256 && query_tiles > 2 && query_tiles <= 8 && !own_partial) {
+        const bool q8 = pool->row_bytes != 2 * pool->dim;
+        const unsigned wanted = (query_tiles + 1) / 2;
+        const uint64_t items = checked_product({seqs, pool->kv_heads});
+        if (checked_product({items, (max_context + UNIT - 1) / UNIT}) >= value.compute_units && (max_context >= 8192 ? q8 || wanted == 2 : wanted == 2 && (q8 || items * 8 <= uint64_t(value.compute_units) * 3))) {
+            const uint64_t groups = std::min<uint64_t>(std::max(1u, resident_slots(value, 256, q8, 2) / wanted), most_groups(seqs, pool->kv_heads, max_context));
+            const size_t need = checked_floats({groups + items, rows, uint64_t(256) + 2});
+            if (partial && partial_bytes >= need && holds(value, partial, need)) parts = wanted;
+        }
+    }
+    if (parts == 1 && query_tiles > (pool->dim == 128 ? 4u : 2u)) {
         if (own_partial) throw std::runtime_error("Straydog paged attention: too many query rows per K/V head for the entry point that allocates nothing");
         // many rows per K/V head (a prefill chunk): every workgroup walks the keys once for a run of rows, nothing to merge
         prefill_attention(value, pool, page_table, table_stride, positions, max_context, q, q_f16, seqs, span, heads, scale, out, out_f16);
@@ -543,8 +565,8 @@ void paged_attention(Device& value, const sdx_kv_pool* pool, const int32_t* page
     args.page_last = unsigned(std::min<uint64_t>(pool->page_count - 1, 0x7fffffffu));
     const uint64_t items = checked_product({seqs, pool->kv_heads});
     if (checked_product({items, (max_context + UNIT - 1) / UNIT}) > 0x7fffffffu) throw std::runtime_error("invalid Straydog paged attention shape");
-    const unsigned slots = resident_slots(value, pool->dim, pool->row_bytes != 2 * pool->dim, query_tiles);
-    args.groups_max = unsigned(std::min<uint64_t>(tuned_groups() ? tuned_groups() : slots, most_groups(seqs, pool->kv_heads, max_context)));
+    const unsigned slots = std::max(1u, resident_slots(value, pool->dim, pool->row_bytes != 2 * pool->dim, parts > 1 ? 2 : query_tiles) / parts);
+    args.groups_max = unsigned(std::min<uint64_t>(tuned_groups() && parts == 1 ? tuned_groups() : slots, most_groups(seqs, pool->kv_heads, max_context)));
     args.share_min = smallest_share;
     const size_t need = checked_floats({uint64_t(args.groups_max) + items, rows, uint64_t(pool->dim) + 2});
     if (own_partial) {
@@ -559,9 +581,10 @@ void paged_attention(Device& value, const sdx_kv_pool* pool, const int32_t* page
     const bool profiled = value.profile;
     if (own_partial) value.profile = false;
     struct Restore { Device& d; bool profile; ~Restore() { d.profile = profile; } } restore{value, profiled};
-    const dim3 grid(args.groups_max);
+    const dim3 grid(args.groups_max, parts);
     const bool q8 = pool->row_bytes != 2 * pool->dim;
     if (pool->dim == 128) { if (q8) launch_tiles<128, true>(value, args, query_tiles, grid); else launch_tiles<128, false>(value, args, query_tiles, grid); }
+    else if (parts > 1) { if (q8) launch<256, 2, true, variant_occupancy(256, true, 2), true>(value, args, grid); else launch<256, 2, false, variant_occupancy(256, false, 2), true>(value, args, grid); }
     else { if (q8) launch_tiles<256, true>(value, args, query_tiles, grid); else launch_tiles<256, false>(value, args, query_tiles, grid); }
     SD_CHECK(hipGetLastError());
     const unsigned outputs = unsigned(checked_product({seqs, span, heads})), merge_groups = (outputs + 3) / 4;

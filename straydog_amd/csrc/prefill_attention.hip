@@ -1145,12 +1145,10 @@ __global__ void __launch_bounds__(256) unpack_operands_kernel(PrefillArgs args, 
 // LDS (160 bytes a cycle asked of its 128 with the tiles' arrival) bounds it ahead of the products.
 // Measured, 2 x 1531 tokens of 24 heads over 2 (57.6 GFLOP): 73 us (0.78 PFLOP/s) where the kernel that converts in its loop takes 205.
 __global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_operands_kernel(PrefillArgs args, const uint8_t* tiles_in,
-                                                                                                             unsigned tiles_per_seq, unsigned first_round, unsigned splits, float* partial) {
-    // The workgroups in the order of their walks, the longest first, as many as there are compute units; then, as the second of each
-    // compute unit, from the shortest of the next as many upwards; then the rest.
-    const unsigned pairs = args.kv_heads * args.seqs, runs = (args.rows + WIDE_GROUP - 1) / WIDE_GROUP, at = blockIdx.x;
-    const unsigned second_end = min(gridDim.x, 2 * first_round), index = at < first_round || at >= second_end ? at : second_end - 1 - (at - first_round);
-    const unsigned item = index / splits, split = index % splits;
+                                                                                                             unsigned tiles_per_seq, unsigned splits, float* partial) {
+    // The longest walks first.  (Paired so that a compute unit's second workgroup is the shorter the longer its first: no faster.)
+    const unsigned pairs = args.kv_heads * args.seqs, runs = (args.rows + WIDE_GROUP - 1) / WIDE_GROUP;
+    const unsigned item = blockIdx.x / splits, split = blockIdx.x % splits;
     const int run = int(runs - 1 - item / pairs), kvh = int(item % pairs % args.kv_heads), seq = int(item % pairs / args.kv_heads);
     const int thread = threadIdx.x, lane = thread & 63, wave = __builtin_amdgcn_readfirstlane(thread >> 6), li = lane & 15, g = lane >> 4;
     const int position = first_position(args.positions, unsigned(seq), args.max_context);
@@ -1373,7 +1371,7 @@ bool launch_operands(Device& d, const PrefillArgs& args) {
     unpack_operands_kernel<Q8><<<dim3(2 * tiles_per_seq, args.kv_heads, args.seqs), 256, 0, d.stream>>>(args, tiles, tiles_per_seq);
     SD_CHECK(hipGetLastError());
     raise_shared_limit(d, reinterpret_cast<const void*>(&prefill_operands_kernel), 2 * WIDE_TILE);
-    timed_launch(d, &prefill_operands_kernel, dim3(items * splits), dim3(GROUPS * 64), 2 * WIDE_TILE, args, static_cast<const uint8_t*>(tiles), tiles_per_seq, d.compute_units, splits, partial);
+    timed_launch(d, &prefill_operands_kernel, dim3(items * splits), dim3(GROUPS * 64), 2 * WIDE_TILE, args, static_cast<const uint8_t*>(tiles), tiles_per_seq, splits, partial);
     if (splits > 1) {
         SD_CHECK(hipGetLastError());
         merge_shares_kernel<<<items * (WIDE_GROUP / 4), 256, 0, d.stream>>>(args, partial, splits);
@@ -1416,11 +1414,12 @@ void prefill_attention(Device& d, const sdx_kv_pool* pool, const int32_t* page_t
         return;
     }
     // Operands unpacked first (2 x 512 B a key and K/V head, written and read again) or the kernel that converts in its loop, a workgroup 64
-    // rows.  The second is the better one only for up to 128 rows a K/V head where these alone fill the card (24 heads over 2, Q8_0, first /
-    // second: 64 sequences of 8192 keys, spans of 8: 547 / 419 us, of 16: 650 / 830; 32 sequences, of 8: 293 / 412; 8 of 16384: 147 / 746;
-    // one of 2000: 24 / 96; whole prompts of 2 x 1531 tokens 89 / 226).
-    const uint64_t filled = seqs * pool->kv_heads * ((args.rows + GROUPS * 16 - 1) / (GROUPS * 16)), groups = seqs * pool->kv_heads * ((args.rows + WIDE_GROUP - 1) / WIDE_GROUP);
-    const bool converting = args.rows <= WIDE_GROUP && filled * 4 > uint64_t(d.compute_units) * 3;
+    // rows.  The second is the better one only for up to 128 rows a K/V head of so many sequences that these alone give half the card a
+    // workgroup (24 heads over 2, Q8_0, first / second: 64 sequences of 8192 keys, 72 rows 543 / 410 us, 36 rows 537 / 414, 192 rows 650 / 830;
+    // 32 sequences, 72 rows 288 / 403; 8 of 16384 147 / 746; one of 2000 24 / 96; whole prompts of 2 x 1531 tokens 89 / 226; FP16, 36 rows, 64
+    // of 1500 128 / 73, 32 of 8192 319 / 342).
+    const uint64_t items = seqs * pool->kv_heads, groups = items * ((args.rows + WIDE_GROUP - 1) / WIDE_GROUP);
+    const bool converting = args.rows <= WIDE_GROUP && items * 8 > uint64_t(d.compute_units) * 3;
     if (!converting && (uintptr_t(q) | uintptr_t(out)) % 16 == 0 && groups < (uint64_t(1) << 24) && (q8 ? launch_operands<true>(d, args) : launch_operands<false>(d, args))) return;
     if (q8) launch<256, 1, true, 2>(d, args, unsigned(seqs)); else launch<256, 1, false, 2>(d, args, unsigned(seqs));
 }

@@ -654,3 +654,24 @@ def test_rows_of_256_columns_over_unpacked_operands(gpu, oracle, fmt, span, head
             assert np.abs(raw.reshape(q.shape)[some] - want).max() <= 2e-3
     for b in (buffer, tb, pb, qb, out, scratch):
         gpu.release(b)
+
+
+@pytest.mark.parametrize("fmt,span,heads,kv_heads,contexts", [("q8", 3, 24, 2, [16400]), ("q8", 8, 16, 2, [4000, 9001]), ("f16", 5, 24, 2, [12000, 5000, 100, 0]), ("q8", 6, 24, 2, [8200, 31]),
+                                                              ("q8", 8, 16, 1, [20000])])
+def test_verify_spans_of_256_columns_in_runs_of_rows(gpu, oracle, fmt, span, heads, kv_heads, contexts):
+    # 33 to 128 rows a K/V head over long batches: runs of 32 rows over the same shares; with scratch too small for their partial results
+    # the prompt's kernels take the call, as they take shorter ones
+    rng = np.random.default_rng(span * 1000 + len(contexts))
+    dim, page_tokens, row_bytes = 256, 256, 272 if fmt == "q8" else 512
+    pool, buffer, host, table, tb = make_pool(gpu, oracle, rng, [c + span for c in contexts], kv_heads, dim, page_tokens, row_bytes,
+                                              dtype=np.float32 if fmt == "q8" else np.float16)
+    q = rng.standard_normal((len(contexts), span, heads, dim)).astype(np.float16).astype(np.float32)
+    scale = 1.0 / np.sqrt(dim)
+    want = oracle.paged_attention(host, row_bytes, page_tokens, kv_heads, dim, table, np.array(contexts, np.int32), q, scale)
+    for q_f16, out_f16 in ((True, False), (False, False)):
+        close_enough(_run(gpu, pool, table, tb, contexts, q, span, heads, scale, q_f16, out_f16), want, f"span {span} of {fmt} rows")
+    pb, qb, out, tiny = gpu.upload(np.array(contexts, np.int32)), gpu.upload(q), gpu.buffer(q.size * 4), gpu.buffer(16)
+    gpu.paged_attention(pool, tb.base(), table.shape[1], pb.base(), max(contexts) + span, qb.base(), False, len(contexts), span, heads, float(scale), out.base(), False, tiny)
+    close_enough(gpu.read_buffer(out, 0, np.float32, q.size).reshape(q.shape), want, "a scratch of 16 bytes")
+    for b in (buffer, tb, pb, qb, out, tiny):
+        gpu.release(b)
