@@ -19,6 +19,8 @@
 #include "../../include/straydog_gpu.h"
 
 #include <algorithm>
+#include <cfloat>
+#include <type_traits>
 
 using namespace sd;
 using namespace sd::paged;
@@ -57,7 +59,7 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
     floatx4* exchange = reinterpret_cast<floatx4*>(DIM == 256 ? kside : lds + 2 * SIDE);               // [wave][TQ][4][64]
 
     const unsigned last_row = a.rows * a.group - 1;
-    int limit[TQ], most = 0;
+    int limit[TQ], most = 0, least = 0x7fffffff;          // the keys a row sees; the most and the fewest of the tile's rows
     float q[TQ][COLS / 2];
     #pragma unroll
     for (int t = 0; t < TQ; ++t) {
@@ -66,6 +68,7 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
         const int seen = seen_keys(a.positions[row], a.context);
         limit[t] = at <= last_row ? seen : 0;
         most = max(most, limit[t]);
+        if (at <= last_row) least = min(least, seen);
         const float* from = a.q + (size_t(row) * a.heads + head) * DIM + wave * COLS + 4 * half;
         #pragma unroll
         for (int c = 0; c < COLS / 8; ++c) {
@@ -75,8 +78,8 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
         }
     }
     #pragma unroll
-    for (int offset = 16; offset; offset /= 2) most = max(most, __shfl_xor(most, offset));
-    most = __builtin_amdgcn_readfirstlane(most);
+    for (int offset = 16; offset; offset /= 2) { most = max(most, __shfl_xor(most, offset)); least = min(least, __shfl_xor(least, offset)); }
+    most = __builtin_amdgcn_readfirstlane(most); least = __builtin_amdgcn_readfirstlane(least);
     const unsigned steps = unsigned(most + 31) / 32;
     const unsigned begin = unsigned(uint64_t(steps) * split / a.splits), end = unsigned(uint64_t(steps) * (split + 1) / a.splits);
 
@@ -103,7 +106,8 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
     }
     settle_loads();
     if (begin < end) { ask(a.keys, kside, begin); ask(a.values, vside, begin); }
-    for (unsigned step = begin; step < end; ++step) {
+    const auto advance = [&](auto every_row_sees, unsigned step) {
+        constexpr bool WHOLE = decltype(every_row_sees)::value;
         // (loads finish in the order they were asked for: K's before V's)
         wait_loads<MINE>();
         ring_barrier();
@@ -145,10 +149,10 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
         #pragma unroll
         for (int t = 0; t < TQ; ++t) {
             float top = NEG_BIG;
-            const int keys_left = limit[t] - int(step * 32) - 4 * half;
+            [[maybe_unused]] const int keys_left = limit[t] - int(step * 32) - 4 * half;
             #pragma unroll
             for (int r = 0; r < 16; ++r) {
-                s[t][r] = 8 * (r / 4) + r % 4 < keys_left ? s[t][r] : -INFINITY;
+                if (!WHOLE) s[t][r] = 8 * (r / 4) + r % 4 < keys_left ? s[t][r] : -INFINITY;
                 top = fmaxf(top, s[t][r]);
             }
             float other = top;
@@ -173,21 +177,64 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
             }
             l[t] += sum;
         }
-        #pragma unroll
-        for (int r = 0; r < 16; ++r) {
-            const int key = 8 * (r / 4) + 4 * half + r % 4;
-            const uint8_t* from = vside + key * ROW + 16 * ((wave * (COLS / 4) + (CT * i) / 4) ^ (key & 15)) + 4 * ((CT * i) % 4);
-            float v[CT];
-            if (CT == 2) { const float2 pair = *reinterpret_cast<const float2*>(from); v[0] = pair.x; v[CT - 1] = pair.y; }
-            else v[0] = *reinterpret_cast<const float*>(from);
+        const auto key_of = [&](int r) { return 8 * (r / 4) + 4 * half + r % 4; };
+        const auto value_place = [&](int r) {
+            return reinterpret_cast<float*>(vside + key_of(r) * ROW + 16 * ((wave * (COLS / 4) + (CT * i) / 4) ^ (key_of(r) & 15)) + 4 * ((CT * i) % 4));
+        };
+        // A value that is no finite number, of a key that only some of the rows see: zero times it is not zero.  The step is then
+        // multiplied without such values, and twice more with the largest number in their places and ones for the weights of the
+        // rows that see them, which takes those rows' sums (and no others') beyond the finite.  (A wave's columns of the tile are its
+        // own: it changes them in place.)
+        bool some_odd = false;
+        if (!WHOLE) {
+            bool odd = false;
+            #pragma unroll 1
+            for (int r = 0; r < 16; ++r)
+                #pragma unroll
+                for (int c = 0; c < CT; ++c) odd |= !(fabsf(value_place(r)[c]) < INFINITY);
+            some_odd = __any(odd);
+        }
+        const auto replace = [&](bool kept) {               // the finite values kept and the others zero, or the reverse
+            #pragma unroll 1
+            for (int r = 0; r < 16; ++r) {
+                const float* from = a.values + (size_t(min(step * 32 + key_of(r), unsigned(most - 1))) * a.kv_heads + kvh) * DIM + wave * COLS + CT * i;
+                #pragma unroll
+                for (int c = 0; c < CT; ++c) {
+                    const float v = from[c];
+                    value_place(r)[c] = (fabsf(v) < INFINITY) != kept ? 0.0f : kept ? v : copysignf(FLT_MAX, v);
+                }
+            }
+        };
+        const auto multiply = [&] {
+            #pragma unroll
+            for (int r = 0; r < 16; ++r) {
+                float v[CT];
+                if (CT == 2) { const float2 pair = *reinterpret_cast<const float2*>(value_place(r)); v[0] = pair.x; v[CT - 1] = pair.y; }
+                else v[0] = value_place(r)[0];
+                #pragma unroll
+                for (int t = 0; t < TQ; ++t)
+                    #pragma unroll
+                    for (int c = 0; c < CT; ++c) acc[t][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[c], s[t][r], acc[t][c], 0, 0, 0);
+            }
+        };
+        if (!WHOLE && some_odd) replace(true);
+        multiply();
+        if (!WHOLE && some_odd) {
+            replace(false);
             #pragma unroll
             for (int t = 0; t < TQ; ++t)
                 #pragma unroll
-                for (int c = 0; c < CT; ++c) acc[t][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[c], s[t][r], acc[t][c], 0, 0, 0);
+                for (int r = 0; r < 16; ++r) s[t][r] = 8 * (r / 4) + r % 4 < limit[t] - int(step * 32) - 4 * half ? 1.0f : 0.0f;
+            #pragma unroll 1
+            for (int twice = 0; twice < 2; ++twice) multiply();
         }
         ring_barrier();
         if (step + 1 < end) ask(a.values, vside, step + 1);
-    }
+    };
+    // the steps whose keys every row sees, then those that some rows see the end of
+    unsigned step = begin;
+    for (; step < end && int(step * 32 + 32) <= least; ++step) advance(std::true_type{}, step);
+    for (; step < end; ++step) advance(std::false_type{}, step);
     ring_barrier();
     // Out through LDS, a stretch of its own for every wave: [32 query rows][COLS + 4]; then 16-byte pieces of rows.
     float* mine = reinterpret_cast<float*>(lds) + wave * 32 * (COLS + 4);

@@ -729,3 +729,30 @@ def test_dense_attention_on_the_matrix_cores(gpu, oracle, rows, heads, kv_heads,
             assert np.abs((got - want) / bound).max() <= 1.0
     for b in (qs, ks, vs, gs, ps, scratch, out):
         gpu.release(b)
+
+
+@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(40, 8, 2, 256), (40, 8, 2, 128), (3, 4, 2, 256), (3, 4, 2, 128)])
+def test_dense_attention_keeps_to_the_keys_a_row_sees(gpu, oracle, rows, heads, kv_heads, dim):
+    # keys and values that are no finite numbers: the rows before them have the results they have without them, the rows that see such a
+    # value have no finite number in its column
+    rng = np.random.default_rng(rows + dim)
+    context, bad = 200, 170
+    q = rng.standard_normal((rows, heads, dim)).astype(np.float32)
+    keys, values = (rng.standard_normal((context, kv_heads, dim)).astype(np.float32) for _ in range(2))
+    positions = np.linspace(bad - 6, bad + 5, rows).astype(np.int32)
+    values[bad, 0, 5], values[bad, 1, 6], values[bad + 2, 1, 7], keys[bad + 3] = np.inf, -np.inf, np.nan, np.nan
+    qs, ks, vs, ps = (gpu.upload(x) for x in (q, keys, values, positions))
+    pairs = rows * heads
+    scratch, out = gpu.buffer(pairs * min(64, max(1, 256 // pairs)) * (dim + 2) * 4), gpu.buffer(q.size * 4)
+    gpu.attention(qs.base(), ks.base(), vs.base(), context, ps.base(), rows, heads, kv_heads, dim, float(dim ** -0.5), None, scratch, out.base())
+    got = _read(gpu, out, np.float32, q.size).reshape(rows, kv_heads, heads // kv_heads, dim)
+    clean = [np.where(np.isfinite(x), x, 0.0).astype(np.float32) for x in (keys, values)]
+    want, bound = (x.reshape(got.shape) for x in oracle.op_attention_f64(q, clean[0], clean[1], positions, float(np.float32(dim ** -0.5)), None))
+    odd = np.zeros(got.shape, bool)
+    for r, p in enumerate(positions):
+        odd[r, 0, :, 5], odd[r, 1, :, 6], odd[r, 1, :, 7] = p >= bad, p >= bad, p >= bad + 2
+        odd[r] |= p >= bad + 3
+    assert np.isfinite(got[~odd]).all() and not np.isfinite(got[odd]).any() and odd.any() and not odd.all()
+    assert np.abs((got - want) / bound)[~odd].max() <= 1.0
+    for b in (qs, ks, vs, ps, scratch, out):
+        gpu.release(b)
