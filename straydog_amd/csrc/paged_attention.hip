@@ -17,6 +17,7 @@
 #include "paged_rows.hpp"
 
 #include <cstdlib>
+#include <type_traits>
 
 namespace sd {
 void validate_pool(Device& d, const sdx_kv_pool* pool);
@@ -394,11 +395,13 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
 // A wave per (sequence, span row, head): the segments' partial results merged and normalised (the algebra of the
 // reference's qsa_decode_merge, gpu/sparse_attention_compute.hpp:139-170).  A lane takes two columns of every segment and
 // every lane reads the segments' maxima and sums for itself (one address a wave: a broadcast), so nothing is exchanged
-// between lanes and nothing waits on LDS or a barrier: the segments are asked for sixteen at a time, all loads in flight at
-// once, under a running maximum.  Four rows a workgroup.
-template<int DIM, bool F16_OUT>
+// between lanes and nothing waits on LDS or a barrier: the segments are asked for sixteen or (MOST) thirty-two at a time, all loads
+// in flight at once, under a running maximum.  Four rows a workgroup.  Thirty-two where the launch is one round of the card and bound
+// by latency (8 sequences of up to 16384 keys, 24 heads of 256 columns: 6.0 us for 8.6; one of 65536: the pass 38.6 us for 48.3); with
+// more rows than that their registers cost more waves than they save trips (2560 rows of 17 segments: 1 us slower).
+template<int DIM, bool F16_OUT, int MOST>
 __global__ void __launch_bounds__(256) paged_merge_kernel(PagedArgs args, void* out, unsigned outputs) {
-    constexpr int STRIDE = DIM + 2, PER = DIM / 128, AT_ONCE = 16;
+    constexpr int STRIDE = DIM + 2, PER = DIM / 128;
     static_assert(DIM % 128 == 0, "a lane takes two columns of every run of 128");
     const unsigned item = blockIdx.x * 4 + threadIdx.x / 64;
     if (item >= outputs) return;
@@ -413,14 +416,15 @@ __global__ void __launch_bounds__(256) paged_merge_kernel(PagedArgs args, void* 
     for (int d = 32; d; d >>= 1) before += __shfl_xor(before, d);
     const unsigned units = unsigned(min(first_position(args.positions, seq, args.max_context) + int(args.span), args.max_context) + int(UNIT) - 1) / UNIT;
     const unsigned begin = (before * args.kv_heads + kvh * units), owner = share_owner(share, begin);
-    const unsigned used = share_owner(share, begin + units - 1) - owner + 1;
+    const unsigned used = __builtin_amdgcn_readfirstlane(share_owner(share, begin + units - 1) - owner + 1);
     const float* base = args.partial + (size_t(owner) + size_t(seq) * args.kv_heads + kvh) * args.rows * STRIDE + size_t(row) * STRIDE;
     const size_t step = size_t(args.rows) * STRIDE;
     float top = NEG_BIG, sum = 0.0f;
     float2 value[PER];
     #pragma unroll
     for (int i = 0; i < PER; ++i) value[i] = make_float2(0.0f, 0.0f);
-    for (unsigned first = 0; first < used; first += AT_ONCE) {
+    const auto take = [&](auto count, unsigned first) {
+        constexpr int AT_ONCE = decltype(count)::value;
         float2 stats[AT_ONCE], v[AT_ONCE][PER];
         #pragma unroll
         for (int c = 0; c < AT_ONCE; ++c) {
@@ -444,7 +448,10 @@ __global__ void __launch_bounds__(256) paged_merge_kernel(PagedArgs args, void* 
             #pragma unroll
             for (int i = 0; i < PER; ++i) { value[i].x += v[c][i].x * w; value[i].y += v[c][i].y * w; }
         }
-    }
+    };
+    unsigned first = 0;
+    for (; first + 16 < used; first += MOST) take(std::integral_constant<int, MOST>{}, first);
+    if (first < used) take(std::integral_constant<int, 16>{}, first);
     #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const float2 result = make_float2(value[i].x / sum, value[i].y / sum);
@@ -588,12 +595,14 @@ void paged_attention(Device& value, const sdx_kv_pool* pool, const int32_t* page
     else { if (q8) launch_tiles<256, true>(value, args, query_tiles, grid); else launch_tiles<256, false>(value, args, query_tiles, grid); }
     SD_CHECK(hipGetLastError());
     const unsigned outputs = unsigned(checked_product({seqs, span, heads})), merge_groups = (outputs + 3) / 4;
+    const auto merge = [&](auto kernel) { kernel<<<merge_groups, 256, 0, value.stream>>>(args, out, outputs); };
+    const bool one_round = merge_groups <= value.compute_units;
     if (pool->dim == 128) {
-        if (out_f16) paged_merge_kernel<128, true><<<merge_groups, 256, 0, value.stream>>>(args, out, outputs);
-        else paged_merge_kernel<128, false><<<merge_groups, 256, 0, value.stream>>>(args, out, outputs);
+        if (out_f16) merge(one_round ? paged_merge_kernel<128, true, 32> : paged_merge_kernel<128, true, 16>);
+        else merge(one_round ? paged_merge_kernel<128, false, 32> : paged_merge_kernel<128, false, 16>);
     } else {
-        if (out_f16) paged_merge_kernel<256, true><<<merge_groups, 256, 0, value.stream>>>(args, out, outputs);
-        else paged_merge_kernel<256, false><<<merge_groups, 256, 0, value.stream>>>(args, out, outputs);
+        if (out_f16) merge(one_round ? paged_merge_kernel<256, true, 32> : paged_merge_kernel<256, true, 16>);
+        else merge(one_round ? paged_merge_kernel<256, false, 32> : paged_merge_kernel<256, false, 16>);
     }
 }
 
