@@ -9,7 +9,7 @@
 // run of consecutive rows is a run of consecutive tokens with all their grouped heads and every K/V row read serves all of
 // them.  A workgroup of 8 waves (two per SIMD) walks the keys 64 at a time, the next steps' operands travelling by 16-byte
 // global->LDS loads into a ring of stages while this one is computed; one barrier per 64 keys; steps that lie wholly after
-// a wave's rows are skipped.  Two kernels:
+// a wave's rows are skipped.  The kernels:
 //   * prefill_dense_kernel (128 columns, the headline shape): a pass before it unpacks the cached rows once per call into
 //     FP16 tiles in a workspace, laid out as LDS wants them, so the kernel's loop converts nothing: it copies a tile, reads
 //     operands without bank conflicts, multiplies and exponentiates, every wave's stream pipelined by hand.  A workgroup
@@ -17,8 +17,8 @@
 //     about the same work, and writes its outputs normalised, with no merge (details at the kernels);
 //   * prefill_operands_kernel (256 columns): the same idea with tiles of 32 keys that hold the products' operands as the lanes take
 //     them, 128 rows a workgroup, two workgroups a compute unit, walks cut into shares of keys where there are few of them;
-//   * prefill_attention_kernel (256 columns, many sequences with few rows each, and the union walk): 4 x QT x 16 rows per workgroup; every wave builds its own operands from the
-//     raw rows in the stage (paged_rows.hpp); a quarter of the rows belongs to a pair of waves, one taking the first 32
+//   * prefill_attention_kernel (256 columns, many sequences with few rows each, and the union walk): 4 x QT x 16 rows per
+//     workgroup; every wave builds its own operands from the raw rows in the stage (paged_rows.hpp); a quarter of the rows belongs to a pair of waves, one taking the first 32
 //     keys of every step and one the last 32, each with its own online softmax, merged through LDS at the end; the
 //     workgroups with the longest walks are dispatched first.
 #include "paged_rows.hpp"
