@@ -13,13 +13,16 @@
 //   * A read of four columns of a key feeds four products a query tile; the C layout of S^T (lane = query row; keys 8 (r / 4) +
 //     4 (lane / 32) + r % 4) is the B operand of O^T, register r for the two keys of the lane halves.
 //   * Few query rows: the keys are cut into runs until every compute unit has two workgroups; dense_merge_kernel joins them.
-// Measured, 128 rows x 16 heads over 2 K/V heads of 256 columns at position 4096 (8.7 GFLOP): 104 us and 8 to merge (84 TFLOP/s) where the general kernel
-// (LDS-fed vector FMAs, a workgroup a row and K/V head) took 5360; one row at 4096: 17 us where it took 295, at 60: 8 where it took 31.
+//   * Values that are no finite numbers: found in the finished sums, which they always reach (a weight of zero does not silence
+//     them), and the workgroup's run is worked again in plain arithmetic (plain_attention.hpp).  Kept out of the products in the loop
+//     instead, and counted beside them by sign, they cost the loop registers: 120 us for the 115 below.
+// Measured, 128 rows x 16 heads over 2 K/V heads of 256 columns at position 4096 (8.7 GFLOP): 115 us with the merge (76 TFLOP/s) where the general kernel
+// (LDS-fed vector FMAs, a workgroup a row and K/V head) took 5360; one row at 4096: 17 us where it took 295, at 60: 10 where it took 31.
 #include "paged_rows.hpp"
+#include "plain_attention.hpp"
 #include "../../include/straydog_gpu.h"
 
 #include <algorithm>
-#include <cfloat>
 #include <type_traits>
 
 using namespace sd;
@@ -179,54 +182,17 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
         }
         const auto key_of = [&](int r) { return 8 * (r / 4) + 4 * half + r % 4; };
         const auto value_place = [&](int r) {
-            return reinterpret_cast<float*>(vside + key_of(r) * ROW + 16 * ((wave * (COLS / 4) + (CT * i) / 4) ^ (key_of(r) & 15)) + 4 * ((CT * i) % 4));
+            return reinterpret_cast<const float*>(vside + key_of(r) * ROW + 16 * ((wave * (COLS / 4) + (CT * i) / 4) ^ (key_of(r) & 15)) + 4 * ((CT * i) % 4));
         };
-        // A value that is no finite number, of a key that only some of the rows see: zero times it is not zero.  The step is then
-        // multiplied without such values, and twice more with the largest number in their places and ones for the weights of the
-        // rows that see them, which takes those rows' sums (and no others') beyond the finite.  (A wave's columns of the tile are its
-        // own: it changes them in place.)
-        bool some_odd = false;
-        if (!WHOLE) {
-            bool odd = false;
-            #pragma unroll 1
-            for (int r = 0; r < 16; ++r)
-                #pragma unroll
-                for (int c = 0; c < CT; ++c) odd |= !(fabsf(value_place(r)[c]) < INFINITY);
-            some_odd = __any(odd);
-        }
-        const auto replace = [&](bool kept) {               // the finite values kept and the others zero, or the reverse
-            #pragma unroll 1
-            for (int r = 0; r < 16; ++r) {
-                const float* from = a.values + (size_t(min(step * 32 + key_of(r), unsigned(most - 1))) * a.kv_heads + kvh) * DIM + wave * COLS + CT * i;
-                #pragma unroll
-                for (int c = 0; c < CT; ++c) {
-                    const float v = from[c];
-                    value_place(r)[c] = (fabsf(v) < INFINITY) != kept ? 0.0f : kept ? v : copysignf(FLT_MAX, v);
-                }
-            }
-        };
-        const auto multiply = [&] {
-            #pragma unroll
-            for (int r = 0; r < 16; ++r) {
-                float v[CT];
-                if (CT == 2) { const float2 pair = *reinterpret_cast<const float2*>(value_place(r)); v[0] = pair.x; v[CT - 1] = pair.y; }
-                else v[0] = value_place(r)[0];
-                #pragma unroll
-                for (int t = 0; t < TQ; ++t)
-                    #pragma unroll
-                    for (int c = 0; c < CT; ++c) acc[t][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[c], s[t][r], acc[t][c], 0, 0, 0);
-            }
-        };
-        if (!WHOLE && some_odd) replace(true);
-        multiply();
-        if (!WHOLE && some_odd) {
-            replace(false);
+        #pragma unroll
+        for (int r = 0; r < 16; ++r) {
+            float v[CT];
+            if (CT == 2) { const float2 pair = *reinterpret_cast<const float2*>(value_place(r)); v[0] = pair.x; v[CT - 1] = pair.y; }
+            else v[0] = value_place(r)[0];
             #pragma unroll
             for (int t = 0; t < TQ; ++t)
                 #pragma unroll
-                for (int r = 0; r < 16; ++r) s[t][r] = 8 * (r / 4) + r % 4 < limit[t] - int(step * 32) - 4 * half ? 1.0f : 0.0f;
-            #pragma unroll 1
-            for (int twice = 0; twice < 2; ++twice) multiply();
+                for (int c = 0; c < CT; ++c) acc[t][c] = __builtin_amdgcn_mfma_f32_32x32x2f32(v[c], s[t][r], acc[t][c], 0, 0, 0);
         }
         ring_barrier();
         if (step + 1 < end) ask(a.values, vside, step + 1);
@@ -235,17 +201,63 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
     unsigned step = begin;
     for (; step < end && int(step * 32 + 32) <= least; ++step) advance(std::true_type{}, step);
     for (; step < end; ++step) advance(std::false_type{}, step);
-    ring_barrier();
-    // Out through LDS, a stretch of its own for every wave: [32 query rows][COLS + 4]; then 16-byte pieces of rows.
-    float* mine = reinterpret_cast<float*>(lds) + wave * 32 * (COLS + 4);
-    constexpr int LANES = COLS / 4, ROWS_AT_ONCE = 64 / LANES;
-    const bool whole = a.splits == 1;
+    // Sums that are no finite numbers: a value is none (zero times it is not zero, so it has reached rows that do not see its key too), or a
+    // score.  The run is then worked again in plain arithmetic.
+    float probe = 0.0f;
     #pragma unroll
     for (int t = 0; t < TQ; ++t) {
         float sum = l[t], other = sum;
         swap_halves(sum, other);
-        sum += other;
-        const float inverse = whole ? 1.0f / sum : 1.0f;
+        l[t] = sum + other;
+        probe = fmaf(l[t], 0.0f, probe);
+        #pragma unroll
+        for (int c = 0; c < CT; ++c)
+            #pragma unroll
+            for (int r = 0; r < 16; ++r) probe = fmaf(acc[t][c][r], 0.0f, probe);
+    }
+    ring_barrier();
+    uint32_t* const odd_waves = reinterpret_cast<uint32_t*>(lds);
+    const bool odd_wave = __any(probe != 0.0f);
+    if (lane == 0) odd_waves[wave] = odd_wave;
+    ring_barrier();
+    const uint4 odds = *reinterpret_cast<const uint4*>(odd_waves);
+    const bool whole = a.splits == 1;
+    const size_t pairs = size_t(a.rows) * a.heads;
+    const auto pair_of = [&](unsigned at) { return size_t(at / a.group) * a.heads + kvh * a.group + at % a.group; };
+    if (__builtin_expect(odds.x | odds.y | odds.z | odds.w, 0)) {
+        constexpr int ROWS = 8;
+        static_assert(plain_attention_bytes(ROWS, DIM) <= 2 * SIDE, "over the keys' and values' buffers");
+        #pragma unroll 1
+        for (unsigned first = tile * 32 * TQ; first < min(tile * 32 * TQ + 32 * TQ, last_row + 1); first += ROWS) {
+            const auto row_of = [&](int row) { return min(first + row, last_row); };
+            const auto sees = [&](int row, unsigned key) { return int(key) < seen_keys(a.positions[row_of(row) / a.group], a.context); };
+            const auto row_at = [&](const float* from, unsigned key) { return PlainRow{from + (size_t(key) * a.kv_heads + kvh) * DIM, false}; };
+            plain_attention<ROWS, DIM, 256>(
+                lds, begin * 32, min(end * 32, unsigned(most)), a.scale, [&](int row, int column) { return a.q[pair_of(row_of(row)) * DIM + column]; },
+                [&](unsigned key) { return row_at(a.keys, key); }, [&](unsigned key) { return row_at(a.values, key); }, sees,
+                [&](int row, int column, float value, float top, float sum) {
+                    if (first + row > last_row) return;
+                    const size_t pair = pair_of(first + row);
+                    if (whole) {
+                        value /= sum;
+                        if (a.gate) value *= 1.0f / (1.0f + expf(-a.gate[pair * DIM + column]));
+                        a.out[pair * DIM + column] = value;
+                        return;
+                    }
+                    a.partial[(pair * a.splits + split) * DIM + column] = value;
+                    float* stats = a.partial + pairs * a.splits * DIM + (pair * a.splits + split) * 2;
+                    if (column == 0) { stats[0] = top; stats[1] = sum; }
+                });
+        }
+        return;
+    }
+    ring_barrier();
+    // Out through LDS, a stretch of its own for every wave: [32 query rows][COLS + 4]; then 16-byte pieces of rows.
+    float* mine = reinterpret_cast<float*>(lds) + wave * 32 * (COLS + 4);
+    constexpr int LANES = COLS / 4, ROWS_AT_ONCE = 64 / LANES;
+    #pragma unroll
+    for (int t = 0; t < TQ; ++t) {
+        const float inverse = whole ? 1.0f / l[t] : 1.0f;
         #pragma unroll
         for (int r = 0; r < 16; ++r) {
             const int x = 8 * (r / 4) + 4 * half + r % 4;
@@ -253,18 +265,17 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
             for (int c = 0; c < CT; ++c) mine[i * (COLS + 4) + CT * x + c] = acc[t][c][r] * inverse;
         }
         const unsigned first = tile * 32 * TQ + 32 * t;
-        const size_t pairs = size_t(a.rows) * a.heads;
         if (!whole && wave == 0 && half == 0 && first + i <= last_row) {
-            const size_t pair = size_t((first + i) / a.group) * a.heads + kvh * a.group + (first + i) % a.group;
+            const size_t pair = pair_of(first + i);
             float* stats = a.partial + pairs * a.splits * DIM + (pair * a.splits + split) * 2;
-            stats[0] = m[t]; stats[1] = sum;
+            stats[0] = m[t]; stats[1] = l[t];
         }
         #pragma unroll 4
         for (int n = 0; n < 32; n += ROWS_AT_ONCE) {
             const unsigned at = first + n + lane / LANES;
             floatx4 x = *reinterpret_cast<const floatx4*>(mine + (n + lane / LANES) * (COLS + 4) + 4 * (lane % LANES));
             if (at > last_row) continue;
-            const size_t pair = size_t(at / a.group) * a.heads + kvh * a.group + at % a.group, column = wave * COLS + 4 * (lane % LANES);
+            const size_t pair = pair_of(at), column = wave * COLS + 4 * (lane % LANES);
             if (whole) {
                 if (a.gate) {
                     const floatx4 gate = *reinterpret_cast<const floatx4*>(a.gate + pair * DIM + column);
@@ -306,9 +317,12 @@ __global__ void __launch_bounds__(256) dense_merge_kernel(DenseArgs a) {
         }
         #pragma unroll
         for (int n = 0; n < AT_ONCE; ++n) {
-            const float weight = s0 + GROUPS * n < a.splits ? __builtin_amdgcn_exp2f((tops[n] - top) * LOG2E) : 0.0f;
-            total += parts[n] * weight;
-            sum += x[n] * weight;
+            // (past the last run: its numbers again; they, and those of a run without a weight, may be none that zero silences)
+            const bool real = s0 + GROUPS * n < a.splits && tops[n] != -INFINITY;
+            const float weight = __builtin_amdgcn_exp2f((tops[n] - top) * LOG2E);
+            total += real ? parts[n] * weight : 0.0f;
+            #pragma unroll
+            for (int j = 0; j < 4; ++j) sum[j] += real ? x[n][j] * weight : 0.0f;
         }
     }
     sums[part][threadIdx.x % LANES] = sum;

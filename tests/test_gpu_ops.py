@@ -756,3 +756,57 @@ def test_dense_attention_keeps_to_the_keys_a_row_sees(gpu, oracle, rows, heads, 
     assert np.abs((got - want) / bound)[~odd].max() <= 1.0
     for b in (qs, ks, vs, ps, scratch, out):
         gpu.release(b)
+
+
+def _plain_attention(q, keys, values, positions, scale):
+    """softmax(q k) v over the keys a row sees, weights in FP32 (those too small for it are zeros) and sums in 64 bits, as the numbers'
+    own arithmetic has it where they are infinities or NaNs."""
+    rows, heads, dim = q.shape
+    group = heads // keys.shape[1]
+    out = np.zeros(q.shape)
+    with np.errstate(all="ignore"):
+        for r, p in enumerate(positions):
+            for h in range(heads):
+                k, v = keys[:p + 1, h // group].astype(np.float64), values[:p + 1, h // group].astype(np.float64)
+                scores = k @ q[r, h].astype(np.float64) * scale
+                weights = np.exp((scores - np.nanmax(scores)).astype(np.float32)).astype(np.float64)
+                out[r, h] = (weights[:, None] * v).sum(0) / weights.sum()
+    return out
+
+
+@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(1, 8, 2, 256), (1, 4, 4, 128), (40, 8, 2, 256), (40, 8, 2, 128)])
+def test_dense_attention_of_odd_values_has_their_own_sums(gpu, rows, heads, kv_heads, dim):
+    # values that are no finite numbers in steps of 32 keys that not every row sees whole: infinities of one sign stay that, of both signs
+    # (or any sign and a weight of zero) are a NaN, a NaN stays one, and the other columns are as they were
+    rng = np.random.default_rng(rows + dim)
+    context, first = 200, 165                 # the last step begins at 192, the one before at 160
+    q = np.abs(rng.standard_normal((rows, heads, dim))).astype(np.float32) + 0.5
+    keys, values = (rng.standard_normal((context, kv_heads, dim)).astype(np.float32) * x for x in (0.1, 1.0))
+    keys = keys.astype(np.float32)
+    positions = np.linspace(first + 12, first + 15, rows).astype(np.int32) if rows > 1 else np.array([first + 15], np.int32)
+    values[first, :, 0] = np.inf                                                  # one infinity
+    values[first, :, 1], values[first + 3, :, 1] = -np.inf, -np.inf               # two of one sign
+    values[first, :, 2], values[first + 1, :, 2] = np.inf, -np.inf                # both signs, neighbours
+    values[first + 2, :, 3], values[first + 9, :, 3] = -np.inf, np.inf            # both signs, apart
+    values[first + 4, :, 4] = np.nan
+    values[first + 4, :, 5] = np.copysign(np.float32(np.nan), np.float32(-1))
+    values[first + 5, :, 6], values[first + 6, :, 6] = np.nan, -np.inf
+    keys[first + 7] = -50.0                                                       # (weighs nothing in any row)
+    values[first + 7, :, 7], values[first + 7, :, 8] = np.inf, -np.inf
+    values[first + 8, :, 9] = np.finfo(np.float32).max / 1024                     # large, but finite
+    values[first + 14, :, 10] = np.inf                                            # seen by the last rows only
+    values[first + 13, :, dim - 1], values[first + 15, :, dim - 1] = -np.inf, np.inf
+    qs, ks, vs, ps = (gpu.upload(x) for x in (q, keys, values, positions))
+    pairs = rows * heads
+    scratch, out = gpu.buffer(pairs * min(64, max(1, 256 // pairs)) * (dim + 2) * 4), gpu.buffer(q.size * 4)
+    scale = float(np.float32(dim ** -0.5))
+    gpu.attention(qs.base(), ks.base(), vs.base(), context, ps.base(), rows, heads, kv_heads, dim, scale, None, scratch, out.base())
+    got, want = _read(gpu, out, np.float32, q.size).reshape(q.shape), _plain_attention(q, keys, values, positions, scale)
+    odd = ~np.isfinite(want)
+    assert np.isnan(want[..., [2, 3, 4, 5, 6, 7, 8]]).all() and np.isposinf(want[..., 0]).all() and np.isneginf(want[..., 1]).all()
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[odd & ~np.isnan(want)], want[odd & ~np.isnan(want)])
+    # (sums of up to 200 weights of FP32 products of 256 columns: below 1e-4 of the largest value in a column)
+    most = np.abs(np.where(np.isfinite(values), values, 0)).max(axis=(0, 1))
+    assert (np.abs(got[~odd] - want[~odd]) <= (1e-4 * np.broadcast_to(most, q.shape))[~odd]).all()
+    for b in (qs, ks, vs, ps, scratch, out):
+        gpu.release(b)
