@@ -202,22 +202,25 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
     for (; step < end && int(step * 32 + 32) <= least; ++step) advance(std::true_type{}, step);
     for (; step < end; ++step) advance(std::false_type{}, step);
     // Sums that are no finite numbers: a value is none (zero times it is not zero, so it has reached rows that do not see its key too), or a
-    // score.  The run is then worked again in plain arithmetic.
-    float probe = 0.0f;
+    // score.  A sum of weights that is not positive, of a row that sees keys of the run: its scores all lie below the reference
+    // maximum that stands for nothing seen.  The run is then worked again in plain arithmetic.
+    bool odd = false;
     #pragma unroll
     for (int t = 0; t < TQ; ++t) {
         float sum = l[t], other = sum;
         swap_halves(sum, other);
         l[t] = sum + other;
-        probe = fmaf(l[t], 0.0f, probe);
+        odd |= begin < end && limit[t] > int(begin * 32) && !(l[t] > 0.0f && l[t] < INFINITY);
         #pragma unroll
-        for (int c = 0; c < CT; ++c)
+        for (int c = 0; c < CT; ++c) {
+            float probe = 0.0f;
             #pragma unroll
             for (int r = 0; r < 16; ++r) probe = fmaf(acc[t][c][r], 0.0f, probe);
+            odd |= probe != 0.0f;
+        }
     }
-    ring_barrier();
-    uint32_t* const odd_waves = reinterpret_cast<uint32_t*>(lds);
-    const bool odd_wave = __any(probe != 0.0f);
+    uint32_t* const odd_waves = reinterpret_cast<uint32_t*>(lds + 2 * SIDE - 16);       // (past the stretches that outputs leave through)
+    const bool odd_wave = __any(odd);
     if (lane == 0) odd_waves[wave] = odd_wave;
     ring_barrier();
     const uint4 odds = *reinterpret_cast<const uint4*>(odd_waves);
@@ -251,10 +254,10 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
         }
         return;
     }
-    ring_barrier();
     // Out through LDS, a stretch of its own for every wave: [32 query rows][COLS + 4]; then 16-byte pieces of rows.
     float* mine = reinterpret_cast<float*>(lds) + wave * 32 * (COLS + 4);
     constexpr int LANES = COLS / 4, ROWS_AT_ONCE = 64 / LANES;
+    static_assert(4 * 32 * (COLS + 4) * 4 <= 2 * SIDE - 16, "the stretches");
     #pragma unroll
     for (int t = 0; t < TQ; ++t) {
         const float inverse = whole ? 1.0f / l[t] : 1.0f;
@@ -268,7 +271,7 @@ __global__ void __launch_bounds__(256, 2) dense_matrix_kernel(DenseArgs a) {
         if (!whole && wave == 0 && half == 0 && first + i <= last_row) {
             const size_t pair = pair_of(first + i);
             float* stats = a.partial + pairs * a.splits * DIM + (pair * a.splits + split) * 2;
-            stats[0] = m[t]; stats[1] = l[t];
+            stats[0] = l[t] > 0.0f ? m[t] : -INFINITY; stats[1] = l[t];
         }
         #pragma unroll 4
         for (int n = 0; n < 32; n += ROWS_AT_ONCE) {
@@ -300,7 +303,7 @@ __global__ void __launch_bounds__(256) dense_merge_kernel(DenseArgs a) {
     const float* stats = a.partial + pairs * a.splits * DIM + pair * a.splits * 2;
     __shared__ floatx4 sums[GROUPS][LANES];
     __shared__ float totals[GROUPS];
-    float top = NEG_BIG;
+    float top = -INFINITY;                    // (a run without a weight has that one)
     for (unsigned s = lane; s < a.splits; s += 64) top = fmaxf(top, stats[2 * s]);
     #pragma unroll
     for (int offset = 32; offset; offset /= 2) top = fmaxf(top, __shfl_xor(top, offset));

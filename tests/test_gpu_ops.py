@@ -810,3 +810,24 @@ def test_dense_attention_of_odd_values_has_their_own_sums(gpu, rows, heads, kv_h
     assert (np.abs(got[~odd] - want[~odd]) <= (1e-4 * np.broadcast_to(most, q.shape))[~odd]).all()
     for b in (qs, ks, vs, ps, scratch, out):
         gpu.release(b)
+
+
+@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(1, 8, 2, 256), (40, 4, 2, 128), (40, 8, 2, 256)])
+def test_dense_attention_of_scores_far_below_zero(gpu, rows, heads, kv_heads, dim):
+    # scores of -1e31 and beyond: the highest a row sees still takes all the weight (they lie a 200th apart, FP32 tells them apart)
+    rng = np.random.default_rng(rows + dim)
+    context = 200
+    q = np.full((rows, heads, dim), 1e16, np.float32)
+    rank = rng.permutation(context)
+    keys = np.broadcast_to((-1e15 * (1 + rank / context)).astype(np.float32)[:, None, None], (context, kv_heads, dim)).copy()
+    values = rng.standard_normal((context, kv_heads, dim)).astype(np.float32)
+    positions = np.linspace(context - 60, context - 1, rows).astype(np.int32)
+    qs, ks, vs, ps = (gpu.upload(x) for x in (q, keys, values, positions))
+    pairs = rows * heads
+    scratch, out = gpu.buffer(pairs * min(64, max(1, 256 // pairs)) * (dim + 2) * 4), gpu.buffer(q.size * 4)
+    gpu.attention(qs.base(), ks.base(), vs.base(), context, ps.base(), rows, heads, kv_heads, dim, 1.0, None, scratch, out.base())
+    got = _read(gpu, out, np.float32, q.size).reshape(rows, kv_heads, heads // kv_heads, dim)
+    for r, p in enumerate(positions):
+        assert np.abs(got[r] - values[np.argmin(rank[:p + 1])][:, None]).max() <= 1e-5
+    for b in (qs, ks, vs, ps, scratch, out):
+        gpu.release(b)
