@@ -7,7 +7,9 @@
 // three BF16 terms (value, what its rounding left, what that one's left: 24 bits, exact).  A BF16 row has one term, so a score is
 // three products a column and a value sum three (the weights' terms); a row in FP32 (the window's, or compressed rows in FP32)
 // takes the six pairs of terms above 2^-24.  Each order of magnitude has accumulators of its own, added smallest first.  An FP32 row
-// whose values fit BF16 gives the bits of the tagged BF16 row: the extra products add zeros.
+// whose values fit BF16 gives the bits of the tagged BF16 row: the extra products add zeros.  Infinities, NaNs and numbers past BF16's
+// largest make NaNs of the sums they reach: the workgroup's run is then worked again in plain arithmetic (plain_attention.hpp); the
+// test for it, once a run, is 0.5 us of one row's 54 and nothing that shows of 256 rows' 418.
 //
 // Shape of the work (wave64, one workgroup a compute unit):
 //   * a workgroup owns one query row, HT x 16 of its heads (64: a gathered row serves all heads at once) and a run of steps of 32
@@ -27,6 +29,7 @@
 // queries and outputs take 13 (67 MB); a step of BF16 rows takes 3.3 us, of which its products are 1.4 and its LDS reads, in phase with them, 0.9.  The differences from 64-bit
 // arithmetic are as large as before, 1e-6 at outputs of order one.
 #include "paged_rows.hpp"
+#include "plain_attention.hpp"
 
 #include <algorithm>
 
@@ -330,8 +333,74 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         if (wide) ring_barrier();          // the planes are written again by the next step
     }
     l = row_sum(l);
-    // out through LDS (an accumulator's four values are columns 8 apart), a stretch of its own for every wave
+    // Sums that are no finite numbers: an operand is none, or lies beyond BF16's largest (its terms, and zero weights, then make NaNs of what
+    // has nothing to do with it), or a score.  The run is worked again in plain arithmetic.
+    bool odd = !(l < INFINITY);
+    #pragma unroll
+    for (int j = 0; j < TILES; j += 4) {
+        float probe = 0.0f;
+        #pragma unroll
+        for (int i = 0; i < 16; ++i) probe = fmaf(acc[j + i / 4][i % 4], 0.0f, probe);
+        odd |= probe != 0.0f;
+    }
+    const bool odd_wave = __any(odd);
     ring_barrier();
+    if (lane == 0) seen[wave] = odd_wave;              // (outside what the outputs leave through)
+    ring_barrier();
+    uint32_t odds = 0;
+    #pragma unroll
+    for (int w = 0; w < WAVES_HERE; ++w) odds |= seen[w];
+    const int back = DIM - 2 * int(a.pairs);
+    float* const to = a.chunks == 1 ? a.out + size_t(row) * a.heads * DIM : a.partial + size_t(blockIdx.x) * a.heads * DIM;
+    float* const stats = a.partial + size_t(gridDim.x) * a.heads * DIM + size_t(blockIdx.x) * a.heads * 2;      // (chunks > 1)
+    if (__builtin_expect(odds, 0)) {
+        constexpr int ROWS = 16;
+        static_assert(plain_attention_bytes(ROWS, DIM) <= 3 * PLANE, "over the tiles");
+        const auto key_row = [&](unsigned index) {
+            if (index < raw_steps * STEP) return PlainRow{index < raw_count ? a.raw + size_t(unsigned(first + index) % a.raw_rows) * DIM : nullptr, false};
+            const unsigned place = index - raw_steps * STEP;
+            const uint32_t at = place < a.selections ? uint32_t(selected[place]) : 0xffffffffu;
+            return PlainRow{at < a.compressed_rows ? static_cast<const uint8_t*>(a.compressed) + size_t(at) * DIM * (BF16 ? 2 : 4) : nullptr, BF16};
+        };
+        float* const results = reinterpret_cast<float*>(tiles);              // [ROWS][DIM]
+        #pragma unroll 1
+        for (int head_first = int(blockIdx.y) * 16 * HT; head_first < min(int(blockIdx.y + 1) * 16 * HT, int(a.heads)); head_first += ROWS) {
+            plain_attention<ROWS, DIM, 128 * HT>(
+                tiles, begin * STEP, end * STEP, a.scale,
+                [&](int r, int column) {
+                    const float* from = a.q + (size_t(row) * a.heads + min(head_first + r, int(a.heads) - 1)) * DIM;
+                    if (column < back) return from[column];
+                    float u = from[column & ~1], v = from[column | 1];
+                    turn(u, v, turns[(column - back) / 2]);
+                    return column & 1 ? v : u;
+                },
+                key_row, key_row, [](int, unsigned) { return true; },
+                [&](int r, int column, float value, float top, float sum) {
+                    const int h = head_first + r;
+                    if (h >= int(a.heads)) return;
+                    if (a.chunks == 1) {
+                        const float sink = a.sinks[h], higher = fmaxf(top, sink), keep = top == -INFINITY ? 0.0f : expf(top - higher);
+                        value = value * keep / (sum * keep + expf(sink - higher));
+                    } else if (column == 0) { stats[2 * h] = top; stats[2 * h + 1] = sum; }
+                    results[r * DIM + column] = value;
+                });
+            for (int i = thread; i < ROWS * DIM; i += 128 * HT) {
+                const int h = head_first + i / DIM, column = i % DIM;
+                if (h >= int(a.heads)) break;
+                float value = results[i];
+                if (a.chunks == 1 && column >= back) {
+                    double2 t = turns[(column - back) / 2];
+                    t.y = -t.y;
+                    float u = results[i & ~1], v = results[i | 1];
+                    turn(u, v, t);
+                    value = column & 1 ? v : u;
+                }
+                to[size_t(h) * DIM + column] = value;
+            }
+        }
+        return;
+    }
+    // out through LDS (an accumulator's four values are columns 8 apart), a stretch of its own for every wave
     constexpr int ROW_WORDS = HALF + 4;
     float* mine = reinterpret_cast<float*>(tiles) + wave * 16 * ROW_WORDS;
     float inverse = 1.0f;
@@ -340,8 +409,7 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
     for (int j = 0; j < TILES; ++j)
         #pragma unroll
         for (int r = 0; r < 4; ++r) mine[li * ROW_WORDS + 128 * (j / 8) + 8 * (4 * g + r) + j % 8] = acc[j][r] * inverse;
-    const int column = HALF * half + 4 * lane, back = DIM - 2 * int(a.pairs);
-    float* to = a.chunks == 1 ? a.out + size_t(row) * a.heads * DIM : a.partial + size_t(blockIdx.x) * a.heads * DIM;
+    const int column = HALF * half + 4 * lane;
     #pragma unroll 4
     for (int h = 0; h < 16; ++h) {
         if (head0 + h >= int(a.heads)) break;
@@ -359,10 +427,7 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         }
         *reinterpret_cast<floatx4*>(to + size_t(head0 + h) * DIM + column) = x;
     }
-    if (a.chunks > 1 && half == 0 && g == 0 && head < int(a.heads)) {
-        float* stats = a.partial + size_t(gridDim.x) * a.heads * DIM + (size_t(blockIdx.x) * a.heads + head) * 2;
-        stats[0] = m; stats[1] = l;
-    }
+    if (a.chunks > 1 && half == 0 && g == 0 && head < int(a.heads)) { stats[2 * head] = m; stats[2 * head + 1] = l; }
 }
 
 // (row, head): the runs merged under their common maximum with the head's sink, normalised, turned back.  The runs' pieces are
@@ -404,9 +469,12 @@ __global__ void __launch_bounds__(DIM / 4) latent_rows_merge_kernel(RowsArgs a) 
         }
         #pragma unroll
         for (unsigned i = 0; i < AT_ONCE; ++i) {
-            const float weight = c0 + i < a.chunks ? __builtin_amdgcn_exp2f((tops[i] - top) * LOG2E) : 0.0f;
-            sum += sums[i] * weight;
-            x += values[i] * weight;
+            // (past the last run: its numbers again, which may be none that zero silences)
+            const bool real = c0 + i < a.chunks;
+            const float weight = __builtin_amdgcn_exp2f((tops[i] - top) * LOG2E);
+            sum += real ? sums[i] * weight : 0.0f;
+            #pragma unroll
+            for (int j = 0; j < 4; ++j) x[j] += real ? values[i][j] * weight : 0.0f;
         }
     }
     x *= 1.0f / sum;

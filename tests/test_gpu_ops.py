@@ -831,3 +831,80 @@ def test_dense_attention_of_scores_far_below_zero(gpu, rows, heads, kv_heads, di
         assert np.abs(got[r] - values[np.argmin(rank[:p + 1])][:, None]).max() <= 1e-5
     for b in (qs, ks, vs, ps, scratch, out):
         gpu.release(b)
+
+
+def _plain_latent(q, raw, positions, window, table, selected, sinks, scale, pairs, frequencies):
+    """Window rows and selected rows as keys and values, a sink, the last columns turned and turned back: sums in 64 bits, weights in FP32
+    (those too small for it are zeros), infinities and NaNs as their own arithmetic has them."""
+    rows, heads, dim = q.shape
+    back = dim - 2 * pairs
+
+    def turned(x, angle):
+        x = x.astype(np.float64)
+        a, b = x[..., back::2].copy(), x[..., back + 1::2].copy()
+        x[..., back::2], x[..., back + 1::2] = a * np.cos(angle) - b * np.sin(angle), a * np.sin(angle) + b * np.cos(angle)
+        return x.astype(np.float32)
+    out = np.zeros(q.shape)
+    with np.errstate(all="ignore"):
+        for r, p in enumerate(positions):
+            angle = float(p) * frequencies.astype(np.float64)
+            keys = np.concatenate([raw[[i % len(raw) for i in range(max(0, p - window + 1), p + 1)]].reshape(-1, dim),
+                                   table[[i for i in selected[r] if 0 <= i < len(table)]].reshape(-1, dim)]).astype(np.float64)
+            queries = turned(q[r], angle) if pairs else q[r]
+            for h in range(heads):
+                scores = np.array([(queries[h].astype(np.float64) * k).sum() for k in keys]) * scale
+                top = np.nanmax(np.append(scores, sinks[h])) if len(scores) else sinks[h]
+                weights = np.where(scores == -np.inf, 0, np.exp((scores - top).astype(np.float32))).astype(np.float64)
+                out[r, h] = (weights[:, None] * keys).sum(0) / (weights.sum() + np.exp(np.float32(sinks[h] - top)))
+            if pairs:
+                out[r] = turned(out[r].astype(np.float32), -angle)
+    return out
+
+
+@pytest.mark.parametrize("rows,heads,selections,bf16", [(1, 64, 100, True), (1, 33, 100, False), (2, 16, 0, True), (200, 20, 33, True), (270, 40, 5, False)])
+@pytest.mark.parametrize("case", ["row of one minus infinity", "row of one infinity", "NaN", "largest value", "query of one infinity"])
+def test_latent_rows_of_odd_numbers_have_their_own_sums(gpu, oracle, rows, heads, selections, bf16, case):
+    # a number that is none, or that BF16's range does not hold, in the window, a selected row or a query: the columns and heads that it
+    # has to do with are what its own arithmetic makes of them, the others what they are without it
+    from straydog_amd.backend import tagged_bf16
+    rng = np.random.default_rng(rows + heads)
+    dim, window, groups, pairs = 512, 40, 60, 32
+    q = rng.standard_normal((rows, heads, dim)).astype(np.float32)
+    q[:, :, 7] = np.abs(q[:, :, 7]) + np.float32(0.5)             # so that an infinity in column 7 has one sign in every score
+    raw = rng.standard_normal((64, dim)).astype(np.float32)
+    bits, table = _bf16_round(oracle, rng.standard_normal((groups, dim)).astype(np.float32))
+    positions = (50 + np.arange(rows) % 3).astype(np.int32)
+    selected = rng.integers(-2, groups, size=(rows, max(selections, 1))).astype(np.int32)
+    where = [(raw, 45)] + ([(table, 11)] if selections else [])
+    selected[0, :3] = (11, 11, 5) if selections else -1
+    some = sorted({0, rows // 2, rows - 1})
+    for target, row in where:
+        if case == "row of one minus infinity":
+            target[row, 7] = -np.inf
+        elif case == "row of one infinity":
+            target[row, 7] = np.inf
+        elif case == "NaN":
+            target[row, 9] = np.nan
+        elif case == "largest value" and (target is raw or not bf16):
+            target[row, 7] = -np.finfo(np.float32).max            # (a score of -1e37 and below: the row weighs nothing)
+    if case == "query of one infinity":
+        q[0, 3, 7] = np.inf
+        raw[:, 7], table[:, 7] = -np.abs(raw[:, 7]), -np.abs(table[:, 7])
+        raw[44, 7] = 1.0
+    bits = (np.ascontiguousarray(table).view(np.uint32) >> 16).astype(np.uint16)
+    sinks = rng.standard_normal(heads).astype(np.float32)
+    freqs = (1.6e5 ** (-(2.0 * np.arange(pairs)) / (2 * pairs))).astype(np.float32)
+    scale = float(np.float32(dim ** -0.5))
+    qb, rb, pb, sb, kb, fb, cb = (gpu.upload(x) for x in (q, raw, positions, selected, sinks, freqs, bits if bf16 else table))
+    out = gpu.buffer(q.size * 4)
+    gpu.sparse_attention(qb.base(), rb.base(), len(raw), pb.base(), window, tagged_bf16(cb.base()) if bf16 else cb.base(), groups, sb.base() if selections else None,
+                         selections, kb.base(), rows, heads, dim, scale, 2 * pairs, fb.base(), None, out.base())
+    got = _read(gpu, out, np.float32, q.size).reshape(q.shape)[some]
+    want = _plain_latent(q[some], raw, positions[some], window, table, selected[some] if selections else np.full((len(some), 0), -1), sinks, scale, pairs, freqs)
+    odd = ~np.isfinite(want)
+    assert np.array_equal(np.isnan(got), np.isnan(want)) and np.array_equal(got[odd & ~np.isnan(want)], want[odd & ~np.isnan(want)])
+    assert np.abs(got[~odd] - want[~odd]).max(initial=0) < 1e-5       # (FP32's: as where every number is finite)
+    if case in ("row of one minus infinity", "largest value"):
+        assert not odd[..., 8:].any()
+    for b in (qb, rb, pb, sb, kb, fb, cb, out):
+        gpu.release(b)
