@@ -169,7 +169,7 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         exists = at < a.compressed_rows;                                                    // (a negative entry is a large unsigned one)
         return exists ? static_cast<const uint8_t*>(a.compressed) + size_t(at) * DIM * (BF16 ? 2 : 4) : reinterpret_cast<const uint8_t*>(a.raw);
     };
-    uint32_t present = 0;                    // bit j: the wave's j-th row of the step asked for ahead exists
+    uint32_t present = 0, any_row = 0;       // bit j: the wave's j-th row of the step asked for ahead, or of any step, exists
     const auto ask = [&](unsigned step) {
         present = 0;
         #pragma unroll
@@ -179,6 +179,7 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
             load_run_to_lds<false, 1>(from, lds_address(tiles + (step & 1) * PLANE + (wave + WAVES_HERE * j) * PITCH), 16 * lane);
             present |= exists ? 1u << j : 0u;
         }
+        any_row |= present;
         if (step + 1 < end) read_names(step + 1);
     };
     if (end > raw_steps) read_names(max(begin, raw_steps));
@@ -231,6 +232,7 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
                 pieces[j][0] = reinterpret_cast<const float4*>(from)[2 * lane]; pieces[j][1] = reinterpret_cast<const float4*>(from)[2 * lane + 1];
                 present |= exists ? 1u << j : 0u;
             }
+            any_row |= present;
             if (!BF16 && step >= raw_steps && step + 1 < end) read_names(step + 1);
             #pragma unroll
             for (int j = 0; j < MINE; ++j) {
@@ -334,7 +336,8 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
     }
     l = row_sum(l);
     // Sums that are no finite numbers: an operand is none, or lies beyond BF16's largest (its terms, and zero weights, then make NaNs of what
-    // has nothing to do with it), or a score.  The run is worked again in plain arithmetic.
+    // has nothing to do with it), or a score.  A head's sum of weights that is zero though there are rows: its scores lie below the reference maximum that stands for
+    // nothing seen.  The run is worked again in plain arithmetic.
     bool odd = !(l < INFINITY);
     #pragma unroll
     for (int j = 0; j < TILES; j += 4) {
@@ -343,9 +346,9 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         for (int i = 0; i < 16; ++i) probe = fmaf(acc[j + i / 4][i % 4], 0.0f, probe);
         odd |= probe != 0.0f;
     }
-    const bool odd_wave = __any(odd);
+    const uint32_t found = (__any(odd) ? 1u : 0u) | (__any(l == 0.0f) ? 2u : 0u) | (any_row ? 4u : 0u);
     ring_barrier();
-    if (lane == 0) seen[wave] = odd_wave;              // (outside what the outputs leave through)
+    if (lane == 0) seen[wave] = found;                 // (outside what the outputs leave through)
     ring_barrier();
     uint32_t odds = 0;
     #pragma unroll
@@ -353,7 +356,7 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
     const int back = DIM - 2 * int(a.pairs);
     float* const to = a.chunks == 1 ? a.out + size_t(row) * a.heads * DIM : a.partial + size_t(blockIdx.x) * a.heads * DIM;
     float* const stats = a.partial + size_t(gridDim.x) * a.heads * DIM + size_t(blockIdx.x) * a.heads * 2;      // (chunks > 1)
-    if (__builtin_expect(odds, 0)) {
+    if (__builtin_expect((odds & 1) || odds >= 6, 0)) {
         constexpr int ROWS = 16;
         static_assert(plain_attention_bytes(ROWS, DIM) <= 3 * PLANE, "over the tiles");
         const auto key_row = [&](unsigned index) {
@@ -404,7 +407,10 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
     constexpr int ROW_WORDS = HALF + 4;
     float* mine = reinterpret_cast<float*>(tiles) + wave * 16 * ROW_WORDS;
     float inverse = 1.0f;
-    if (a.chunks == 1) inverse = 1.0f / (l + __builtin_amdgcn_exp2f(fmaf(a.sinks[min(head, int(a.heads) - 1)], LOG2E, -m * LOG2E)));
+    if (a.chunks == 1) {
+        const float sink = a.sinks[min(head, int(a.heads) - 1)], top = fmaxf(l > 0.0f ? m : -INFINITY, sink), keep = l > 0.0f ? __builtin_amdgcn_exp2f((m - top) * LOG2E) : 0.0f;
+        inverse = keep / (l * keep + __builtin_amdgcn_exp2f((sink - top) * LOG2E));
+    }
     #pragma unroll
     for (int j = 0; j < TILES; ++j)
         #pragma unroll
@@ -427,7 +433,7 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         }
         *reinterpret_cast<floatx4*>(to + size_t(head0 + h) * DIM + column) = x;
     }
-    if (a.chunks > 1 && half == 0 && g == 0 && head < int(a.heads)) { stats[2 * head] = m; stats[2 * head + 1] = l; }
+    if (a.chunks > 1 && half == 0 && g == 0 && head < int(a.heads)) { stats[2 * head] = l > 0.0f ? m : -INFINITY; stats[2 * head + 1] = l; }
 }
 
 // (row, head): the runs merged under their common maximum with the head's sink, normalised, turned back.  The runs' pieces are
@@ -447,7 +453,7 @@ __global__ void __launch_bounds__(DIM / 4) latent_rows_merge_kernel(RowsArgs a) 
     }
     constexpr unsigned AT_ONCE = 8;
     const float sink = a.sinks[head];
-    float top = fmaxf(sink, NEG_BIG);
+    float top = sink;                                  // (a run without a weight has minus infinity for its maximum)
     for (unsigned c0 = 0; c0 < a.chunks; c0 += AT_ONCE) {
         float tops[AT_ONCE];
         #pragma unroll
@@ -469,8 +475,8 @@ __global__ void __launch_bounds__(DIM / 4) latent_rows_merge_kernel(RowsArgs a) 
         }
         #pragma unroll
         for (unsigned i = 0; i < AT_ONCE; ++i) {
-            // (past the last run: its numbers again, which may be none that zero silences)
-            const bool real = c0 + i < a.chunks;
+            // (past the last run: its numbers again; they, and those of a run without a weight, may be none that zero silences)
+            const bool real = c0 + i < a.chunks && tops[i] != -INFINITY;
             const float weight = __builtin_amdgcn_exp2f((tops[i] - top) * LOG2E);
             sum += real ? sums[i] * weight : 0.0f;
             #pragma unroll

@@ -908,3 +908,35 @@ def test_latent_rows_of_odd_numbers_have_their_own_sums(gpu, oracle, rows, heads
         assert not odd[..., 8:].any()
     for b in (qb, rb, pb, sb, kb, fb, cb, out):
         gpu.release(b)
+
+
+@pytest.mark.parametrize("rows,selections", [(1, 100), (300, 40)])
+@pytest.mark.parametrize("sink", [-np.inf, -np.finfo(np.float32).max, 1.0, np.inf])
+def test_latent_rows_whose_scores_lie_far_below_zero(gpu, rows, selections, sink):
+    # scores of -1e31 and beyond against a sink far below or above them, rows without any key, and sinks that are infinities
+    rng = np.random.default_rng(rows)
+    dim, window, heads, groups = 512, 8, 20, 64
+    q = np.full((rows, heads, dim), 1e16, np.float32)
+    raw = -1e15 * (1 + rng.permutation(16).astype(np.float32)[:, None] / 16 + rng.random((16, dim)).astype(np.float32) * 1e-4).astype(np.float32)
+    table = -2e15 * (1 + rng.permutation(groups).astype(np.float32)[:, None] / groups + rng.random((groups, dim)).astype(np.float32) * 1e-4).astype(np.float32)
+    raw[12:] = rng.standard_normal((4, dim)) * 1e-16          # (rows 12-15: ordinary scores)
+    positions = np.where(np.arange(rows) % 3 == 1, 15, 11).astype(np.int32)
+    if rows > 1:
+        positions[2] = -1                                     # no window row
+    selected = rng.integers(0, groups, size=(rows, selections)).astype(np.int32)
+    if rows > 1:
+        selected[2:4] = -1
+    sinks = np.full(heads, sink, np.float32)
+    sinks[1:3] = (-np.inf, 0.5)
+    raw, table = raw.astype(np.float32), table.astype(np.float32)
+    qb, rb, pb, sb, kb, cb = (gpu.upload(x) for x in (q, raw, positions, selected, sinks, table))
+    out = gpu.buffer(q.size * 4)
+    some = sorted({0, *range(min(rows, 5)), rows - 1})
+    gpu.sparse_attention(qb.base(), rb.base(), 16, pb.base(), window, cb.base(), groups, sb.base(), selections, kb.base(), rows, heads, dim, 1.0, 0, None, None, out.base())
+    got = _read(gpu, out, np.float32, q.size).reshape(q.shape)[some].astype(np.float64)
+    want = _plain_latent(q[some], raw, positions[some], window, table, selected[some], sinks, 1.0, 0, np.zeros(0))
+    assert np.array_equal(np.isnan(got), np.isnan(want))
+    finite = np.isfinite(want)
+    assert (np.abs(got[finite] - want[finite]) <= 1e-5 * np.abs(want[finite])).all()
+    for b in (qb, rb, pb, sb, kb, cb, out):
+        gpu.release(b)
