@@ -121,7 +121,8 @@ int sd_op_attention(void* handle, const float* q, const float* keys, const float
  * attends the window rows of `raw` ending at its position (position p in row p % raw_rows) and the compressed rows
  * `selected` lists (-1: none), keys = values, with a per-head sink in the max and the denominator.  `compressed` may
  * carry bit 0 (BF16 rows, gpu/ops.hpp:1205-1214).  rope_dims rotates q's last values by positions * frequencies on the
- * way in and the output back.  scratch is optional and unused by this implementation. */
+ * way in and the output back.  scratch is optional and unused by this implementation.  Refused where 8 x (dim + window + selections + 5)
+ * floats are more than a compute unit's LDS holds (160 KiB less 256 bytes): at 512 columns, more than 4595 rows. */
 int sd_op_sparse_attention(void* handle, const float* q, const float* raw, uint64_t raw_rows, const int32_t* positions, uint64_t window,
                            const float* compressed, uint64_t compressed_rows, const int32_t* selected, uint64_t selections,
                            const float* sinks, uint64_t rows, uint64_t heads, uint64_t dim, float scale, uint64_t rope_dims,

@@ -166,11 +166,18 @@ __global__ void __launch_bounds__(THREADS) latent_attention_kernel(LatentArgs a)
     }
 }
 
-void launch(Device& d, const LatentArgs& args, size_t rows, size_t total_keys, bool bf16) {
-    const size_t shared = (HB * (args.kdim + PAD) + HB * total_keys + HB) * 4;
-    if (shared > 160 * 1024 - 256) throw std::runtime_error("invalid Straydog attention shape");
-    raise_shared_limit(d, reinterpret_cast<const void*>(&latent_attention_kernel<true>), 160 * 1024 - 256);
-    raise_shared_limit(d, reinterpret_cast<const void*>(&latent_attention_kernel<false>), 160 * 1024 - 256);
+// The LDS of a row's queries and weights; refused where a compute unit has less.
+constexpr size_t SHARED_MOST = 160 * 1024 - 256;
+size_t shared_bytes(uint64_t kdim, uint64_t first_keys, uint64_t second_keys) {
+    if (first_keys > SHARED_MOST || second_keys > SHARED_MOST || (HB * (kdim + PAD) + HB * (first_keys + second_keys) + HB) * 4 > SHARED_MOST)
+        throw std::runtime_error("invalid Straydog attention shape");
+    return size_t(HB * (kdim + PAD) + HB * (first_keys + second_keys) + HB) * 4;
+}
+
+void launch(Device& d, const LatentArgs& args, size_t rows, bool bf16) {
+    const size_t shared = shared_bytes(args.kdim, args.window, args.selections);
+    raise_shared_limit(d, reinterpret_cast<const void*>(&latent_attention_kernel<true>), SHARED_MOST);
+    raise_shared_limit(d, reinterpret_cast<const void*>(&latent_attention_kernel<false>), SHARED_MOST);
     const dim3 grid(unsigned((args.heads + HB - 1) / HB), unsigned(rows));
     if (bf16) latent_attention_kernel<true><<<grid, THREADS, shared, d.stream>>>(args);
     else latent_attention_kernel<false><<<grid, THREADS, shared, d.stream>>>(args);
@@ -328,13 +335,15 @@ int sd_op_sparse_attention(void* handle, const float* q, const float* raw, uint6
         args.inverse = value.turns + value.turns_rows * value.turns_pairs;
     }
     value.turns_ready = false;
-    // rows of 512 columns: the matrix-core kernel (latent_rows.hip); the general one takes every other shape
+    // rows of 512 columns: the matrix-core kernel (latent_rows.hip); the general one takes every other shape.  What is refused is what the
+    // general one cannot hold, wherever the operands lie.
+    shared_bytes(dim, window, selections);
     if (latent_rows_supported(dim, raw_rows, window, compressed_rows, selections, q, raw, args.compressed, out)) {
         latent_rows(value, q, raw, raw_rows, positions, window, args.compressed, state_bf16(compressed), compressed_rows, selected, selections, sinks, rows, heads, scale,
                     args.pairs, frequencies, args.forward, out);
         return 0;
     }
-    launch(value, args, size_t(rows), size_t(window + selections), state_bf16(compressed));
+    launch(value, args, size_t(rows), state_bf16(compressed));
     SD_OP_END
 }
 
@@ -359,7 +368,7 @@ int sdx_latent_attention(void* handle, const void* q, const void* latents, const
     args.q_bf16 = static_cast<const uint16_t*>(q); args.compressed = latents; args.compressed_batch_stride = size_t(groups * kdim);
     args.selected = selected; args.selections = size_t(k); args.heads = size_t(heads); args.kdim = size_t(kdim); args.vdim = size_t(vdim);
     args.scale = scale; args.out = out;
-    launch(value, args, size_t(batch), size_t(k), true);
+    launch(value, args, size_t(batch), true);
     SD_OP_END
 }
 

@@ -940,3 +940,26 @@ def test_latent_rows_whose_scores_lie_far_below_zero(gpu, rows, selections, sink
     assert (np.abs(got[finite] - want[finite]) <= 1e-5 * np.abs(want[finite])).all()
     for b in (qb, rb, pb, sb, kb, cb, out):
         gpu.release(b)
+
+
+def test_sparse_attention_takes_the_same_lists_on_any_boundary(gpu):
+    # the longest window and list that the op takes do not depend on where its operands lie: 4595 rows at 512 columns
+    heads, dim, groups = 2, 512, 5000
+    rng = np.random.default_rng(3)
+    raw, table = (rng.standard_normal((n, dim)).astype(np.float32) for n in (128, groups))
+    q, selected = rng.standard_normal((1, heads, dim)).astype(np.float32), rng.integers(0, groups, 4600).astype(np.int32)
+    rb, tb, sb, kb, pb = (gpu.upload(x) for x in (raw, table, selected, np.zeros(heads, np.float32), np.array([500], np.int32)))
+    qb, out = gpu.upload(np.concatenate([q.ravel(), q.ravel()[:1], q.ravel()])), gpu.buffer(q.size * 4 + 4)
+    got = []
+    for at in (0, q.size * 4 + 4):                # (the second query lies 4 bytes off a boundary, and its output with it)
+        def attend(selections):
+            gpu.sparse_attention(qb.at(at), rb.base(), 128, pb.base(), 128, tb.base(), groups, sb.base(), selections, kb.base(), 1, heads, dim, dim ** -0.5, 0, None,
+                                 None, out.at(at % 16))
+        attend(4595 - 128)
+        got.append(_read(gpu, out, np.float32, q.size + 1)[at % 16 // 4:][:q.size])
+        for selections in (4596 - 128, 4600):
+            with pytest.raises(RuntimeError, match="invalid Straydog attention shape"):
+                attend(selections)
+    assert np.abs(got[0] - got[1]).max() < 1e-5
+    for b in (rb, tb, sb, kb, pb, qb, out):
+        gpu.release(b)
