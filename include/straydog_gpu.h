@@ -60,7 +60,8 @@ int sd_buffer_read(void* handle, const void* buffer, uint64_t offset, void* outp
 /* reference straydog_gpu.h:177-183 (gpu/kernels.cpp:4765-4813): between sd_graph_begin and sd_graph_end (keep: store it under key,
  * replacing any; else drop it) the ops queued on the device's stream are recorded rather than run; only ops with no host data
  * (no buffer writes) that allocate nothing may be recorded.  sd_graph_run queues a recorded graph: 0, or 1 when none is stored
- * under key. */
+ * under key.  Recorded graphs hold the addresses of the library's own workspaces: they are dropped where one of those moves, and where an
+ * allocation only fits the budget (or the card) once the workspaces that ops can do without are given back. */
 int sd_graph_begin(void* handle);
 int sd_graph_end(void* handle, uint64_t key, int keep);
 int sd_graph_run(void* handle, uint64_t key);

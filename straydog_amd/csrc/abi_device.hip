@@ -56,9 +56,12 @@ static void* try_allocate(Device& d, size_t bytes, bool zero) {
     return pointer;
 }
 
-// The optional workspaces back to the budget; false: there were none (or a graph is being recorded, which may hold them).
-static bool give_back_optional_spaces(Device& d) {
+// The optional workspaces given back where `bytes` then fit into the `room` there is without them, and the graphs that may hold them
+// dropped.  False: nothing has changed -- they would not do, there are none, or a graph is being recorded, which may hold them too.
+static bool give_back_optional_spaces(Device& d, size_t bytes, size_t room) {
     if (d.optional_spaces.empty() || d.recording) return false;
+    for (const auto& space : d.optional_spaces) room += space.second + allocation_tail;
+    if (bytes > room || allocation_tail > room - bytes) return false;
     drop_recorded_graphs(d);
     for (const auto& space : d.optional_spaces) release(d, space.first);
     d.optional_spaces.clear();
@@ -66,11 +69,15 @@ static bool give_back_optional_spaces(Device& d) {
 }
 
 void* allocate(Device& d, size_t bytes, bool zero) {
-    const auto available = [&] { return d.budget > d.used ? d.budget - d.used : 0; };
-    const auto over = [&] { return !bytes || bytes > available() || allocation_tail > available() - bytes; };
-    if (over() && (!bytes || !give_back_optional_spaces(d) || over())) throw std::runtime_error(budget_exceeded(d, bytes));
+    const size_t available = d.budget > d.used ? d.budget - d.used : 0;
+    const bool over = !bytes || bytes > available || allocation_tail > available - bytes;
+    if (over && (!bytes || !give_back_optional_spaces(d, bytes, available))) throw std::runtime_error(budget_exceeded(d, bytes));
     void* pointer = try_allocate(d, bytes, zero);
-    if (!pointer && give_back_optional_spaces(d)) pointer = try_allocate(d, bytes, zero);
+    if (!pointer) {
+        size_t free_now = 0, total = 0;
+        SD_CHECK(hipMemGetInfo(&free_now, &total));
+        if (give_back_optional_spaces(d, bytes, free_now)) pointer = try_allocate(d, bytes, zero);
+    }
     if (!pointer) SD_CHECK(hipErrorOutOfMemory);
     return pointer;
 }

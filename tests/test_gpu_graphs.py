@@ -331,3 +331,59 @@ def test_batched_sparse_step_recorded(gpu, oracle):
             gpu.synchronize()
     for b in (kb, lb, qb, wb, vb, ab, indices, out):
         gpu.release(b)
+
+
+class _Dense:
+    """sd_op_attention of one row whose keys are cut into more runs than the caller's scratch holds: it takes an optional workspace."""
+
+    def __init__(self, gpu, oracle, context=4200, heads=16, kv_heads=2, dim=256):
+        rng = np.random.default_rng(context)
+        self.gpu, self.shape = gpu, (context, heads, kv_heads, dim)
+        q, keys, values = (rng.standard_normal(n).astype(np.float32) for n in ((1, heads, dim), (context, kv_heads, dim), (context, kv_heads, dim)))
+        positions = np.array([context - 1], np.int32)
+        self.buffers = [gpu.upload(x) for x in (q, keys, values, positions)]
+        self.scratch, self.out = gpu.buffer(heads * (256 // heads) * (dim + 2) * 4), gpu.buffer(q.size * 4)
+        self.want, self.bound = oracle.op_attention_f64(q, keys, values, positions, float(np.float32(dim ** -0.5)), None)
+
+    def queue(self):
+        context, heads, kv_heads, dim = self.shape
+        q, keys, values, positions = (b.base() for b in self.buffers)
+        self.gpu.attention(q, keys, values, context, positions, 1, heads, kv_heads, dim, float(dim ** -0.5), None, self.scratch, self.out.base())
+
+    def right(self, how):
+        self.gpu.write_buffer(self.out, 0, np.zeros(self.want.size, np.float32))
+        ran = how()
+        got = _read(self.gpu, self.out, np.float32, self.want.size).reshape(self.want.shape)
+        assert np.abs((got - self.want) / self.bound).max() <= 1.0
+        return ran
+
+
+def test_optional_workspaces_are_given_back_where_that_helps(oracle):
+    # an allocation that fits once the ops' optional workspaces are gone takes them, and the graphs that hold them; one that would not fit
+    # even then is refused and leaves both as they are
+    from straydog_amd.backend import StraydogError
+    budget = 64 << 20
+    with backend(budget) as gpu:
+        work = _Dense(gpu, oracle)
+        gpu.graph_begin()
+        gpu.graph_end(7, keep=False)           # (what a first recording reserves)
+        used, before = gpu.memory()[0], gpu.device_state()[0]
+        work.right(work.queue)
+        assert before - gpu.device_state()[0] >= 2 << 20, "the op has taken a workspace"
+        gpu.graph_begin()
+        work.queue()
+        gpu.graph_end(7)
+        for size in (budget, budget << 10, budget - (8 << 20)):
+            with pytest.raises(StraydogError, match="budget exceeded"):
+                gpu.buffer(size)
+            assert work.right(lambda: gpu.graph_run(7)), "a refused allocation drops no graph"
+        rest = gpu.buffer(budget - used - 64)
+        assert not gpu.graph_run(7), "the graph that held the workspace is gone with it"
+        work.right(work.queue)                 # without room it does with the caller's scratch
+        gpu.graph_begin()
+        work.queue()
+        gpu.graph_end(7)
+        gpu.release(rest)
+        for _ in range(2):
+            work.right(work.queue)             # (with a workspace again)
+            assert work.right(lambda: gpu.graph_run(7))
