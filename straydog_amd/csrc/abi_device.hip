@@ -164,10 +164,19 @@ void* optional_space(Device& d, size_t bytes) {
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
     SD_CHECK(hipStreamIsCapturing(d.stream, &capturing));
     if (bytes > optional_space_most || capturing != hipStreamCaptureStatusNone) return nullptr;
-    const size_t rounded = std::min(optional_space_most, std::max((bytes + (size_t(4) << 20) - 1) & ~((size_t(4) << 20) - 1), 2 * held));
-    // (what is held already is not given back for this)
-    const size_t available = d.budget > d.used ? d.budget - d.used : 0;
+    // What is held already makes room where no recorded graph can hold it.  Twice its size if there is room for that, else what is asked for.
+    const bool outgrown = d.graphs.empty() && !d.optional_spaces.empty();
+    size_t available = d.budget > d.used ? d.budget - d.used : 0;
+    if (outgrown)
+        for (const auto& space : d.optional_spaces) available += space.second + allocation_tail;
+    const auto in_units = [](size_t size) { return (size + (size_t(4) << 20) - 1) & ~((size_t(4) << 20) - 1); };
+    size_t rounded = std::min(optional_space_most, std::max(in_units(bytes), in_units(2 * held)));
+    if (rounded > available || allocation_tail > available - rounded) rounded = in_units(bytes);
     if (rounded > available || allocation_tail > available - rounded) return nullptr;
+    if (outgrown) {
+        for (const auto& space : d.optional_spaces) release(d, space.first);
+        d.optional_spaces.clear();
+    }
     void* space = try_allocate(d, rounded, false);
     if (space) d.optional_spaces.emplace_back(space, rounded);
     return space;

@@ -56,7 +56,7 @@ struct Device {
     void* sequence_input = nullptr; size_t sequence_input_bytes = 0;
     void* sequence_output = nullptr; size_t sequence_output_bytes = 0;
     void* workspace = nullptr; size_t workspace_bytes = 0;
-    std::vector<std::pair<void*, size_t>> optional_spaces;      // each at least twice the one before; the last is in use
+    std::vector<std::pair<void*, size_t>> optional_spaces;      // the last is in use; recorded graphs may hold the smaller ones before it
     // The attention rope table of a pass (sd_attention_turns_reserve / _arm): forward[row][pair] = (cosine, sine), then the
     // inverse turns at the same stride.  Armed for `turns_armed` rows, the next sd_op_norm_rope of that many rows fills it;
     // ready, the next sd_op_sparse_attention of those rows reads it instead of forming the angles again.
@@ -145,7 +145,7 @@ void download(Device& d, void* output, const void* source, size_t bytes);  // de
 void* workspace(Device& d, size_t bytes);
 // A workspace for ops that can also do without: null where it is too small and a graph is being recorded, where the budget or the
 // card has no room left, and beyond optional_space_most.  Unlike the one above it never moves under a recorded graph: what it has
-// outgrown is kept, and all of it is given back (and the graphs dropped) when an allocation would otherwise fail.
+// outgrown is kept while there are any, and all of it is given back (and the graphs dropped) when an allocation would otherwise fail.
 constexpr size_t optional_space_most = size_t(2) << 30;
 void* optional_space(Device& d, size_t bytes);
 // Recorded graphs hold the addresses of the library's own buffers: when one of them moves, the graphs recorded so far go.

@@ -334,21 +334,23 @@ def test_batched_sparse_step_recorded(gpu, oracle):
 
 
 class _Dense:
-    """sd_op_attention of one row whose keys are cut into more runs than the caller's scratch holds: it takes an optional workspace."""
+    """sd_op_attention of rows whose keys are cut into more runs than the caller's scratch holds: it takes an optional workspace."""
 
-    def __init__(self, gpu, oracle, context=4200, heads=16, kv_heads=2, dim=256):
+    def __init__(self, gpu, oracle, rows=1, context=4200, heads=16, kv_heads=2, dim=256):
         rng = np.random.default_rng(context)
-        self.gpu, self.shape = gpu, (context, heads, kv_heads, dim)
-        q, keys, values = (rng.standard_normal(n).astype(np.float32) for n in ((1, heads, dim), (context, kv_heads, dim), (context, kv_heads, dim)))
-        positions = np.array([context - 1], np.int32)
+        self.gpu, self.shape = gpu, (context, rows, heads, kv_heads, dim)
+        q, keys, values = (rng.standard_normal(n).astype(np.float32) for n in ((rows, heads, dim), (context, kv_heads, dim), (context, kv_heads, dim)))
+        positions = np.arange(context - rows, context, dtype=np.int32)
         self.buffers = [gpu.upload(x) for x in (q, keys, values, positions)]
-        self.scratch, self.out = gpu.buffer(heads * (256 // heads) * (dim + 2) * 4), gpu.buffer(q.size * 4)
-        self.want, self.bound = oracle.op_attention_f64(q, keys, values, positions, float(np.float32(dim ** -0.5)), None)
+        pairs = rows * heads
+        self.scratch, self.out = gpu.buffer(pairs * min(64, max(1, 256 // pairs)) * (dim + 2) * 4), gpu.buffer(q.size * 4)
+        if oracle:
+            self.want, self.bound = oracle.op_attention_f64(q, keys, values, positions, float(np.float32(dim ** -0.5)), None)
 
     def queue(self):
-        context, heads, kv_heads, dim = self.shape
+        context, rows, heads, kv_heads, dim = self.shape
         q, keys, values, positions = (b.base() for b in self.buffers)
-        self.gpu.attention(q, keys, values, context, positions, 1, heads, kv_heads, dim, float(dim ** -0.5), None, self.scratch, self.out.base())
+        self.gpu.attention(q, keys, values, context, positions, rows, heads, kv_heads, dim, float(dim ** -0.5), None, self.scratch, self.out.base())
 
     def right(self, how):
         self.gpu.write_buffer(self.out, 0, np.zeros(self.want.size, np.float32))
@@ -387,3 +389,28 @@ def test_optional_workspaces_are_given_back_where_that_helps(oracle):
         for _ in range(2):
             work.right(work.queue)             # (with a workspace again)
             assert work.right(lambda: gpu.graph_run(7))
+
+
+@pytest.mark.parametrize("recorded", [False, True])
+def test_optional_workspaces_grow_into_the_room_there_is(oracle, recorded):
+    # partial results of 25 and of 32 MB: the second workspace fits the budget, twice the first does not; where a graph was recorded
+    # over the first it stays, and the graph is right
+    with backend(4 << 30) as gpu:
+        for rows in (44, 60):
+            _Dense(gpu, None, rows, 1120)
+        used = gpu.memory()[0]
+    with backend(used + (2 << 20) + ((72 if recorded else 44) << 20)) as gpu:
+        first, second = (_Dense(gpu, oracle, rows, 1120) for rows in (44, 60))
+        first.right(first.queue)
+        free = gpu.device_state()[0]
+        if recorded:
+            gpu.graph_begin()
+            first.queue()
+            gpu.graph_end(1)
+        second.right(second.queue)
+        assert free - gpu.device_state()[0] >= (30 if recorded else 2) << 20, "the second call has a workspace of its size"
+        for _ in range(2):
+            first.right(first.queue)
+            second.right(second.queue)
+            if recorded:
+                assert first.right(lambda: gpu.graph_run(1))
