@@ -19,12 +19,16 @@ void select_thin_reserve(Device& d);     // block_index.hip
 // graphs recorded so far would replay on freed memory: they are dropped, sd_graph_run then answers 1 ("none stored under
 // this key") and the caller records again -- what the reference does when its K/V views change (kv_clear_graphs,
 // gpu/kv_stage.hpp:96-104).
-void drop_recorded_graphs(Device& d) {
+static void destroy_graphs(Device& d) {       // (with optional_mutex)
     for (auto& entry : d.graphs) {
         if (entry.second.executable) (void)hipGraphExecDestroy(entry.second.executable);
         if (entry.second.graph) (void)hipGraphDestroy(entry.second.graph);
     }
     d.graphs.clear();
+}
+void drop_recorded_graphs(Device& d) {
+    std::lock_guard<std::mutex> lock(d.optional_mutex);
+    destroy_graphs(d);
 }
 
 Device& device(void* handle) {
@@ -58,17 +62,19 @@ static void* try_allocate(Device& d, size_t bytes, bool zero) {
 
 // The optional workspaces given back where `bytes` then fit into the `room` there is without them, and the graphs that may hold them
 // dropped.  False: nothing has changed -- they would not do, there are none, or a graph is being recorded, which may hold them too.
-static bool give_back_optional_spaces(Device& d, size_t bytes, size_t room) {
+static bool give_back_optional_spaces(Device& d, size_t bytes, size_t room) {       // (with optional_mutex)
     if (d.optional_spaces.empty() || d.recording) return false;
     for (const auto& space : d.optional_spaces) room += space.second + allocation_tail;
     if (bytes > room || allocation_tail > room - bytes) return false;
-    drop_recorded_graphs(d);
+    SD_CHECK(hipStreamSynchronize(d.stream));
+    destroy_graphs(d);
     for (const auto& space : d.optional_spaces) release(d, space.first);
     d.optional_spaces.clear();
     return true;
 }
 
 void* allocate(Device& d, size_t bytes, bool zero) {
+    std::lock_guard<std::mutex> lock(d.optional_mutex);
     const size_t available = d.budget > d.used ? d.budget - d.used : 0;
     const bool over = !bytes || bytes > available || allocation_tail > available - bytes;
     if (over && (!bytes || !give_back_optional_spaces(d, bytes, available))) throw std::runtime_error(budget_exceeded(d, bytes));
@@ -158,7 +164,7 @@ void* workspace(Device& d, size_t bytes) {
     return d.workspace;
 }
 
-void* optional_space(Device& d, size_t bytes) {
+static void* optional_space_locked(Device& d, size_t bytes) {
     const size_t held = d.optional_spaces.empty() ? 0 : d.optional_spaces.back().second;
     if (bytes <= held) return held ? d.optional_spaces.back().first : nullptr;
     hipStreamCaptureStatus capturing = hipStreamCaptureStatusNone;
@@ -179,6 +185,12 @@ void* optional_space(Device& d, size_t bytes) {
     }
     void* space = try_allocate(d, rounded, false);
     if (space) d.optional_spaces.emplace_back(space, rounded);
+    return space;
+}
+
+OptionalSpace optional_space(Device& d, size_t bytes) {
+    OptionalSpace space{std::unique_lock<std::mutex>(d.optional_mutex)};
+    space.at = optional_space_locked(d, bytes);
     return space;
 }
 
@@ -591,6 +603,7 @@ int sd_graph_begin(void* handle) {
         // (made here, not by the op that uses it: a capture takes no allocation; reference gpu/kernels.cpp:4769-4773)
         try { select_thin_reserve(d); } catch (const std::exception&) {}
         kv_settle(d);
+        std::lock_guard<std::mutex> lock(d.optional_mutex);
         SD_CHECK(hipStreamBeginCapture(d.stream, hipStreamCaptureModeThreadLocal));
         d.recording = true;
         return 0;
@@ -601,6 +614,7 @@ int sd_graph_end(void* handle, uint64_t key, int keep) {
     try {
         Device& d = device(handle);
         if (!d.recording) throw std::runtime_error("no Straydog graph is being recorded");
+        std::lock_guard<std::mutex> lock(d.optional_mutex);
         d.recording = false;
         Device::Recorded made;
         SD_CHECK(hipStreamEndCapture(d.stream, &made.graph));
@@ -624,6 +638,7 @@ int sd_graph_end(void* handle, uint64_t key, int keep) {
 int sd_graph_run(void* handle, uint64_t key) {
     try {
         Device& d = device(handle);
+        std::lock_guard<std::mutex> lock(d.optional_mutex);
         const auto found = d.graphs.find(key);
         if (found == d.graphs.end()) return 1;
         // page moves queued since the recording (a resume, a stage) come first: the graph's ops read the pages they fill

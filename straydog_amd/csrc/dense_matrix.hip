@@ -379,8 +379,10 @@ void dense_matrix(Device& d, const float* q, const float* keys, const float* val
     // hold them they go to the handle's workspace
     const uint64_t steps = (context + 31) / 32, items = uint64_t(tiles) * kv_heads;
     args.splits = unsigned(std::min<uint64_t>({std::max<uint64_t>(1, 2 * uint64_t(d.compute_units) / items), steps, 128}));
+    OptionalSpace space;
     if (args.splits > scratch_splits || uintptr_t(scratch) % 16) {
-        args.partial = args.splits > 1 ? static_cast<float*>(optional_space(d, size_t(rows * heads) * args.splits * (dim + 2) * 4)) : nullptr;
+        if (args.splits > 1) space = optional_space(d, size_t(rows * heads) * args.splits * (dim + 2) * 4);
+        args.partial = static_cast<float*>(space.at);
         if (!args.partial) {                              // (a graph is being recorded and the workspace is smaller)
             args.splits = uintptr_t(scratch) % 16 ? 1 : unsigned(std::min<uint64_t>(args.splits, scratch_splits));
             args.partial = scratch;

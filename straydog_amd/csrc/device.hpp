@@ -56,6 +56,8 @@ struct Device {
     void* sequence_input = nullptr; size_t sequence_input_bytes = 0;
     void* sequence_output = nullptr; size_t sequence_output_bytes = 0;
     void* workspace = nullptr; size_t workspace_bytes = 0;
+    // Optional workspaces and recorded graphs belong to optional_mutex: another thread's allocation may give them back.
+    std::mutex optional_mutex;
     std::vector<std::pair<void*, size_t>> optional_spaces;      // the last is in use; recorded graphs may hold the smaller ones before it
     // The attention rope table of a pass (sd_attention_turns_reserve / _arm): forward[row][pair] = (cosine, sine), then the
     // inverse turns at the same stride.  Armed for `turns_armed` rows, the next sd_op_norm_rope of that many rows fills it;
@@ -147,7 +149,12 @@ void* workspace(Device& d, size_t bytes);
 // card has no room left, and beyond optional_space_most.  Unlike the one above it never moves under a recorded graph: what it has
 // outgrown is kept while there are any, and all of it is given back (and the graphs dropped) when an allocation would otherwise fail.
 constexpr size_t optional_space_most = size_t(2) << 30;
-void* optional_space(Device& d, size_t bytes);
+// The space stays while this lives: until the op's kernels are queued (giving it back waits for the stream).  Nothing may be allocated meanwhile.
+struct OptionalSpace {
+    std::unique_lock<std::mutex> held;
+    void* at = nullptr;
+};
+OptionalSpace optional_space(Device& d, size_t bytes);
 // Recorded graphs hold the addresses of the library's own buffers: when one of them moves, the graphs recorded so far go.
 void drop_recorded_graphs(Device& d);
 

@@ -527,8 +527,10 @@ void latent_rows(Device& d, const float* q, const float* raw, uint64_t raw_rows,
     // few rows: their steps of 32 keys in as many runs as give every compute unit a workgroup, the runs merged by a second launch
     const uint64_t steps = (window + STEP - 1) / STEP + (selections + STEP - 1) / STEP, room = d.compute_units / (rows * blocks);
     args.chunks = unsigned(std::min<uint64_t>(std::min<uint64_t>(steps, 64), std::max<uint64_t>(1, room)));
+    OptionalSpace space;
     if (args.chunks > 1) {
-        args.partial = static_cast<float*>(optional_space(d, size_t(rows) * args.chunks * heads * (DIM + 2) * 4));
+        space = optional_space(d, size_t(rows) * args.chunks * heads * (DIM + 2) * 4);
+        args.partial = static_cast<float*>(space.at);
         if (!args.partial) args.chunks = 1;            // (a graph is being recorded and the workspace is smaller: one run a row needs none)
     }
     if (ht == 4) { if (bf16) launch<4, true>(d, args, rows, blocks); else launch<4, false>(d, args, rows, blocks); }

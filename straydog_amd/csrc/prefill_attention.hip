@@ -1365,7 +1365,8 @@ bool launch_operands(Device& d, const PrefillArgs& args) {
     }
     const uint64_t tile_bytes = checked_product({args.seqs, args.kv_heads, tiles_per_seq, uint64_t(WIDE_TILE)});
     const uint64_t partial_bytes = splits > 1 ? uint64_t(items) * splits * WIDE_GROUP * (WIDE + 2) * 4 : 0;
-    uint8_t* tiles = static_cast<uint8_t*>(optional_space(d, tile_bytes + partial_bytes));
+    const OptionalSpace space = optional_space(d, tile_bytes + partial_bytes);
+    uint8_t* const tiles = static_cast<uint8_t*>(space.at);
     if (!tiles) return false;
     float* partial = reinterpret_cast<float*>(tiles + tile_bytes);
     unpack_operands_kernel<Q8><<<dim3(2 * tiles_per_seq, args.kv_heads, args.seqs), 256, 0, d.stream>>>(args, tiles, tiles_per_seq);

@@ -414,3 +414,29 @@ def test_optional_workspaces_grow_into_the_room_there_is(oracle, recorded):
             second.right(second.queue)
             if recorded:
                 assert first.right(lambda: gpu.graph_run(1))
+
+
+def test_optional_workspaces_under_allocations_of_another_thread(oracle):
+    # one thread queues an op that takes an optional workspace while another allocates what only fits without it: the op's kernels keep
+    # the workspace they were given
+    import threading
+    budget = 64 << 20
+    with backend(budget) as gpu:
+        work = _Dense(gpu, oracle)
+        rest, done, failed = budget - gpu.memory()[0] - 64, threading.Event(), []
+
+        def allocate():
+            try:
+                while not done.is_set():
+                    gpu.release(gpu.buffer(rest))
+            except Exception as error:
+                failed.append(error)
+        other = threading.Thread(target=allocate)
+        other.start()
+        try:
+            for _ in range(50):
+                work.right(work.queue)
+        finally:
+            done.set()
+            other.join()
+        assert not failed
