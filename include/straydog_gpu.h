@@ -33,7 +33,8 @@ int sd_device_info(int ordinal, char* name, size_t capacity, uint64_t* free_byte
  * allocation is charged against; one compute stream. */
 void* sd_create(int ordinal, uint64_t budget);
 void sd_destroy(void* handle);
-/* reference straydog_gpu.h:37: bytes allocated so far and the budget. */
+/* reference straydog_gpu.h:37: bytes allocated so far and the budget.  The workspaces that ops can do without are not counted: an
+ * allocation that needs their room gets it (see the graphs below). */
 int sd_memory(void* handle, uint64_t* used, uint64_t* budget);
 
 /* ---- Allocations and transfers ---- */

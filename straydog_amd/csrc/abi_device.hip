@@ -39,7 +39,9 @@ Device& device(void* handle) {
 }
 
 static std::string budget_exceeded(const Device& d, size_t bytes) {
-    const size_t left = d.budget > d.used ? d.budget - d.used : 0;
+    size_t left = d.budget > d.used ? d.budget - d.used : 0;
+    if (!d.recording)
+        for (const auto& space : d.optional_spaces) left += space.second + allocation_tail;
     return "Straydog VRAM budget exceeded (" + std::to_string(bytes >> 20) + " MiB asked, " + std::to_string(left >> 20) + " MiB of " +
            std::to_string(d.budget >> 20) + " MiB left)";
 }
@@ -296,7 +298,10 @@ void sd_destroy(void* handle) {
 int sd_memory(void* handle, uint64_t* used, uint64_t* budget) {
     try {
         Device& d = device(handle);
-        if (used) *used = d.used;
+        std::lock_guard<std::mutex> lock(d.optional_mutex);
+        size_t optional = 0;
+        for (const auto& space : d.optional_spaces) optional += space.second + allocation_tail;
+        if (used) *used = d.used - optional;
         if (budget) *budget = d.budget;
         return 0;
     } catch (const std::exception& e) { last_error = e.what(); return -1; }

@@ -372,6 +372,7 @@ def test_optional_workspaces_are_given_back_where_that_helps(oracle):
         used, before = gpu.memory()[0], gpu.device_state()[0]
         work.right(work.queue)
         assert before - gpu.device_state()[0] >= 2 << 20, "the op has taken a workspace"
+        assert gpu.memory() == (used, budget), "what an allocation can have is not less for it"
         gpu.graph_begin()
         work.queue()
         gpu.graph_end(7)
