@@ -1088,55 +1088,77 @@ __global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_e
 // keys {4 g .., 16 + 4 g ..} of column 32 (j / 2) + 8 (li / 4) + 4 (j % 2) + li % 4, so that the results of two operands are eight
 // neighbouring columns of a lane's query row.
 constexpr int WIDE = 256, WIDE_BLOCKS = WIDE / 32, WIDE_TILES = WIDE / 16, WIDE_TILE = 2 * STEP * WIDE * 2, WIDE_ROWS = 32, WIDE_GROUP = GROUPS * WIDE_ROWS;
-// A workgroup builds a tile's K operands or its V operands.
+// A workgroup builds a tile's K operands or its V operands, and goes on to every gridDim.x / 2-th tile of the rows that are there: the
+// host knows only max_context, and workgroups for all of that cost 10 us where 4 sequences hold 756 of 131072 tokens.
 template<bool Q8>
 __global__ void __launch_bounds__(256) unpack_operands_kernel(PrefillArgs args, uint8_t* tiles_out, unsigned tiles_per_seq) {
     constexpr int ROW = Q8 ? WIDE + WIDE / 16 : 2 * WIDE, PIECES = ROW / 16, ALL = STEP * PIECES;
-    const int tile = blockIdx.x / 2, value = blockIdx.x % 2, kvh = blockIdx.y, seq = blockIdx.z, thread = threadIdx.x;
+    const int value = blockIdx.x % 2, kvh = blockIdx.y, seq = blockIdx.z, thread = threadIdx.x;
     const int position = first_position(args.positions, unsigned(seq), args.max_context);
     const int cached = min(position + int(args.span), args.max_context);
-    if (tile * STEP >= cached) return;
     const int32_t* table = args.page_table + size_t(seq) * args.table_stride;
     const size_t plane_bytes = size_t(args.page_tokens) * ROW;
     __shared__ __attribute__((aligned(16))) uint8_t raw[STEP][ROW];
-    // rows past the sequence's end are never read: they are zeros
-    #pragma unroll
-    for (int first = 0; first < ALL; first += 256) {
-        const int at = first + thread, piece = at % PIECES, row = at / PIECES, token = tile * STEP + row;
-        if (at >= ALL) break;
-        uint4 bytes = {0u, 0u, 0u, 0u};
-        if (token < cached)
-            bytes = *reinterpret_cast<const uint4*>(args.pages + (size_t(pool_page(table[token / int(args.page_tokens)], args.page_last)) * 2 * args.kv_heads +
-                                                                  (value ? args.kv_heads : 0) + kvh) * plane_bytes + size_t(token % int(args.page_tokens)) * ROW + 16 * piece);
-        *reinterpret_cast<uint4*>(&raw[row][16 * piece]) = bytes;
-    }
-    __syncthreads();
-    const int lane = thread & 63, li = lane & 15, g = lane >> 4;
-    uint8_t* out = tiles_out + ((size_t(seq) * args.kv_heads + kvh) * tiles_per_seq + tile) * WIDE_TILE + 1024 * 2 * WIDE_BLOCKS * value + 16 * lane;
-    #pragma unroll
-    for (int n = 0; n < 4; ++n) {
-        const int operand = thread / 64 + 4 * n;
-        half8 x;
-        if (!value) {
-            const int b = operand % WIDE_BLOCKS;
-            const uint8_t* row = raw[16 * (operand / WIDE_BLOCKS) + li];
-            if (Q8) {
-                const uint2 bytes = *reinterpret_cast<const uint2*>(row + 32 * b + 8 * g);
-                const _Float16 scale = *reinterpret_cast<const _Float16*>(row + WIDE + 2 * b);
-                #pragma unroll
-                for (int i = 0; i < 8; ++i) x[i] = (_Float16)float(int8_t((i < 4 ? bytes.x : bytes.y) >> (8 * (i & 3)))) * scale;
-            } else x = *reinterpret_cast<const half8*>(row + 64 * b + 16 * g);
-        } else {
-            const int column = 32 * (operand / 2) + 8 * (li / 4) + 4 * (operand % 2) + li % 4;
-            #pragma unroll
-            for (int e = 0; e < 8; ++e) {
-                const uint8_t* row = raw[4 * g + (e < 4 ? e : 12 + e)];
-                if (Q8) x[e] = (_Float16)float(int8_t(row[column])) * *reinterpret_cast<const _Float16*>(row + WIDE + 2 * (column / 32));
-                else x[e] = *reinterpret_cast<const _Float16*>(row + 2 * column);
-            }
+    for (int tile = blockIdx.x / 2; tile * STEP < cached; tile += int(gridDim.x / 2)) {
+        // rows past the sequence's end are never read: they are zeros
+        #pragma unroll
+        for (int first = 0; first < ALL; first += 256) {
+            const int at = first + thread, piece = at % PIECES, row = at / PIECES, token = tile * STEP + row;
+            if (at >= ALL) break;
+            uint4 bytes = {0u, 0u, 0u, 0u};
+            if (token < cached)
+                bytes = *reinterpret_cast<const uint4*>(args.pages + (size_t(pool_page(table[token / int(args.page_tokens)], args.page_last)) * 2 * args.kv_heads +
+                                                                      (value ? args.kv_heads : 0) + kvh) * plane_bytes + size_t(token % int(args.page_tokens)) * ROW + 16 * piece);
+            *reinterpret_cast<uint4*>(&raw[row][16 * piece]) = bytes;
         }
-        *reinterpret_cast<half8*>(out + 1024 * operand) = x;
+        __syncthreads();
+        const int lane = thread & 63, li = lane & 15, g = lane >> 4;
+        uint8_t* out = tiles_out + ((size_t(seq) * args.kv_heads + kvh) * tiles_per_seq + tile) * WIDE_TILE + 1024 * 2 * WIDE_BLOCKS * value + 16 * lane;
+        #pragma unroll
+        for (int n = 0; n < 4; ++n) {
+            const int operand = thread / 64 + 4 * n;
+            half8 x;
+            if (!value) {
+                const int b = operand % WIDE_BLOCKS;
+                const uint8_t* row = raw[16 * (operand / WIDE_BLOCKS) + li];
+                if (Q8) {
+                    const uint2 bytes = *reinterpret_cast<const uint2*>(row + 32 * b + 8 * g);
+                    const _Float16 scale = *reinterpret_cast<const _Float16*>(row + WIDE + 2 * b);
+                    #pragma unroll
+                    for (int i = 0; i < 8; ++i) x[i] = (_Float16)float(int8_t((i < 4 ? bytes.x : bytes.y) >> (8 * (i & 3)))) * scale;
+                } else x = *reinterpret_cast<const half8*>(row + 64 * b + 16 * g);
+            } else {
+                const int column = 32 * (operand / 2) + 8 * (li / 4) + 4 * (operand % 2) + li % 4;
+                #pragma unroll
+                for (int e = 0; e < 8; ++e) {
+                    const uint8_t* row = raw[4 * g + (e < 4 ? e : 12 + e)];
+                    if (Q8) x[e] = (_Float16)float(int8_t(row[column])) * *reinterpret_cast<const _Float16*>(row + WIDE + 2 * (column / 32));
+                    else x[e] = *reinterpret_cast<const _Float16*>(row + 2 * column);
+                }
+            }
+            *reinterpret_cast<half8*>(out + 1024 * operand) = x;
+        }
+        __syncthreads();
     }
+}
+
+// Where the walks are too few for the card they are cut into up to 16 shares of keys: a share costs its steps (about 1 us each) and
+// a sixteenth of a step a workgroup for its sums' way through memory, and any shares at all their merge (4 us: 64 rows of one sequence at
+// 100 19 us in two, 16 in one; at 400 22 in four, 25 in one).  The launch has shares for max_context; a sequence uses those that
+// its own steps are worth (128 rows at 0 of 8192 31 us in the launch's, 17 in its own; tight 14).
+constexpr unsigned SHARES_MOST = 16, SHARES_MERGE = 64;
+__host__ __device__ inline unsigned shares_of(unsigned steps, unsigned items, unsigned most) {
+    unsigned shares = 1, cost = 16 * steps;
+    #pragma unroll
+    for (unsigned s = 2; s <= SHARES_MOST; ++s) {
+        const unsigned this_cost = 16 * ((steps + s - 1) / s) + items * s + SHARES_MERGE;
+        if (s <= most && this_cost < cost) { cost = this_cost; shares = s; }
+    }
+    return shares;
+}
+__device__ __forceinline__ unsigned used_shares(unsigned cached, unsigned tiles_per_seq, unsigned items, unsigned launched) {
+    const unsigned steps = __builtin_amdgcn_readfirstlane((cached + STEP - 1) / STEP);      // (all that follows on the scalar unit)
+    return launched == 1 || steps == tiles_per_seq ? launched : shares_of(steps, items, launched);
 }
 
 // 128 query rows a workgroup, 32 a wave (two tiles of 16: 128 registers of outputs, 64 of queries), a step of 32 keys at a time,
@@ -1145,16 +1167,22 @@ __global__ void __launch_bounds__(256) unpack_operands_kernel(PrefillArgs args, 
 // LDS (160 bytes a cycle asked of its 128 with the tiles' arrival) bounds it ahead of the products.
 // Measured, 2 x 1531 tokens of 24 heads over 2 (57.6 GFLOP): 73 us (0.78 PFLOP/s) where the kernel that converts in its loop takes 205.
 __global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_operands_kernel(PrefillArgs args, const uint8_t* tiles_in,
-                                                                                                             unsigned tiles_per_seq, unsigned splits, float* partial) {
+                                                                                                             unsigned tiles_per_seq, unsigned most, float* partial) {
     // The longest walks first.  (Paired so that a compute unit's second workgroup is the shorter the longer its first: no faster.)
     const unsigned pairs = args.kv_heads * args.seqs, runs = (args.rows + WIDE_GROUP - 1) / WIDE_GROUP;
-    const unsigned item = blockIdx.x / splits, split = blockIdx.x % splits;
+    const unsigned item = blockIdx.x / most;
+    unsigned split = blockIdx.x % most;
     const int run = int(runs - 1 - item / pairs), kvh = int(item % pairs % args.kv_heads), seq = int(item % pairs / args.kv_heads);
     const int thread = threadIdx.x, lane = thread & 63, wave = __builtin_amdgcn_readfirstlane(thread >> 6), li = lane & 15, g = lane >> 4;
     const int position = first_position(args.positions, unsigned(seq), args.max_context);
     const int cached = min(position + int(args.span), args.max_context);
     const int row0 = run * WIDE_GROUP + wave * WIDE_ROWS, group_last = min(int(args.rows), (run + 1) * WIDE_GROUP) - 1;
     const int keys = min(position + group_last / int(args.group) + 1, cached), steps = (keys + STEP - 1) / STEP;
+    const unsigned splits = used_shares(unsigned(cached), tiles_per_seq, pairs * runs, most);
+    // (Workgroups go round the eight dies.  A launched share stays on the same dies, whose L2 keeps its keys for all runs; where not all are
+    // used, the places of the used ones move on whenever the items have gone round.)
+    if (splits < most) split = (split + item / (8 / min(8u, most & -most))) % most;
+    if (split >= splits) return;
     const int begin = int(unsigned(steps) * split / splits), end = int(unsigned(steps) * (split + 1) / splits);
     const bool idle = row0 >= int(args.rows);                   // a wave past the last row only helps copying
     const int wave_first = position + row0 / int(args.group);
@@ -1275,7 +1303,7 @@ __global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_e
         const float sum = row_sum(l[qt]);
         if (row >= int(args.rows)) continue;
         if (splits > 1) {
-            const size_t at = (size_t(item) * splits + split) * WIDE_GROUP + (row - run * WIDE_GROUP), all = size_t(gridDim.x) * WIDE_GROUP;
+            const size_t at = (size_t(item) * most + split) * WIDE_GROUP + (row - run * WIDE_GROUP), all = size_t(gridDim.x) * WIDE_GROUP;
             #pragma unroll
             for (int jj = 0; jj < WIDE_TILES; ++jj) *reinterpret_cast<floatx4*>(partial + at * WIDE + 32 * (jj / 2) + 8 * g + 4 * (jj % 2)) = acc[qt][jj];
             if (g == 0) *reinterpret_cast<float2*>(partial + all * WIDE + 2 * at) = float2{ref[qt], sum};
@@ -1298,38 +1326,43 @@ __global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_e
     }
 }
 
-// A wave a query row: the shares of its keys under their common maximum, normalised.
-__global__ void __launch_bounds__(256) merge_shares_kernel(PrefillArgs args, const float* partial, unsigned splits) {
+// A wave a query row: the shares of its keys under their common maximum, normalised.  At most a round of the card's workgroups, each going on to
+// further rows: where the outputs are finished already a wave has nothing to do but find that out (24576 rows 12 us a wave each).
+constexpr unsigned MERGE_ROWS = 4;
+__global__ void __launch_bounds__(64 * MERGE_ROWS) merge_shares_kernel(PrefillArgs args, const float* partial, unsigned tiles_per_seq, unsigned launched) {
     const unsigned pairs = args.kv_heads * args.seqs, runs = (args.rows + WIDE_GROUP - 1) / WIDE_GROUP, lane = threadIdx.x % 64;
-    const unsigned item = blockIdx.x / (WIDE_GROUP / 4), in_run = blockIdx.x % (WIDE_GROUP / 4) * 4 + threadIdx.x / 64;
-    const unsigned run = runs - 1 - item / pairs, kvh = item % pairs % args.kv_heads, seq = item % pairs / args.kv_heads, row = run * WIDE_GROUP + in_run;
-    if (row >= args.rows) return;
-    const size_t first = size_t(item) * splits * WIDE_GROUP + in_run;
-    const float2* const stats = reinterpret_cast<const float2*>(partial + size_t(pairs) * runs * splits * WIDE_GROUP * WIDE);
-    constexpr unsigned MOST = 16;
-    floatx4 values[MOST];
-    float2 stat[MOST];
-    #pragma unroll
-    for (unsigned i = 0; i < MOST; ++i) {
-        const size_t at = first + size_t(min(i, splits - 1)) * WIDE_GROUP;
-        if (i < splits) { values[i] = *reinterpret_cast<const floatx4*>(partial + at * WIDE + 4 * lane); stat[i] = stats[at]; }
-        else { values[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f}; stat[i] = float2{NEG_BIG, 0.0f}; }
+    for (unsigned unit = blockIdx.x; unit < pairs * runs * (WIDE_GROUP / MERGE_ROWS); unit += gridDim.x) {
+        const unsigned item = unit / (WIDE_GROUP / MERGE_ROWS), in_run = unit % (WIDE_GROUP / MERGE_ROWS) * MERGE_ROWS + threadIdx.x / 64;
+        const unsigned run = runs - 1 - item / pairs, kvh = item % pairs % args.kv_heads, seq = item % pairs / args.kv_heads, row = run * WIDE_GROUP + in_run;
+        const int cached = min(first_position(args.positions, seq, args.max_context) + int(args.span), args.max_context);
+        const unsigned splits = used_shares(unsigned(cached), tiles_per_seq, pairs * runs, launched);
+        if (splits == 1 || row >= args.rows) continue;         // (the outputs of one share are finished)
+        const size_t first = size_t(item) * launched * WIDE_GROUP + in_run;
+        const float2* const stats = reinterpret_cast<const float2*>(partial + size_t(pairs) * runs * launched * WIDE_GROUP * WIDE);
+        floatx4 values[SHARES_MOST];
+        float2 stat[SHARES_MOST];
+        #pragma unroll
+        for (unsigned i = 0; i < SHARES_MOST; ++i) {
+            const size_t at = first + size_t(min(i, splits - 1)) * WIDE_GROUP;
+            if (i < splits) { values[i] = *reinterpret_cast<const floatx4*>(partial + at * WIDE + 4 * lane); stat[i] = stats[at]; }
+            else { values[i] = floatx4{0.0f, 0.0f, 0.0f, 0.0f}; stat[i] = float2{NEG_BIG, 0.0f}; }
+        }
+        float top = NEG_BIG, sum = 0.0f;
+        #pragma unroll
+        for (unsigned i = 0; i < SHARES_MOST; ++i) top = fmaxf(top, stat[i].x);
+        floatx4 x = {0.0f, 0.0f, 0.0f, 0.0f};
+        #pragma unroll
+        for (unsigned i = 0; i < SHARES_MOST; ++i) {
+            const float weight = __builtin_amdgcn_exp2f(stat[i].x - top);
+            sum += stat[i].y * weight;
+            x += values[i] * weight;
+        }
+        x *= 1.0f / sum;
+        const size_t out = ((size_t(seq) * args.span + row / args.group) * args.heads + kvh * args.group + row % args.group) * WIDE + 4 * lane;
+        typedef _Float16 half4 __attribute__((ext_vector_type(4)));
+        if (args.out_f16) *reinterpret_cast<half4*>(static_cast<_Float16*>(args.out) + out) = half4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
+        else *reinterpret_cast<floatx4*>(static_cast<float*>(args.out) + out) = x;
     }
-    float top = NEG_BIG, sum = 0.0f;
-    #pragma unroll
-    for (unsigned i = 0; i < MOST; ++i) top = fmaxf(top, stat[i].x);
-    floatx4 x = {0.0f, 0.0f, 0.0f, 0.0f};
-    #pragma unroll
-    for (unsigned i = 0; i < MOST; ++i) {
-        const float weight = __builtin_amdgcn_exp2f(stat[i].x - top);
-        sum += stat[i].y * weight;
-        x += values[i] * weight;
-    }
-    x *= 1.0f / sum;
-    const size_t out = ((size_t(seq) * args.span + row / args.group) * args.heads + kvh * args.group + row % args.group) * WIDE + 4 * lane;
-    typedef _Float16 half4 __attribute__((ext_vector_type(4)));
-    if (args.out_f16) *reinterpret_cast<half4*>(static_cast<_Float16*>(args.out) + out) = half4{(_Float16)x[0], (_Float16)x[1], (_Float16)x[2], (_Float16)x[3]};
-    else *reinterpret_cast<floatx4*>(static_cast<float*>(args.out) + out) = x;
 }
 
 // `tiles`: where the cached rows' FP16 tiles go -- the device's workspace, rebuilt whole on every call, or a buffer the caller
@@ -1356,26 +1389,21 @@ template<bool Q8>
 bool launch_operands(Device& d, const PrefillArgs& args) {
     const unsigned tiles_per_seq = unsigned((args.max_context + STEP - 1) / STEP);
     const unsigned runs = (args.rows + WIDE_GROUP - 1) / WIDE_GROUP, items = runs * args.kv_heads * args.seqs;
-    // Where the walks are too few for the card they are cut into up to 16 shares of keys: a share costs its steps (about 1 us each) and
-    // a sixteenth of a step a workgroup for its sums' way through memory.
-    unsigned splits = 1, cost = 16 * tiles_per_seq;
-    for (unsigned s = 2; s <= 16 && items * s <= 2 * d.compute_units; ++s) {
-        const unsigned this_cost = 16 * ((tiles_per_seq + s - 1) / s) + items * s;
-        if (this_cost < cost) { cost = this_cost; splits = s; }
-    }
+    const unsigned splits = shares_of(tiles_per_seq, items, std::min(SHARES_MOST, 2 * d.compute_units / items));
     const uint64_t tile_bytes = checked_product({args.seqs, args.kv_heads, tiles_per_seq, uint64_t(WIDE_TILE)});
     const uint64_t partial_bytes = splits > 1 ? uint64_t(items) * splits * WIDE_GROUP * (WIDE + 2) * 4 : 0;
     const OptionalSpace space = optional_space(d, tile_bytes + partial_bytes);
     uint8_t* const tiles = static_cast<uint8_t*>(space.at);
     if (!tiles) return false;
     float* partial = reinterpret_cast<float*>(tiles + tile_bytes);
-    unpack_operands_kernel<Q8><<<dim3(2 * tiles_per_seq, args.kv_heads, args.seqs), 256, 0, d.stream>>>(args, tiles, tiles_per_seq);
+    const unsigned unpackers = std::min(tiles_per_seq, std::max(1u, 4 * d.compute_units / (args.kv_heads * args.seqs)));      // (one round of the card)
+    unpack_operands_kernel<Q8><<<dim3(2 * unpackers, args.kv_heads, args.seqs), 256, 0, d.stream>>>(args, tiles, tiles_per_seq);
     SD_CHECK(hipGetLastError());
     raise_shared_limit(d, reinterpret_cast<const void*>(&prefill_operands_kernel), 2 * WIDE_TILE);
     timed_launch(d, &prefill_operands_kernel, dim3(items * splits), dim3(GROUPS * 64), 2 * WIDE_TILE, args, static_cast<const uint8_t*>(tiles), tiles_per_seq, splits, partial);
     if (splits > 1) {
         SD_CHECK(hipGetLastError());
-        merge_shares_kernel<<<items * (WIDE_GROUP / 4), 256, 0, d.stream>>>(args, partial, splits);
+        merge_shares_kernel<<<std::min(items * (WIDE_GROUP / MERGE_ROWS), 4 * d.compute_units), 64 * MERGE_ROWS, 0, d.stream>>>(args, partial, tiles_per_seq, splits);
     }
     return true;
 }
@@ -1420,7 +1448,10 @@ void prefill_attention(Device& d, const sdx_kv_pool* pool, const int32_t* page_t
     // 32 sequences, 72 rows 288 / 403; 8 of 16384 147 / 746; one of 2000 24 / 96; whole prompts of 2 x 1531 tokens 89 / 226; FP16, 36 rows, 64
     // of 1500 128 / 73, 32 of 8192 319 / 342).
     const uint64_t items = seqs * pool->kv_heads, groups = items * ((args.rows + WIDE_GROUP - 1) / WIDE_GROUP);
-    const bool converting = args.rows <= WIDE_GROUP && items * 8 > uint64_t(d.compute_units) * 3;
+    // It is also the better one for up to 128 keys where its workgroups are one round of the card: the operands are a launch more (64 tokens
+    // at 0 12.2 / 10.3, 128 14.3 / 13.2, 200 16.4 / 18.3; 4 sequences of 64 12.5 / 10.8, 16 of 64, more than a round, 14.8 / 21.5).
+    const bool few_keys = max_context <= 128 && items * ((args.rows + GROUPS * 16 - 1) / (GROUPS * 16)) <= d.compute_units;
+    const bool converting = few_keys || (args.rows <= WIDE_GROUP && items * 8 > uint64_t(d.compute_units) * 3);
     if (!converting && (uintptr_t(q) | uintptr_t(out)) % 16 == 0 && groups < (uint64_t(1) << 24) && (q8 ? launch_operands<true>(d, args) : launch_operands<false>(d, args))) return;
     if (q8) launch<256, 1, true, 2>(d, args, unsigned(seqs)); else launch<256, 1, false, 2>(d, args, unsigned(seqs));
 }

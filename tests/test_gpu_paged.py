@@ -675,3 +675,32 @@ def test_verify_spans_of_256_columns_in_runs_of_rows(gpu, oracle, fmt, span, hea
     close_enough(gpu.read_buffer(out, 0, np.float32, q.size).reshape(q.shape), want, "a scratch of 16 bytes")
     for b in (buffer, tb, pb, qb, out, tiny):
         gpu.release(b)
+
+
+@pytest.mark.parametrize("fmt,span,heads,kv_heads,contexts", [("q8", 64, 24, 2, [400]), ("f16", 64, 24, 2, [700, 0, 333]), ("q8", 11, 24, 2, [2000, 100, 31, 32]), ("q8", 40, 8, 8, [0, 1000]),
+                                                              ("q8", 200, 16, 2, [0])])
+def test_prompts_of_256_columns_do_not_depend_on_the_capacity(gpu, oracle, fmt, span, heads, kv_heads, contexts):
+    # max_context says how far the page table reaches; what a sequence's walk is cut into follows from the rows that are there, so a
+    # larger one leaves the bits as they are
+    rng = np.random.default_rng(span + len(contexts))
+    dim, page_tokens, row_bytes, capacity = 256, 64, 272 if fmt == "q8" else 512, 16384
+    pool, buffer, host, table, tb = make_pool(gpu, oracle, rng, [c + span for c in contexts], kv_heads, dim, page_tokens, row_bytes,
+                                              dtype=np.float32 if fmt == "q8" else np.float16)
+    wide = np.zeros((len(contexts), capacity // page_tokens), np.int32)
+    wide[:, :table.shape[1]] = table
+    q = rng.standard_normal((len(contexts), span, heads, dim)).astype(np.float16).astype(np.float32)
+    scale = 1.0 / np.sqrt(dim)
+    want = oracle.paged_attention(host, row_bytes, page_tokens, kv_heads, dim, table, np.array(contexts, np.int32), q, scale)
+    pb, qb, out, wb = gpu.upload(np.array(contexts, np.int32)), gpu.upload(q), gpu.buffer(q.size * 4), gpu.upload(wide)
+    got = []
+    for at, stride, most in ((tb, table.shape[1], max(contexts) + span), (wb, wide.shape[1], capacity), (wb, wide.shape[1], 4096)):
+        scratch = gpu.buffer(16)           # (too small for runs of rows: the prompt's kernels)
+        gpu.write_buffer(out, 0, np.zeros(q.size, np.float32))
+        gpu.paged_attention(pool, at.base(), stride, pb.base(), most, qb.base(), False, len(contexts), span, heads, float(scale), out.base(), False, scratch)
+        got.append(gpu.read_buffer(out, 0, np.float32, q.size).reshape(q.shape))
+        gpu.release(scratch)
+    for result in got:
+        close_enough(result, want)
+        assert np.array_equal(result.view(np.uint32), got[0].view(np.uint32))
+    for b in (buffer, tb, pb, qb, out, wb):
+        gpu.release(b)
