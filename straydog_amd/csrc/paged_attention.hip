@@ -396,7 +396,8 @@ __global__ void __launch_bounds__(WAVES * 64) __attribute__((amdgpu_waves_per_eu
 // reference's qsa_decode_merge, gpu/sparse_attention_compute.hpp:139-170).  A lane takes two columns of every segment and
 // every lane reads the segments' maxima and sums for itself (one address a wave: a broadcast), so nothing is exchanged
 // between lanes and nothing waits on LDS or a barrier: the segments are asked for sixteen or (MOST) thirty-two at a time, all loads
-// in flight at once, under a running maximum.  Four rows a workgroup.  Thirty-two where the launch is one round of the card and bound
+// in flight at once, under a running maximum; up to four, the rule where the sequences are as many as the workgroups, in one go
+// of their own (16 sequences of 2000 keys, 64 rows of 8 K/V heads: the pass 75 us with sixteen, 67).  Four rows a workgroup.  Thirty-two where the launch is one round of the card and bound
 // by latency (8 sequences of up to 16384 keys, 24 heads of 256 columns: 6.0 us for 8.6; one of 65536: the pass 38.6 us for 48.3); with
 // more rows than that their registers cost more waves than they save trips (2560 rows of 17 segments: 1 us slower).
 template<int DIM, bool F16_OUT, int MOST>
@@ -451,7 +452,8 @@ __global__ void __launch_bounds__(256) paged_merge_kernel(PagedArgs args, void* 
     };
     unsigned first = 0;
     for (; first + 16 < used; first += MOST) take(std::integral_constant<int, MOST>{}, first);
-    if (first < used) take(std::integral_constant<int, 16>{}, first);
+    if (first + 4 < used) take(std::integral_constant<int, 16>{}, first);
+    else if (first < used) take(std::integral_constant<int, 4>{}, first);
     #pragma unroll
     for (int i = 0; i < PER; ++i) {
         const float2 result = make_float2(value[i].x / sum, value[i].y / sum);
@@ -523,6 +525,23 @@ bool holds(Device& d, const void* at, size_t bytes) {
     try { op_span(d, at, bytes, "attention scratch"); return true; } catch (const std::exception&) { return false; }
 }
 
+// Whether rows of 256 columns are better worked as `runs` runs of 32 query rows that walk the same shares side by side (their keys come
+// from memory about once, and are converted once a run) than by a prompt's kernels, of which one unpacks every key first and the other
+// converts in its loop a workgroup 64 rows.  It takes a batch that gives each compute unit 128 keys, and then sequences long enough that a
+// segment's start and end do not show.  items: sequences x K/V heads; measured in us, here / the better of the others:
+//   Q8_0, two runs: 1024 keys, 4096 where the items are more than the card's units (32 items of 2000 keys 34 / 44, 128 of 308
+//     34 / 23, of 1500 57 / 81, of 4000 108 / 207; 512 of 1500 206 / 190, of 4000 407 / 432).
+//   Q8_0, three and four: 8192 keys (32 items of 2000 42 / 47 and of 8192 104 / 149; 128 of 1500 85 / 86, of 8192 329 / 414).
+//   FP16, two: where the converting kernel has work for less than half the card 1024 keys (32 items of 8192 104 / 166), up to half an
+//     item a unit 8192 (128 of 1500 89 / 73, of 8192 333 / 407), with more never (512 of 8192 1315 / 837).
+// The host knows max_context and no lengths: 128 items of 500 keys in tables of 16384 take 37 / 33 in two runs, 62 / 37 in three.
+bool runs_of_rows_pay(uint64_t units, bool q8, unsigned runs, uint64_t items, uint64_t max_context) {
+    const uint64_t pieces = checked_product({items, (max_context + UNIT - 1) / UNIT});
+    if (pieces < units || pieces > 0x7fffffffu || max_context < 1024) return false;
+    if (runs > 2) return q8 && max_context >= 8192;
+    return q8 ? items <= units || max_context >= 4096 : items * 8 <= units * 3 || (max_context >= 8192 && items * 2 <= units);
+}
+
 // What both entry points do once their partial-result area is known.  `timed`: the main kernel may go through the extended
 // launch when the handle is being profiled (that creates events, which the entry point that allocates nothing must not).
 void paged_attention(Device& value, const sdx_kv_pool* pool, const int32_t* page_table, uint64_t table_stride, const int32_t* positions,
@@ -538,22 +557,20 @@ void paged_attention(Device& value, const sdx_kv_pool* pool, const int32_t* page
     op_span(value, positions, checked_floats({seqs}), "query positions");
     op_span(value, q, checked_product({seqs, span, heads, pool->dim, q_f16 ? 2u : 4u}), "attention queries");
     op_span(value, out, checked_product({seqs, span, heads, pool->dim, out_f16 ? 2u : 4u}), "an attention output");
-    // Up to 32 rows a K/V head at 256 columns (64 at 128) are one workgroup's.  At 256 columns up to 64 rows, over Q8_0 up to 128, can be
-    // runs of 32 rows that walk the same shares side by side (their keys come from memory about once, and are converted once a run),
-    // instead of a prompt's kernels, which unpack every key: the better way for batches that give each compute unit 128 keys, and
-    // with more than two runs, or over FP16 rows where the prompt's converting kernel has work for half the card, for long sequences.  (24 heads over 2, Q8_0, here / there: 36 rows, 16 sequences of 8192 keys 66 / 139 us, 64
-    // of 8192 190 / 537, one of 16384 37 / 55, one of 2000 26 / 23; 72 rows, 16 of 8192 104 / 147, 16 of 2000 55 / 47.  FP16 rows: 36 rows,
-    // 16 of 8192 103 / 166, 64 of 1500 89 / 73, 64 of 8192 347 / 347, 60 rows 354 / 402; 72 rows 571 / 434.)  The caller's scratch has to hold the partial results.
+    const bool q8 = pool->row_bytes != 2 * pool->dim;
+    const uint64_t items = checked_product({seqs, pool->kv_heads});
+    // What the rows take as `parts` runs side by side (1: one workgroup has them all): a run's workgroups, and the bytes of partial results.
+    const auto plan = [&](unsigned parts) {
+        const unsigned slots = std::max(1u, resident_slots(value, pool->dim, q8, parts > 1 ? 2 : query_tiles) / parts);
+        const uint64_t groups = std::min<uint64_t>(tuned_groups() && parts == 1 ? tuned_groups() : slots, most_groups(seqs, pool->kv_heads, max_context));
+        return std::pair<unsigned, size_t>(unsigned(groups), checked_floats({groups + items, rows, uint64_t(pool->dim) + 2}));
+    };
+    // Up to 32 rows a K/V head at 256 columns (64 at 128) are one workgroup's; up to 128 may be runs of 32.  The caller's scratch has to hold
+    // their partial results; where it does not they are a prompt's.
     unsigned parts = 1;
-    if (pool->dim == 256 && query_tiles > 2 && query_tiles <= 8 && !own_partial) {
-        const bool q8 = pool->row_bytes != 2 * pool->dim;
-        const unsigned wanted = (query_tiles + 1) / 2;
-        const uint64_t items = checked_product({seqs, pool->kv_heads});
-        if (checked_product({items, (max_context + UNIT - 1) / UNIT}) >= value.compute_units && (max_context >= 8192 ? q8 || wanted == 2 : wanted == 2 && (q8 || items * 8 <= uint64_t(value.compute_units) * 3))) {
-            const uint64_t groups = std::min<uint64_t>(std::max(1u, resident_slots(value, 256, q8, 2) / wanted), most_groups(seqs, pool->kv_heads, max_context));
-            const size_t need = checked_floats({groups + items, rows, uint64_t(256) + 2});
-            if (partial && partial_bytes >= need && holds(value, partial, need)) parts = wanted;
-        }
+    if (pool->dim == 256 && query_tiles > 2 && query_tiles <= 8 && !own_partial && runs_of_rows_pay(value.compute_units, q8, (query_tiles + 1) / 2, items, max_context)) {
+        const size_t need = plan((query_tiles + 1) / 2).second;
+        if (partial && partial_bytes >= need && holds(value, partial, need)) parts = (query_tiles + 1) / 2;
     }
     if (parts == 1 && query_tiles > (pool->dim == 128 ? 4u : 2u)) {
         if (own_partial) throw std::runtime_error("Straydog paged attention: too many query rows per K/V head for the entry point that allocates nothing");
@@ -570,12 +587,10 @@ void paged_attention(Device& value, const sdx_kv_pool* pool, const int32_t* page
     args.rows = unsigned(rows); args.seqs = unsigned(seqs);
     args.max_context = int(max_context);
     args.page_last = unsigned(std::min<uint64_t>(pool->page_count - 1, 0x7fffffffu));
-    const uint64_t items = checked_product({seqs, pool->kv_heads});
     if (checked_product({items, (max_context + UNIT - 1) / UNIT}) > 0x7fffffffu) throw std::runtime_error("invalid Straydog paged attention shape");
-    const unsigned slots = std::max(1u, resident_slots(value, pool->dim, pool->row_bytes != 2 * pool->dim, parts > 1 ? 2 : query_tiles) / parts);
-    args.groups_max = unsigned(std::min<uint64_t>(tuned_groups() && parts == 1 ? tuned_groups() : slots, most_groups(seqs, pool->kv_heads, max_context)));
+    const auto [groups, need] = plan(parts);
+    args.groups_max = groups;
     args.share_min = smallest_share;
-    const size_t need = checked_floats({uint64_t(args.groups_max) + items, rows, uint64_t(pool->dim) + 2});
     if (own_partial) {
         if (need > partial_bytes)
             throw std::runtime_error("Straydog paged attention: this batch needs " + std::to_string(need) + " bytes of partial results, the entry point that allocates nothing holds " +
@@ -589,7 +604,6 @@ void paged_attention(Device& value, const sdx_kv_pool* pool, const int32_t* page
     if (own_partial) value.profile = false;
     struct Restore { Device& d; bool profile; ~Restore() { d.profile = profile; } } restore{value, profiled};
     const dim3 grid(args.groups_max, parts);
-    const bool q8 = pool->row_bytes != 2 * pool->dim;
     if (pool->dim == 128) { if (q8) launch_tiles<128, true>(value, args, query_tiles, grid); else launch_tiles<128, false>(value, args, query_tiles, grid); }
     else if (parts > 1) { if (q8) launch<256, 2, true, variant_occupancy(256, true, 2), true>(value, args, grid); else launch<256, 2, false, variant_occupancy(256, false, 2), true>(value, args, grid); }
     else { if (q8) launch_tiles<256, true>(value, args, query_tiles, grid); else launch_tiles<256, false>(value, args, query_tiles, grid); }

@@ -656,8 +656,33 @@ def test_rows_of_256_columns_over_unpacked_operands(gpu, oracle, fmt, span, head
         gpu.release(b)
 
 
+def _runs_of_rows(gpu, f16, seqs, span, heads, kv_heads, max_context, dim=256):
+    """Whether a call of this shape goes to the kernel of the decode and verify spans: that one writes partial results to its scratch."""
+    page_tokens, rows = 256, seqs * span * heads * dim
+    stride = (max_context + page_tokens - 1) // page_tokens
+    pool, buffer = gpu.kv_pool(1, page_tokens, kv_heads, dim, 512 if f16 else 272)
+    table, positions, q, out = gpu.buffer(seqs * stride * 4), gpu.buffer(seqs * 4), gpu.buffer(rows * 2), gpu.buffer(rows * 2)
+    scratch = gpu.buffer(gpu.paged_attention_scratch(seqs, span, heads, dim, max_context))
+    gpu.paged_attention(pool, table.base(), stride, positions.base(), max_context, q.base(), True, seqs, span, heads, 0.0625, out.base(), True, scratch)
+    written = gpu.read_buffer(scratch, 0, np.uint32, min(scratch.size // 4, 1 << 20)).any()
+    for b in (buffer, table, positions, q, out, scratch):
+        gpu.release(b)
+    return bool(written)
+
+
+@pytest.mark.parametrize("f16,seqs,span,heads,kv_heads,max_context,runs", [
+    (0, 32, 5, 24, 2, 1024, True), (0, 32, 5, 24, 2, 1023, False), (0, 4, 64, 8, 8, 1024, True), (0, 64, 64, 8, 8, 64, False), (0, 32, 64, 8, 8, 264, False),
+    (0, 64, 8, 64, 8, 4095, False), (0, 64, 8, 64, 8, 4096, True), (0, 32, 8, 64, 8, 1500, True), (0, 1, 3, 24, 2, 16000, False), (0, 1, 3, 24, 2, 16384, True),
+    (0, 16, 8, 24, 2, 8191, False), (0, 16, 8, 24, 2, 8192, True), (0, 16, 11, 24, 2, 8192, False), (1, 16, 8, 24, 2, 8192, False), (1, 16, 5, 24, 2, 2048, True),
+    (1, 64, 5, 24, 2, 8191, False), (1, 64, 5, 24, 2, 8192, True), (1, 32, 8, 64, 8, 8192, False)])
+def test_the_line_between_runs_of_rows_and_prompts(gpu, f16, seqs, span, heads, kv_heads, max_context, runs):
+    # either side of each line of the rule (a card of 256 compute units)
+    assert gpu.compute_units() == 256
+    assert _runs_of_rows(gpu, f16, seqs, span, heads, kv_heads, max_context) == runs
+
+
 @pytest.mark.parametrize("fmt,span,heads,kv_heads,contexts", [("q8", 3, 24, 2, [16400]), ("q8", 8, 16, 2, [4000, 9001]), ("f16", 5, 24, 2, [12000, 5000, 100, 0]), ("q8", 6, 24, 2, [8200, 31]),
-                                                              ("q8", 8, 16, 1, [20000])])
+                                                              ("q8", 8, 16, 1, [33000]), ("q8", 7, 16, 1, [20000, 16000]), ("q8", 5, 24, 2, [2100] * 8)])
 def test_verify_spans_of_256_columns_in_runs_of_rows(gpu, oracle, fmt, span, heads, kv_heads, contexts):
     # 33 to 128 rows a K/V head over long batches: runs of 32 rows over the same shares; with scratch too small for their partial results
     # the prompt's kernels take the call, as they take shorter ones
@@ -670,6 +695,7 @@ def test_verify_spans_of_256_columns_in_runs_of_rows(gpu, oracle, fmt, span, hea
     want = oracle.paged_attention(host, row_bytes, page_tokens, kv_heads, dim, table, np.array(contexts, np.int32), q, scale)
     for q_f16, out_f16 in ((True, False), (False, False)):
         close_enough(_run(gpu, pool, table, tb, contexts, q, span, heads, scale, q_f16, out_f16), want, f"span {span} of {fmt} rows")
+    assert _runs_of_rows(gpu, 0 if fmt == "q8" else 1, len(contexts), span, heads, kv_heads, max(contexts) + span)
     pb, qb, out, tiny = gpu.upload(np.array(contexts, np.int32)), gpu.upload(q), gpu.buffer(q.size * 4), gpu.buffer(16)
     gpu.paged_attention(pool, tb.base(), table.shape[1], pb.base(), max(contexts) + span, qb.base(), False, len(contexts), span, heads, float(scale), out.base(), False, tiny)
     close_enough(gpu.read_buffer(out, 0, np.float32, q.size).reshape(q.shape), want, "a scratch of 16 bytes")
