@@ -347,12 +347,12 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
         odd |= probe != 0.0f;
     }
     const uint32_t found = (__any(odd) ? 1u : 0u) | (__any(l == 0.0f) ? 2u : 0u) | (any_row ? 4u : 0u);
-    ring_barrier();
-    if (lane == 0) seen[wave] = found;                 // (outside what the outputs leave through)
+    uint32_t* const found_by = seen + (end & 1) * STEP;        // (the half that the last step did not use)
+    if (lane == 0) found_by[wave] = found;
     ring_barrier();
     uint32_t odds = 0;
     #pragma unroll
-    for (int w = 0; w < WAVES_HERE; ++w) odds |= seen[w];
+    for (int w = 0; w < WAVES_HERE; ++w) odds |= found_by[w];
     const int back = DIM - 2 * int(a.pairs);
     float* const to = a.chunks == 1 ? a.out + size_t(row) * a.heads * DIM : a.partial + size_t(blockIdx.x) * a.heads * DIM;
     float* const stats = a.partial + size_t(gridDim.x) * a.heads * DIM + size_t(blockIdx.x) * a.heads * 2;      // (chunks > 1)
@@ -475,8 +475,8 @@ __global__ void __launch_bounds__(DIM / 4) latent_rows_merge_kernel(RowsArgs a) 
         }
         #pragma unroll
         for (unsigned i = 0; i < AT_ONCE; ++i) {
-            // (past the last run: its numbers again; they, and those of a run without a weight, may be none that zero silences)
-            const bool real = c0 + i < a.chunks && tops[i] != -INFINITY;
+            // (past the last run: its numbers again, which may be none that zero silences)
+            const bool real = c0 + i < a.chunks;
             const float weight = __builtin_amdgcn_exp2f((tops[i] - top) * LOG2E);
             sum += real ? sums[i] * weight : 0.0f;
             #pragma unroll
