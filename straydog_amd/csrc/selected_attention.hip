@@ -13,6 +13,8 @@
 // unnormalised output) are merged, normalised and gated by a second kernel, a block per (row, head).
 #include "paged_rows.hpp"
 
+#include <type_traits>
+
 using namespace sd;
 using namespace sd::paged;
 
@@ -224,8 +226,6 @@ __global__ void __launch_bounds__(DIM) selected_merge_kernel(SelectedArgs a) {
     const unsigned head = blockIdx.x % a.heads, kvh = head / a.group, col = threadIdx.x;
     const unsigned used = __builtin_amdgcn_readfirstlane((list_length(a, row) + CHUNK - 1) / CHUNK);
     const float* base = a.partial + ((row * a.kv_heads + kvh) * a.chunks) * 16 * STRIDE + size_t(head % a.group) * STRIDE;
-    // the chunks' pieces are asked for twenty at a time (a list of 2052 has 17): as many loads in flight, not one after the other
-    constexpr unsigned AT_ONCE = 20;
     Running so_far{NEG_BIG, 0.0f}, quarter{NEG_BIG, 0.0f};
     float value = 0.0f, quarter_value = 0.0f, keep, take;
     unsigned quarters = 0;                             // those closed
@@ -236,23 +236,31 @@ __global__ void __launch_bounds__(DIM) selected_merge_kernel(SelectedArgs a) {
         quarter_value = 0.0f;
         ++quarters;
     };
-    for (unsigned c0 = 0; c0 < used; c0 += AT_ONCE) {
-        float tops[AT_ONCE], sums[AT_ONCE], values[AT_ONCE];
-        #pragma unroll
-        for (unsigned i = 0; i < AT_ONCE; ++i) {
-            const float* part = base + size_t(min(c0 + i, used - 1)) * 16 * STRIDE;
-            tops[i] = part[DIM]; sums[i] = part[DIM + 1]; values[i] = part[col];
+    // the chunks' pieces are asked for twenty at a time (a list of 2052 has 17): as many loads in flight, not one after the other; four or
+    // eight where there are no more (32 rows of 128 entries, the call 14.2 us with twenty, 12.1; 2048 of 1024 364, 335)
+    const auto add = [&](auto at_once) {
+        constexpr unsigned AT_ONCE = decltype(at_once)::value;
+        for (unsigned c0 = 0; c0 < used; c0 += AT_ONCE) {
+            float tops[AT_ONCE], sums[AT_ONCE], values[AT_ONCE];
+            #pragma unroll
+            for (unsigned i = 0; i < AT_ONCE; ++i) {
+                const float* part = base + size_t(min(c0 + i, used - 1)) * 16 * STRIDE;
+                tops[i] = part[DIM]; sums[i] = part[DIM + 1]; values[i] = part[col];
+            }
+            #pragma unroll
+            for (unsigned i = 0; i < AT_ONCE; ++i) asm volatile("" : "+v"(values[i]), "+v"(tops[i]), "+v"(sums[i]));      // (here, not one by one behind the branches below)
+            #pragma unroll
+            for (unsigned i = 0; i < AT_ONCE; ++i) {
+                if (c0 + i >= used) break;
+                while (c0 + i >= quarter_begin(used, quarters + 1)) close();
+                chunk_factors(quarter, tops[i], sums[i], keep, take);
+                quarter_value = chunk_added(quarter_value, values[i], keep, take);
+            }
         }
-        #pragma unroll
-        for (unsigned i = 0; i < AT_ONCE; ++i) asm volatile("" : "+v"(values[i]), "+v"(tops[i]), "+v"(sums[i]));      // (here, not one by one behind the branches below)
-        #pragma unroll
-        for (unsigned i = 0; i < AT_ONCE; ++i) {
-            if (c0 + i >= used) break;
-            while (c0 + i >= quarter_begin(used, quarters + 1)) close();
-            chunk_factors(quarter, tops[i], sums[i], keep, take);
-            quarter_value = chunk_added(quarter_value, values[i], keep, take);
-        }
-    }
+    };
+    if (used <= 4) add(std::integral_constant<unsigned, 4>{});
+    else if (used <= 8) add(std::integral_constant<unsigned, 8>{});
+    else add(std::integral_constant<unsigned, 20>{});
     while (quarters < QUARTERS) close();
     value = finished(value, so_far.sum);
     if (a.gate) value = gated(value, a.gate[row * a.gate_row_stride + head * a.gate_stride + col]);
@@ -504,6 +512,23 @@ __global__ void __launch_bounds__(WAVES * 64, Q8 ? 2 : 1) selected_list_kernel(S
 }
 static_assert(WAVES == QUARTERS, "a wave a quarter");
 
+// Whether rows are better worked a workgroup a row and K/V head (an item) than their chunks of 128 entries a workgroup each: once there are enough
+// items for the card, and the lists long enough for a workgroup's four waves, each of which has whole chunks of the list, and for the
+// merge that chunks need, which grows with the query heads of a K/V head (the group).  Measured in us, chunks / lists:
+//   2052 entries, the stage of a prompt chunk over two K/V heads: Q8_0 32 rows 108 / 127, 48 123 / 132, 64 138 / 134, 256 304 / 175; FP16, whose chunks
+//     fill a compute unit's LDS, 16 rows 106 / 115, 24 122 / 118, 64 185 / 125.  Q8_0 over four K/V heads of four: 32 rows 48 / 55 (the call).
+//   1024 and 512: Q8_0, 128 items of 12 heads 31 / 31 and 20 / 20, of 4 heads 24 / 30 and 15 / 19, 192 of 8 41 / 31 and 26 / 20.
+//   256: Q8_0, 128 items 15 / 17, 256 of 8 heads 19 / 18, of 4 15 / 17, 512 of one 24 / 22; FP16, 128 items of 12 heads 17 / 16, of 4 14 / 15.
+//   128, one chunk: Q8_0, 256 items of 8 heads 15 / 17, 512 of 12 26 / 20, 1024 of 4 30 / 35, 2048 of one 43 / 67; FP16, 128 of 12 15 / 14, 1024 of one 47 / 56.
+//   64 and 32: Q8_0, 128 items of 12 heads 13 / 12, 512 of 4 16 / 13, of one 12 / 13; FP16, 96 of 4 heads 11 / 10, 512 of one 19 / 22.
+bool lists_pay(uint64_t units, bool q8, unsigned group, uint64_t entries, uint64_t items) {
+    if (entries <= 128 && group < 4) return false;
+    if (entries <= 64 || (entries > 1024 && (group >= 8 || !q8))) return items * (q8 ? 2 : 6) >= units;
+    if (entries <= 128) return group >= 8 && (q8 ? items >= 2 * units : items * 4 >= units);
+    if (entries <= 256) return q8 ? items >= (group >= 8 ? units : 2 * units) : items * 2 >= units;
+    return q8 ? items * 4 >= 3 * units : items * (entries <= 512 ? 4 : 6) >= units;       // (and Q8_0 lists of more under few heads)
+}
+
 uint64_t scratch_bytes_for(uint64_t rows, uint64_t kv_heads, uint64_t selected) {
     return checked_floats({rows, kv_heads, (selected + CHUNK - 1) / CHUNK, 16, uint64_t(DIM) + 2});
 }
@@ -569,10 +594,7 @@ int sdx_selected_attention(void* handle, const sdx_kv_pool* pool, const int32_t*
     args.chunks = unsigned((selected + CHUNK - 1) / CHUNK);
     args.gate = gate; args.gate_stride = size_t(gate_stride); args.gate_row_stride = size_t(gate_row_stride); args.out = out;
     const bool q8 = pool->row_bytes != 2 * pool->dim;
-    // A workgroup a row and K/V head once there are enough of them.  The stage of a chunk, lists of 2052 over two K/V heads, chunks as
-    // workgroups / lists: Q8_0 32 rows 108 / 127 us, 48: 123 / 132, 64: 138 / 134, 256: 304 / 175; FP16, whose chunks fill a compute unit's
-    // LDS, 16 rows 106 / 115, 24: 122 / 118, 64: 185 / 125.
-    const bool lists = rows * pool->kv_heads * (q8 ? 2 : 6) >= value.compute_units && args.chunks * CHUNK <= LIST_MAX &&
+    const bool lists = lists_pay(value.compute_units, q8, args.group, selected, rows * pool->kv_heads) && args.chunks * CHUNK <= LIST_MAX &&
                        checked_product({pool->page_count, 2, pool->kv_heads, pool->page_tokens, pool->row_bytes / 16}) <= (uint64_t(1) << 32) && rows * pool->kv_heads < (uint64_t(1) << 31) &&
                        (uintptr_t(out) | uintptr_t(gate)) % 16 == 0 && (gate_stride | gate_row_stride) % 4 == 0;
     if (q8) { if (out_f16) launch<true, true>(value, args, rows, lists); else launch<true, false>(value, args, rows, lists); }

@@ -683,3 +683,58 @@ def test_prompt_rows_have_the_bits_of_single_rows(gpu, oracle, row_bytes, paged,
         assert np.array_equal(together, alone) and not together[0].any() and together[8].any()
     for b in (pool_buffer, table, kb, vb, ib, cb, qb, gb, out, scratch):
         gpu.release(b)
+
+
+def _lists(gpu, f16, rows, heads, kv_heads, entries):
+    """Whether a call of this shape is worked a row's whole list a workgroup: the form by chunks writes partial results to its scratch."""
+    context = 2560
+    pool, buffer = gpu.kv_pool(1, context, kv_heads, 256, 512 if f16 else 272)
+    indices, counts = gpu.buffer(rows * entries * 4), gpu.upload(np.ones(rows, np.float32))
+    q, out = gpu.buffer(rows * heads * 512), gpu.buffer(rows * heads * 512)
+    scratch = gpu.buffer(gpu.selected_attention_scratch(rows, kv_heads, entries))
+    gpu.selected_attention(pool, None, context, 2048, indices.base(), entries, counts.base(), q.base(), True, rows, heads, 0.0625, out.base(), True, scratch)
+    written = gpu.read_buffer(scratch, 0, np.uint32, min(scratch.size // 4, 1 << 20)).any()
+    for b in (buffer, indices, counts, q, out, scratch):
+        gpu.release(b)
+    return not written
+
+
+@pytest.mark.parametrize("f16,rows,heads,kv_heads,entries,lists", [
+    (0, 64, 24, 2, 2052, True), (0, 63, 24, 2, 2052, False), (1, 22, 24, 2, 2052, True), (1, 21, 24, 2, 2052, False), (0, 64, 24, 2, 1024, False), (0, 96, 24, 2, 1024, True),
+    (0, 64, 24, 2, 512, False), (0, 24, 64, 8, 512, True), (1, 32, 24, 2, 512, True), (1, 31, 24, 2, 512, False), (0, 256, 8, 1, 256, True), (0, 64, 16, 4, 256, False),
+    (0, 64, 8, 8, 256, True), (1, 64, 24, 2, 256, True), (0, 256, 24, 2, 128, True), (0, 255, 24, 2, 128, False), (0, 256, 8, 8, 128, False), (1, 256, 16, 4, 128, False),
+    (1, 32, 24, 2, 128, True), (0, 32, 16, 4, 2052, False), (0, 64, 16, 4, 2052, True), (0, 64, 24, 2, 64, True), (0, 128, 16, 4, 33, True), (0, 256, 16, 8, 32, False), (1, 100, 8, 8, 1, False)])
+def test_the_line_between_lists_and_chunks(gpu, f16, rows, heads, kv_heads, entries, lists):
+    # either side of each line of the rule (a card of 256 compute units)
+    assert gpu.compute_units() == 256
+    assert _lists(gpu, f16, rows, heads, kv_heads, entries) == lists
+
+
+@pytest.mark.parametrize("row_bytes,rows,heads,kv_heads,selected", [(272, 130, 16, 2, 20), (272, 70, 8, 8, 200), (272, 257, 16, 2, 128), (512, 66, 24, 2, 128), (272, 200, 8, 1, 600),
+                                                                    (272, 30, 24, 2, 128), (272, 30, 24, 2, 1000), (272, 30, 24, 2, 1200)])
+def test_short_lists_have_the_bits_of_single_rows(gpu, oracle, row_bytes, rows, heads, kv_heads, selected):
+    # both forms, and merges of four, eight and more chunks: the same bits as every row alone
+    rng = np.random.default_rng(rows + selected)
+    context = 2048
+    pool, pool_buffer = gpu.kv_pool(1, context, kv_heads, 256, row_bytes)
+    table = gpu.upload(np.zeros(1, np.int32))
+    kb, vb = (gpu.upload(rng.standard_normal((context, kv_heads, 256)).astype(np.float32)) for _ in range(2))
+    gpu.kv_write(pool, table.base(), 1, gpu.upload(np.zeros(1, np.int32)).base(), kb.base(), vb.base(), False, 1, context)
+    base = context - rows
+    counts = np.where(np.arange(rows) % 3 == 0, selected, rng.integers(0, selected + 1, size=rows)).astype(np.float32)
+    indices = np.stack([np.sort(rng.permutation(base)[:selected]) for _ in range(rows)]).astype(np.float32)
+    q = rng.standard_normal((rows, heads, 256)).astype(np.float32)
+    ib, cb, qb = (gpu.upload(x) for x in (indices, counts, q))
+    out, scratch = gpu.buffer(q.size * 4), gpu.buffer(gpu.selected_attention_scratch(rows, kv_heads, selected))
+
+    def run(first, count):
+        gpu.selected_attention(pool, None, context, base + first, ib.at(first * selected * 4), selected, cb.at(first * 4), qb.at(first * heads * 1024), False, count, heads, 0.0625,
+                               out.at(first * heads * 1024), False, scratch)
+    run(0, rows)
+    together = _read(gpu, out, np.uint32, q.size)
+    gpu.write_buffer(out, 0, np.zeros(q.size, np.float32))
+    for r in range(rows):
+        run(r, 1)
+    assert np.array_equal(together, _read(gpu, out, np.uint32, q.size)) and together.any()
+    for b in (pool_buffer, table, kb, vb, ib, cb, qb, out, scratch):
+        gpu.release(b)
