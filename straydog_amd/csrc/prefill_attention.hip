@@ -1449,9 +1449,12 @@ void prefill_attention(Device& d, const sdx_kv_pool* pool, const int32_t* page_t
     // of 1500 128 / 73, 32 of 8192 319 / 342).
     const uint64_t items = seqs * pool->kv_heads, groups = items * ((args.rows + WIDE_GROUP - 1) / WIDE_GROUP);
     // It is also the better one for up to 128 keys where its workgroups are one round of the card: the operands are a launch more (64 tokens
-    // at 0 12.2 / 10.3, 128 14.3 / 13.2, 200 16.4 / 18.3; 4 sequences of 64 12.5 / 10.8, 16 of 64, more than a round, 14.8 / 21.5).
+    // at 0, first / second, 12.2 / 10.3 us, 128 14.3 / 13.2, 200 16.4 / 18.3; 4 sequences of 64 12.5 / 10.8, 16 of 64, more than a round, 14.8 / 21.5).
     const bool few_keys = max_context <= 128 && items * ((args.rows + GROUPS * 16 - 1) / (GROUPS * 16)) <= d.compute_units;
-    const bool converting = few_keys || (args.rows <= WIDE_GROUP && items * 8 > uint64_t(d.compute_units) * 3);
+    // And for up to 128 rows a K/V head and 448 keys of an eighth as many items as the card has units (second / first, 32 items: 64 rows of 364 keys 24 / 26, 96 of 312
+    // 22 / 25, 128 of 428 27 / 31, 36 of 2036 97 / 41; 64 items of 308 22 / 28; 16 of 303 20 / 16).
+    const bool few_rows = args.rows <= WIDE_GROUP && (items * 8 > uint64_t(d.compute_units) * 3 || (max_context <= 448 && items * 8 >= d.compute_units));
+    const bool converting = few_keys || few_rows;
     if (!converting && (uintptr_t(q) | uintptr_t(out)) % 16 == 0 && groups < (uint64_t(1) << 24) && (q8 ? launch_operands<true>(d, args) : launch_operands<false>(d, args))) return;
     if (q8) launch<256, 1, true, 2>(d, args, unsigned(seqs)); else launch<256, 1, false, 2>(d, args, unsigned(seqs));
 }
