@@ -1106,7 +1106,11 @@ void launch_scores(Device& d, const float* q, const void* keys, bool bf16, size_
                    size_t rows, size_t groups, size_t heads, size_t dim, float scale, float* scores, size_t score_stride,
                    const int32_t* candidates, size_t blocks, size_t block) {
     const size_t scored = candidates ? blocks * block : groups;
-    if (dim == 128 && (uintptr_t(q) | uintptr_t(keys)) % 16 == 0) {
+    // The matrix products' tiles are 32 heads: up to four over BF16 keys are the vector units' where there are 256 scores a compute unit (256 rows x 8256
+    // groups, vector / matrix: one head 100 / 166 us, four 135 / 165, eight 192 / 165; 8 x 16250 11.5 / 13.9 and 15.0 / 14.5; one row 9.5 / 7.6 and
+    // 12 / 7.6; FP32 keys, which the vector kernel reads a value at a time, 256 rows of one head 515 / 242).
+    const bool vector = bf16 && heads <= 4 && rows * scored >= 256 * size_t(d.compute_units);
+    if (dim == 128 && !vector && (uintptr_t(q) | uintptr_t(keys)) % 16 == 0) {
         // Waves are single workgroups, two a SIMD (eight a compute unit) at once.  A row's tiles of 64 groups are cut into equal runs,
         // one a wave, so that the waves fill whole rounds of the card; a run costs its tiles and about one more for the row's queries.
         // (256 rows x 129 tiles: runs of 17, one round, 312 us; 8, two and a bit, 364 us; 1, 401 us.)

@@ -628,7 +628,7 @@ def test_sparse_path_operands_off_16_byte_boundaries(gpu, oracle):
         gpu.release(b)
 
 
-@pytest.mark.parametrize("heads,groups,rows", [(1, 1, 1), (31, 63, 2), (32, 64, 1), (33, 65, 3), (64, 300, 2), (64, 16500, 1), (32, 1030, 40), (64, 8200, 70)])
+@pytest.mark.parametrize("heads,groups,rows", [(1, 1, 1), (4, 300, 3), (4, 1100, 60), (5, 1100, 60), (31, 63, 2), (32, 64, 1), (33, 65, 3), (64, 300, 2), (64, 16500, 1), (32, 1030, 40), (64, 8200, 70)])
 def test_matrix_core_chains_are_the_canonical_scores(gpu, oracle, heads, groups, rows):
     # 128 columns go through the FP32 matrix instruction: the same bits at the edges of its tiles (32 heads, 64 groups, several tiles a
     # wave), with values whose products are denormal among them, nothing or everything visible, FP32 and BF16 keys
