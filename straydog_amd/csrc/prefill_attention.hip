@@ -1270,8 +1270,10 @@ __global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_e
         #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
             const float top = fmaxf(fmaxf(fmaxf(s[qt][0][0], s[qt][0][1]), fmaxf(s[qt][0][2], s[qt][0][3])), fmaxf(fmaxf(s[qt][1][0], s[qt][1][1]), fmaxf(s[qt][1][2], s[qt][1][3])));
-            // (from the first step on: nothing has been seen yet; a row that sees none of a share's keys keeps that)
-            if (__any(fmaf(top, args.scale_log2, -ref[qt]) > SLACK)) {
+            // (from the first step on: nothing has been seen yet; a row that sees none of a share's keys keeps that).  In the first four steps the
+            // reference follows every new maximum: a row of few keys has its largest weight exact in FP16 then, as the kernel that converts in its
+            // loop has (2 x 1531 tokens, distance from 64 bits 3.80e-4 without, 3.76e-4 with, there 3.77e-4; 0.3 us of 82).
+            if (__any(fmaf(top, args.scale_log2, -ref[qt]) > (step < begin + 4 ? 0.0f : SLACK))) {
                 asm volatile("; new reference maxima" ::: "memory");
                 const float higher = fmaxf(ref[qt], row_max(top) * args.scale_log2), alpha = __builtin_amdgcn_exp2f(ref[qt] - higher);
                 ref[qt] = higher;

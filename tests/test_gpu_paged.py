@@ -730,3 +730,30 @@ def test_prompts_of_256_columns_do_not_depend_on_the_capacity(gpu, oracle, fmt, 
         assert np.array_equal(result.view(np.uint32), got[0].view(np.uint32))
     for b in (buffer, tb, pb, qb, out, wb):
         gpu.release(b)
+
+
+def test_the_largest_weight_of_a_row_of_few_keys_is_exact(gpu, oracle):
+    # two keys share the weight, in different steps of 32: the larger weight is one, which FP16 holds, and the other key's value is zero, so
+    # the output is right to FP32 (rounded to FP16 against the first key's maximum it was up to 1e-4 away)
+    dim, page_tokens, span, heads, scale = 256, 64, 64, 16, 0.0625
+    context, capacity = 700, 1024
+    worst = 0.0
+    for larger in (0.703125, 0.84375, 1.171875, 1.40625, 1.7421875, 2.0390625):
+        k = np.zeros((1, context + span, 1, dim), np.float32)
+        k[0, :, 0, 0] = -1000.0
+        k[0, 3, 0, 0], k[0, 35, 0, 0] = 0.0, larger * 16
+        v = np.zeros((1, context + span, 1, dim), np.float32)
+        v[0, 35] = 1.0
+        table = np.zeros((1, capacity // page_tokens), np.int32)
+        table[0] = np.arange(capacity // page_tokens)[::-1]
+        host = np.zeros(oracle.pool_bytes(16, 1, page_tokens, 512), dtype=np.uint8)
+        oracle.kv_write(host, 512, page_tokens, 1, dim, table, np.zeros(1, np.int32), k, v)
+        pool, buffer = gpu.kv_pool(16, page_tokens, 1, dim, 512)
+        gpu.write_buffer(buffer, 0, host)
+        q = np.zeros((1, span, heads, dim), np.float32)
+        q[..., 0] = 1.0
+        got = _run(gpu, pool, table, gpu.upload(table), [context], q, span, heads, scale, False, False, max_context=capacity)
+        worst = max(worst, np.abs(got - 1.0 / (1.0 + np.exp(-larger))).max())
+        gpu.release(buffer)
+    # an exponential, a sum and a quotient in FP32
+    assert worst <= 1e-6
