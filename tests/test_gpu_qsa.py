@@ -561,15 +561,20 @@ def test_decode_stage_in_one_call_equals_its_parts(gpu, oracle, row_bytes, paged
     assert np.all(np.isfinite(got["attended"])) and np.abs(got["attended"]).max() > 0
 
 
-@pytest.mark.parametrize("row_bytes,paged,context,first,spans", [(272, True, 4096, 1990, (100,)), (512, False, 40960, 36001, (64, 37))])
-def test_prompt_chunk_stage_in_one_call_equals_its_parts(gpu, oracle, row_bytes, paged, context, first, spans):
+# (a wave takes one vector of a row, from 128 rows on two and from 512 on eight; eight K/V heads leave a wave more than one key to encode)
+@pytest.mark.parametrize("row_bytes,paged,context,first,spans,kv_heads", [(272, True, 4096, 1990, (100,), 2), (512, False, 40960, 36001, (64, 37), 2),
+                                                                          (272, True, 4096, 1990, (128, 129), 8), (512, False, 4096, 701, (130, 127), 8),
+                                                                          (272, True, 4096, 1001, (512, 511), 8), (512, False, 4096, 1990, (520, 33), 2)])
+def test_prompt_chunk_stage_in_one_call_equals_its_parts(gpu, oracle, monkeypatch, row_bytes, paged, context, first, spans, kv_heads):
     # sdx_qsa_prefill_attend (the stage of qsa_prefill, gpu/sparse_attention.hpp:444-506): normalised rows, K/V bytes, pooled blocks
     # and ring equal those of sdx_qsa_normalize + sdx_kv_write + sdx_qsa_pool over the span, and the attended rows equal
     # sdx_qsa_index_interval + sdx_selected_attention (gated) on them, bit for bit: before the 512-block line and across it with
     # the exact kernels, and past 32768 positions by intervals, the packed keys carried from one chunk to the next
     rng = np.random.default_rng(context + first)
-    heads, kv_heads = 24, 2
-    pool_blocks, stride = context // 4 + 1, 24 * 512 + 2 * 512 + 640 + 5
+    held, buffer_of = [], gpu.buffer
+    monkeypatch.setattr(gpu, "buffer", lambda size: held.append(buffer_of(size)) or held[-1])       # (given back at the end)
+    heads = 24
+    pool_blocks, stride = context // 4 + 1, 24 * 512 + kv_heads * 512 + 640 + 5
     norms = [(0.4 + 1.2 * rng.random(n)).astype(np.float32) for n in (256, 256, 128, 128)]
     blocks = np.zeros((128, pool_blocks), dtype=np.float32)
     blocks[:, :first // 4] = rng.standard_normal((128, first // 4)).astype(np.float32)
@@ -578,11 +583,11 @@ def test_prompt_chunk_stage_in_one_call_equals_its_parts(gpu, oracle, row_bytes,
     pages = context // page_tokens
     order = rng.permutation(pages).astype(np.int32)
     if row_bytes == 272:
-        filled = rng.integers(0, 256, pages * 4 * page_tokens * row_bytes, dtype=np.uint8)
+        filled = rng.integers(0, 256, pages * 2 * kv_heads * page_tokens * row_bytes, dtype=np.uint8)
         rows = filled.reshape(-1, 272)
         rows[:, 256:] = np.tile(np.frombuffer(np.float16(0.01).tobytes(), np.uint8), 8)
     else:
-        filled = rng.standard_normal(pages * 4 * page_tokens * 256).astype(np.float16).view(np.uint8)
+        filled = rng.standard_normal(pages * 2 * kv_heads * page_tokens * 256).astype(np.float16).view(np.uint8)
     most = max(spans)
 
     def fresh():
@@ -634,7 +639,6 @@ def test_prompt_chunk_stage_in_one_call_equals_its_parts(gpu, oracle, row_bytes,
         for what in ("kv", "blocks", "history", "projections", "attended"):
             assert np.array_equal(got[what].view(np.uint8), want[what].view(np.uint8)), f"{what} after the chunk at {at}"
         assert valid_one == valid_two and np.all(np.isfinite(got["attended"])) and np.abs(got["attended"]).max() > 0
-        gpu.release(start)
         at += steps
     if first >= 32768:
         assert valid_one[0] > 0, "past 32768 positions the packed keys are carried to the next chunk"
@@ -642,6 +646,8 @@ def test_prompt_chunk_stage_in_one_call_equals_its_parts(gpu, oracle, row_bytes,
         gpu.qsa_prefill_attend(state, one["projections"].base(), stride, most, first, gpu.buffer(4096), one["attended"].base())
     with pytest.raises(RuntimeError, match="inside the context"):
         gpu.qsa_prefill_attend(state, one["projections"].base(), stride, most, context - 1, scratch, one["attended"].base())
+    for buffer in held:
+        gpu.release(buffer)
 
 
 @pytest.mark.parametrize("row_bytes,paged,rows,f16", [(272, True, 65, False), (272, False, 70, True), (512, True, 64, True), (512, False, 35, False)])
