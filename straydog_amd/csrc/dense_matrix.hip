@@ -16,7 +16,8 @@
 //   * Values that are no finite numbers: found in the finished sums, which they always reach (a weight of zero does not silence
 //     them), and the workgroup's run is worked again in plain arithmetic (plain_attention.hpp).  Kept out of the products in the loop
 //     instead, and counted beside them by sign, they cost the loop registers: 120 us for the 115 below.
-// Measured, 128 rows x 16 heads over 2 K/V heads of 256 columns at position 4096 (8.7 GFLOP): 115 us with the merge (76 TFLOP/s) where the general kernel
+// Measured, 128 rows x 16 heads over 2 K/V heads of 256 columns at position 4096 (8.7 GFLOP): 115 us (76 TFLOP/s; 107 the kernel, 8 the merge; in the
+// first milliseconds of load 118-122 the kernel) where the general kernel
 // (LDS-fed vector FMAs, a workgroup a row and K/V head) took 5360; one row at 4096: 17 us where it took 295, at 60: 10 where it took 31.
 #include "paged_rows.hpp"
 #include "plain_attention.hpp"

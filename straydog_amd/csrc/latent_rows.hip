@@ -6,8 +6,9 @@
 // FP32 in, FP32 out: the products run on v_mfma_f32_16x16x32_bf16, sixteen times the FP32 matrix rate, with every FP32 operand as
 // three BF16 terms (value, what its rounding left, what that one's left: 24 bits, exact).  A BF16 row has one term, so a score is
 // three products a column and a value sum three (the weights' terms); a row in FP32 (the window's, or compressed rows in FP32)
-// takes the six pairs of terms above 2^-24.  Each order of magnitude has accumulators of its own, added smallest first.  An FP32 row
-// whose values fit BF16 gives the bits of the tagged BF16 row: the extra products add zeros.  Infinities, NaNs and numbers past BF16's
+// takes the six pairs of terms above 2^-24; the three smallest pairs, below the last place of an FP32 product, are left out.  A score
+// has an accumulator for each order of magnitude, added smallest first; a value sum has one, which takes a step's planes of terms
+// smallest first.  An FP32 row whose values fit BF16 gives the bits of the tagged BF16 row: the extra products add zeros.  Infinities, NaNs and numbers past BF16's
 // largest make NaNs of the sums they reach: the workgroup's run is then worked again in plain arithmetic (plain_attention.hpp); the
 // test for it, once a run, is 0.5 us of one row's 54 and nothing that shows of 256 rows' 418.
 //
@@ -18,14 +19,14 @@
 //     value columns (64 registers).  That fits two waves a SIMD, which a wave with all 512 columns (320 registers) does not;
 //   * a wave brings in whole rows (32 / waves of them a step, the row's address the wave's): BF16 rows go from memory to a padded tile
 //     in LDS by themselves, a step ahead, their numbers in the selection read another step ahead (fetched through registers they left
-//     51 registers to spill, and each number waited for the row before it: 128 us, then 109, now 97); FP32 rows are split into three
+//     51 registers to spill, and each number waited for the row before it: 128 us, then 109, then 97); FP32 rows are split into three
 //     planes of terms on their way;
 //   * the scores S^T = K . Q^T leave the weights in the B-operand layout of O^T += V^T . P^T; a lane's place in a value operand
 //     stands for eight neighbouring columns in eight products, so nothing is transposed (as in latent_gather.hip).
 // Many rows (a prompt) give every compute unit a workgroup that finishes its outputs; few rows are cut into runs of steps whose
 // (maximum, sum, unnormalised outputs) latent_rows_merge_kernel puts together.
-// Measured at 64 heads, a window of 128 and 512 selected BF16 rows: 256 rows in 97 us where the general kernel (FP32 on the vector
-// units, a key row read once for eight heads) took 1400; one row in 14 + 4.6 us where it took 447.  Of the 97 us the
+// Measured at 64 heads, a window of 128 and 512 selected BF16 rows: 256 rows in 89 us (93-97 in the first milliseconds of load, as the figures above) where the general kernel (FP32 on the vector
+// units, a key row read once for eight heads) took 1400; one row in 15.4 + 4.6 us where it took 447.  Of the 97 us the
 // queries and outputs take 13 (67 MB); a step of BF16 rows takes 3.3 us, of which its products are 1.4 and its LDS reads, in phase with them, 0.9.  The differences from 64-bit
 // arithmetic are as large as before, 1e-6 at outputs of order one.
 #include "paged_rows.hpp"

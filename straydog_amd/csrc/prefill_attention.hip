@@ -1165,7 +1165,8 @@ __device__ __forceinline__ unsigned used_shares(unsigned cached, unsigned tiles_
 // the next tile on its way while this one is multiplied; one meeting a step.  64 KB of LDS and 256 registers: two workgroups a compute
 // unit, so that one multiplies while the other forms its weights.  A step is 64 products a wave (1024 cycles) and 32 reads of LDS: the
 // LDS (160 bytes a cycle asked of its 128 with the tiles' arrival) bounds it ahead of the products.
-// Measured, 2 x 1531 tokens of 24 heads over 2 (57.6 GFLOP): 73 us (0.78 PFLOP/s) where the kernel that converts in its loop takes 205.
+// Measured, 2 x 1531 tokens of 24 heads over 2 (57.6 GFLOP): 66 us (0.87 PFLOP/s; 75-78 us in the first milliseconds of load) where the kernel
+// that converts in its loop takes 205.
 __global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_eu(2, 2))) prefill_operands_kernel(PrefillArgs args, const uint8_t* tiles_in,
                                                                                                              unsigned tiles_per_seq, unsigned most, float* partial) {
     // The longest walks first.  (Paired so that a compute unit's second workgroup is the shorter the longer its first: no faster.)

@@ -4,7 +4,10 @@
 // with the validity rule of attention_scores (gpu/kernels.cpp:100-165: an entry counts iff 0 <= raw <= position and
 // raw < context) and the output gate qsa_gate (gpu/sparse_attention.hpp:439-442, sigmoid as gpu/core.hpp:1108-1111).
 //
-// Shape of the work on gfx950: a workgroup of 4 waves owns (row, K/V head, 128 entries of the row's list); a wave takes 32
+// Two forms on gfx950, with the same bits: the chunks of a list on workgroups of their own, described here, and for many rows a workgroup
+// for a row's whole list (selected_list_kernel; lists_pay says where).
+//
+// Chunks: a workgroup of 4 waves owns (row, K/V head, 128 entries of the row's list); a wave takes 32
 // entries, one per lane for the address arithmetic (list entry -> position -> page -> row address), and gathers the 32 K rows
 // and 32 V rows into its LDS stage by 16-byte global->LDS loads whose lanes each name their own piece of a row (a row is 17 or
 // 32 such pieces), so a gathered step lands in the stage exactly as a contiguous step of the paged decode kernel does and the
