@@ -1,9 +1,8 @@
 // Devices, allocations and transfers of the C ABI (reference gpu/kernels.cpp:3511-3614 sd_create, :4555-4592 sd_buffer*,
 // gpu/host_io.hpp:81-180 upload/download/allocate), for one MI355X per handle.
-#include "device.hpp"
+#include "kernels.hpp"
 
 #include "../../include/straydog_gpu.h"
-#include "../../include/straydog_gpu_ext.h"
 
 #include <algorithm>
 #include <cstring>
@@ -11,9 +10,6 @@
 namespace sd {
 
 thread_local std::string last_error;
-void paged_attention_setup(Device& d);   // paged_attention.hip
-void harness_setup(Device& d);           // harness.hip
-void select_thin_reserve(Device& d);     // block_index.hip
 
 // Recorded graphs hold the addresses their ops were given.  When a buffer the library owns moves (the workspace grows), the
 // graphs recorded so far would replay on freed memory: they are dropped, sd_graph_run then answers 1 ("none stored under

@@ -16,10 +16,9 @@
 // prefill chunk (FP32 FMA-bound); a 1024-thread workgroup per row for the selection, the row's scores read once and held in LDS (and registers,
 // beyond 32768 blocks), four 8-bit radix passes over per-wave LDS histograms (the first, where nearly all values share a digit, counted by ballots), and
 // one ordered pass whose slots come from 64-wide ballots and a scan over (run, wave) counts.
-#include "device.hpp"
+#include "kernels.hpp"
 #include "kv_codec.hpp"
 #include "tree_sum.hpp"
-#include "../../include/straydog_gpu_ext.h"
 
 using namespace sd;
 
@@ -728,13 +727,6 @@ void launch_rows(Device& d, const float* queries, size_t stride, const float* bl
 }  // namespace
 
 namespace sd {
-void validate_pool(Device& d, const sdx_kv_pool* pool);     // kv_write.hip
-// block_interval.hip
-size_t interval_scratch_bytes(size_t steps, size_t pool);
-bool interval_serves(size_t base);
-const uint32_t* interval_select(Device& d, const float* queries, size_t stride, const float* blocks, size_t pool, size_t base, size_t steps,
-                                size_t selected, float* scores, float* indices, float* counts, void* scratch, uint64_t* valid, unsigned* gate);
-size_t interval_undecided(Device& d, const void* scratch, size_t steps, size_t pool);
 // The lists of a short span's thinned rows: allocated once per handle, never while a graph is being recorded (sd_graph_begin
 // calls this first, so that a recorded pass takes the same path as an eager one).
 constexpr size_t thin_list_bytes = size_t(THIN_ROWS) * THIN_SEGMENTS * THIN_CAP * sizeof(uint2);

@@ -22,8 +22,7 @@
 // result.  Among the kept blocks the 512th highest lower bound Lk and upper bound Uk split them: lower bound above Uk is
 // certainly selected, upper bound below Lk certainly not, the rest (the band) is scored exactly, in the exact kernels' order of
 // operations, and T is the (512 - certain)th highest of those; ties at T go to the earliest blocks, the list is in block order.
-#include "device.hpp"
-#include "../../include/straydog_gpu_ext.h"
+#include "kernels.hpp"
 
 #include <algorithm>
 #include <type_traits>

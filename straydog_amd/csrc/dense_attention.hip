@@ -6,18 +6,11 @@
 // key sums its columns in order), the online softmax runs a wave per head with lane = key, values are summed a
 // thread per column.  The splits' (max, sum, unnormalised output) are merged by a second kernel that also applies
 // the optional sigmoid gate.
-#include "device.hpp"
+#include "kernels.hpp"
 #include "kv_codec.hpp"
 #include "../../include/straydog_gpu.h"
 
 using namespace sd;
-
-namespace sd {
-bool dense_matrix_supported(uint64_t context, uint64_t rows, uint64_t heads, uint64_t kv_heads, uint64_t dim, const float* q, const float* keys, const float* values,
-                            const float* gate, const float* out);
-void dense_matrix(Device& d, const float* q, const float* keys, const float* values, uint64_t context, const int32_t* positions, uint64_t rows, uint64_t heads,
-                  uint64_t kv_heads, uint64_t dim, float scale, const float* gate, float* scratch, uint64_t scratch_splits, float* out);
-}
 
 namespace {
 

@@ -19,6 +19,7 @@
 // Measured, 128 rows x 16 heads over 2 K/V heads of 256 columns at position 4096 (8.7 GFLOP): 115 us (76 TFLOP/s; 107 the kernel, 8 the merge; in the
 // first milliseconds of load 118-122 the kernel) where the general kernel
 // (LDS-fed vector FMAs, a workgroup a row and K/V head) took 5360; one row at 4096: 17 us where it took 295, at 60: 10 where it took 31.
+#include "kernels.hpp"
 #include "paged_rows.hpp"
 #include "plain_attention.hpp"
 #include "../../include/straydog_gpu.h"
@@ -32,12 +33,6 @@ using namespace sd::paged;
 namespace {
 
 typedef float floatx16 __attribute__((ext_vector_type(16)));
-constexpr float LOG2E = 1.44269504088896341f;
-template<int N> __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14)); }
-
-// The same number, in a way the compiler cannot see through: what is formed from it inside a loop (addresses) is formed there and does
-// not sit in registers through it.
-__device__ __forceinline__ int fresh(int x) { asm volatile("" : "+v"(x)); return x; }
 
 struct DenseArgs {
     const float *q, *keys, *values;

@@ -1,14 +1,11 @@
 // Entry points for harnesses, none of them on the attention path: seeded device-side fills for synthetic workloads, a plain
 // copy and read-only streaming probes (the measured memory ceilings a benchmark reports beside the roofline), a matrix-core
 // probe (the measured dense FP16 ceiling).
-#include "device.hpp"
-#include "../../include/straydog_gpu_ext.h"
+#include "kernels.hpp"
 
 #include <hip/hip_fp16.h>
 
 using namespace sd;
-
-namespace sd { void validate_pool(Device& d, const sdx_kv_pool* pool); }
 
 namespace {
 

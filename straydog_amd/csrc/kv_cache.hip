@@ -21,17 +21,12 @@
 // back to the host pages with `unstage` (kv_after_prefill, gpu/kv_stage.hpp:151-155).  `grow` is sd_kv_grow's VRAM
 // branch for a pool (gpu/kernels.cpp:4048-4140): a larger allocation, the pages copied on the device, the old one
 // released, recorded graphs dropped.
-#include "device.hpp"
-#include "../../include/straydog_gpu_ext.h"
+#include "kernels.hpp"
 
 #include <algorithm>
 #include <memory>
 
 using namespace sd;
-
-namespace sd {
-void validate_pool(Device& d, const sdx_kv_pool* pool);
-}
 
 namespace {
 

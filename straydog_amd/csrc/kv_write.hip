@@ -1,9 +1,8 @@
 // Appending rows to the paged K/V cache.
 // The Q8_0 arithmetic is the reference's kv_encode/kv_put (gpu/kernels.cpp:58-74): scale = f16(max|x| / 127) over a
 // 32-value block, q = clamp(rint(x / f32(scale)), -127, 127), q = 0 when the scale is 0.
-#include "device.hpp"
+#include "kernels.hpp"
 #include "kv_codec.hpp"
-#include "../../include/straydog_gpu_ext.h"
 
 #include <hip/hip_fp16.h>
 

@@ -6,23 +6,10 @@
 //
 // A workgroup owns one row and 8 of its heads, so a gathered row is read once for 8 heads: scores with 8 adjacent
 // lanes (the heads) sharing a key row, a wave per head for the softmax, then a thread per output column.
-#include "device.hpp"
+#include "kernels.hpp"
 #include "../../include/straydog_gpu.h"
-#include "../../include/straydog_gpu_ext.h"
 
 using namespace sd;
-
-namespace sd {
-bool latent_gather_supported(uint64_t kdim, uint64_t vdim);
-uint64_t latent_gather_scratch(uint64_t batch, uint64_t k, uint64_t heads, uint64_t vdim);
-void latent_gather(Device& d, const void* q, const void* latents, const int32_t* selected, uint64_t batch, uint64_t groups, uint64_t k,
-                   uint64_t heads, float scale, float* out, float* partial);
-bool latent_rows_supported(uint64_t dim, uint64_t raw_rows, uint64_t window, uint64_t compressed_rows, uint64_t selections, const void* q, const void* raw,
-                           const void* compressed, const void* out);
-void latent_rows(Device& d, const float* q, const float* raw, uint64_t raw_rows, const int32_t* positions, uint64_t window, const void* compressed, bool bf16,
-                 uint64_t compressed_rows, const int32_t* selected, uint64_t selections, const float* sinks, uint64_t rows, uint64_t heads, float scale,
-                 uint64_t pairs, const float* frequencies, const double2* turns, float* out);
-}
 
 namespace {
 

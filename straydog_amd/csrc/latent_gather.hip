@@ -15,6 +15,7 @@
 //   * S^T = K . Q^T (rows x heads) leaves the weights in the B-operand layout of O^T += V^T . P^T, so they never move
 //     between lanes (the layout notes of paged_rows.hpp apply);
 //   * the chunks' (maximum, sum, unnormalised output) are merged by a second kernel.
+#include "kernels.hpp"
 #include "paged_rows.hpp"
 
 using namespace sd;

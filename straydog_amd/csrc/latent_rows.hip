@@ -29,6 +29,7 @@
 // units, a key row read once for eight heads) took 1400; one row in 15.4 + 4.6 us where it took 447.  Of the 97 us the
 // queries and outputs take 13 (67 MB); a step of BF16 rows takes 3.3 us, of which its products are 1.4 and its LDS reads, in phase with them, 0.9.  The differences from 64-bit
 // arithmetic are as large as before, 1e-6 at outputs of order one.
+#include "kernels.hpp"
 #include "paged_rows.hpp"
 #include "plain_attention.hpp"
 
@@ -42,7 +43,6 @@ namespace {
 typedef __bf16 bf16x8 __attribute__((ext_vector_type(8)));
 
 constexpr int DIM = 512, HALF = DIM / 2, PITCH = 2 * DIM + 16, PLANE = STEP * PITCH, PAIRS_MAX = 64;
-constexpr float LOG2E = 1.44269504088896341f;
 
 struct RowsArgs {
     const float* q;                    // [rows][heads][512]
@@ -77,8 +77,6 @@ __device__ __forceinline__ void split_pair(float x, float y, uint32_t& high, uin
     x -= __uint_as_float(middle << 16); y -= __uint_as_float(middle & 0xffff0000u);
     low = to_bf16_pair(x, y);
 }
-// every load of the wave, those to LDS included
-__device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(0)" ::: "memory"); }
 struct Terms { uint4 high, middle, low; };       // eight values
 __device__ __forceinline__ Terms split_eight(const float (&x)[8]) {
     Terms t;
@@ -249,7 +247,7 @@ __global__ void __launch_bounds__(128 * HT, HT == 4 ? 2 : 1) latent_rows_kernel(
             }
         } else {
             if (step == begin || step == raw_steps) ask(step);
-            wait_loads();
+            wait_loads_here<0>();
             #pragma unroll
             for (int j = 0; j < MINE; ++j) {
                 const int r = wave + WAVES_HERE * j;

@@ -14,21 +14,12 @@
 //     global->LDS loads into the wave's own LDS stage, operands are read from there in MFMA layout, and the next step's
 //     copy is in flight while this step is computed;
 //   * operand layouts and the Q8_0 -> FP16 conversion: paged_rows.hpp.
+#include "kernels.hpp"
 #include "paged_rows.hpp"
 
 #include <cstdlib>
 #include <type_traits>
 
-namespace sd {
-void validate_pool(Device& d, const sdx_kv_pool* pool);
-void prefill_attention(Device& d, const sdx_kv_pool* pool, const int32_t* page_table, uint64_t table_stride, const int32_t* positions,
-                       uint64_t max_context, const void* q, int q_f16, uint64_t seqs, uint64_t span, uint64_t heads, float scale, void* out,
-                       int out_f16);
-void prefill_chunk(Device& d, const sdx_kv_pool* pool, const int32_t* page_table, uint64_t table_stride, const int32_t* positions,
-                   uint64_t max_context, const void* keys, const void* values, int kv_f16, const void* q, int q_f16, uint64_t seqs, uint64_t span,
-                   uint64_t heads, float scale, void* out, int out_f16, void* tiles, const int32_t* valid);
-uint64_t prefill_tiles_bytes(uint64_t seqs, uint64_t kv_heads, uint64_t max_context);
-}
 using namespace sd;
 using namespace sd::paged;
 
@@ -106,8 +97,6 @@ __device__ __forceinline__ bool locate(const PagedArgs& args, unsigned u, Segmen
 
 constexpr float SLACK = 8.0f;     // how far (base-2 exponent) a row's true maximum may run ahead of its reference maximum
 constexpr int stages_per_wave(int slab, int occupancy) { return occupancy <= 2 && WAVES * 2 * 2 * slab * occupancy <= 160 * 1024 ? 2 : 1; }
-// s_waitcnt for the vector-memory counter alone: wait until at most N of the wave's loads are outstanding.
-template<int N> __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14)); }
 
 // A step's K and V slabs (32 contiguous rows each) are copied by fully coalesced 16-byte global->LDS loads into the wave's
 // own LDS stage; operands are then read from LDS in MFMA layout while the next step's copy is in flight.  OCC = the waves per

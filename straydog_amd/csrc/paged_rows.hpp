@@ -21,7 +21,16 @@ typedef __attribute__((address_space(3))) void* lds_ptr;
 typedef __attribute__((address_space(4))) const int32_t* table_ptr;   // read through the scalar cache: a page number is wave-uniform
 
 constexpr int WAVES = 4, STEP = 32;
+constexpr float LOG2E = 1.44269504088896341f;
 constexpr float NEG_BIG = -1.0e30f;   // a finite "nothing seen yet" maximum: exp2(NEG_BIG - m) is 0, no inf - inf anywhere
+
+// s_waitcnt for the vector-memory counter alone: wait until at most N of the wave's loads are outstanding (loads to LDS are among them).
+template<int N> __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14)); }
+// The same where the compiler must also move no access to memory across it.
+template<int N> __device__ __forceinline__ void wait_loads_here() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
+// The same number, in a way the compiler cannot see through: the addresses formed from it inside a loop are formed there and do not
+// sit in registers through it.
+__device__ __forceinline__ int fresh(int x) { asm volatile("" : "+v"(x)); return x; }
 
 struct PagedArgs {
     const uint8_t* pages;

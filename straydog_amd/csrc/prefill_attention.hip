@@ -21,6 +21,7 @@
 //     workgroup; every wave builds its own operands from the raw rows in the stage (paged_rows.hpp); a quarter of the rows belongs to a pair of waves, one taking the first 32
 //     keys of every step and one the last 32, each with its own online softmax, merged through LDS at the end; the
 //     workgroups with the longest walks are dispatched first.
+#include "kernels.hpp"
 #include "paged_rows.hpp"
 #include "kv_codec.hpp"
 
@@ -37,9 +38,6 @@ constexpr float SLACK = 8.0f;     // how far (base-2 exponent) a row's true maxi
 constexpr int stages_for(int stage_bytes) { return 150 * 1024 / stage_bytes < 4 ? 150 * 1024 / stage_bytes : 4; }
 constexpr int GROUPS = 4, HALVES = 2, TEAM = GROUPS * HALVES;   // row quarters x key halves = waves of a workgroup
 constexpr int WALK = HALVES * STEP;                            // keys per step of the workgroup
-
-// s_waitcnt for the vector-memory counter alone: wait until at most N of the wave's loads are outstanding.
-template<int N> __device__ __forceinline__ void wait_loads() { __builtin_amdgcn_s_waitcnt(0x0f70 | (N & 15) | ((N >> 4) << 14)); }
 
 struct PrefillArgs {
     const uint8_t* pages;

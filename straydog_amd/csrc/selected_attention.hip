@@ -14,16 +14,13 @@
 // operand code (paged_rows.hpp) is shared: S^T = K . Q^T and O^T += V^T . P^T on v_mfma_f32_16x16x32_f16 with the group's
 // query heads (up to 16) as one tile.  The four waves merge through LDS; the workgroups' partial results (maximum, sum,
 // unnormalised output) are merged, normalised and gated by a second kernel, a block per (row, head).
+#include "kernels.hpp"
 #include "paged_rows.hpp"
 
 #include <type_traits>
 
 using namespace sd;
 using namespace sd::paged;
-
-namespace sd {
-void validate_pool(Device& d, const sdx_kv_pool* pool);
-}
 
 namespace {
 
@@ -293,10 +290,6 @@ template<bool Q8> struct ListShape {
     static constexpr int BYTES = STAGES + WAVES * 16 * 8 + LIST_MAX / 8;      // the list follows
     static_assert(STAGES >= WAVES * WAVES * 4 * 1024, "the waves' sums meet over the stages");
 };
-// The same number, in a way the compiler cannot see through: the addresses formed from it inside a loop are formed there and do not
-// sit in registers through it.
-__device__ __forceinline__ int fresh(int x) { asm volatile("" : "+v"(x)); return x; }
-template<int N> __device__ __forceinline__ void wait_loads() { asm volatile("s_waitcnt vmcnt(%0)" : : "n"(N) : "memory"); }
 // Four global->LDS loads to `to` and the three KiB after it, from four addresses a lane.
 __device__ __forceinline__ void load_four_to_lds(const uint8_t* const (&from)[4], uint32_t to) {
     uint32_t keep;
@@ -404,7 +397,7 @@ __global__ void __launch_bounds__(WAVES * 64, Q8 ? 2 : 1) selected_list_kernel(S
         if (++ahead_slab == 2 * n) { ahead_slab = 0; ++ahead_chunk; }
     };
     const auto landed = [&] {                               // the next slab, complete
-        if (asked - taken > 1) wait_loads<Shape::LOADS>(); else wait_loads<0>();
+        if (asked - taken > 1) wait_loads_here<Shape::LOADS>(); else wait_loads_here<0>();
         return ring + (taken++ & 1) * Shape::SLAB;
     };
     const auto read = [] { asm volatile("s_waitcnt lgkmcnt(0)" ::: "memory"); };       // its operands are in registers: it may be overwritten

@@ -13,20 +13,11 @@
 // Three launches before the walk: marks[tile][position] |= bit(token) for every entry that counts (at most the token's own
 // position, inside the context; sdx_selected_attention's rule); the counts of marked positions per 4096-position segment;
 // the ordered lists (position, mask) of every tile.  Any list does, sorted or not; an entry named twice counts once.
-#include "device.hpp"
-#include "../../include/straydog_gpu_ext.h"
+#include "kernels.hpp"
 
 #include <algorithm>
 
 using namespace sd;
-
-namespace sd {
-void validate_pool(Device& d, const sdx_kv_pool* pool);
-unsigned union_tile_rows();
-void prefill_union(Device& d, const sdx_kv_pool* pool, const int32_t* page_table, uint64_t base, const void* q, int q_f16, uint64_t tokens,
-                   uint64_t heads, float scale, const float* gate, uint64_t gate_stride, uint64_t gate_row_stride, void* out, int out_f16,
-                   const int32_t* union_pos, const uint32_t* union_mask, const uint32_t* union_count, unsigned union_cap);
-}
 
 namespace {
 
