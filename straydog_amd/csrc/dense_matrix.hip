@@ -319,9 +319,9 @@ __global__ void __launch_bounds__(256) dense_merge_kernel(DenseArgs a) {
             // (past the last run: its numbers again; they, and those of a run without a weight, may be none that zero silences)
             const bool real = s0 + GROUPS * n < a.splits && tops[n] != -INFINITY;
             const float weight = __builtin_amdgcn_exp2f((tops[n] - top) * LOG2E);
-            total += real ? parts[n] * weight : 0.0f;
+            total = real ? fmaf(parts[n], weight, total) : total;
             #pragma unroll
-            for (int j = 0; j < 4; ++j) sum[j] += real ? x[n][j] * weight : 0.0f;
+            for (int j = 0; j < 4; ++j) sum[j] = real ? fmaf(x[n][j], weight, sum[j]) : sum[j];
         }
     }
     sums[part][threadIdx.x % LANES] = sum;

@@ -477,9 +477,9 @@ __global__ void __launch_bounds__(DIM / 4) latent_rows_merge_kernel(RowsArgs a) 
             // (past the last run: its numbers again, which may be none that zero silences)
             const bool real = c0 + i < a.chunks;
             const float weight = __builtin_amdgcn_exp2f((tops[i] - top) * LOG2E);
-            sum += real ? sums[i] * weight : 0.0f;
+            sum = real ? fmaf(sums[i], weight, sum) : sum;
             #pragma unroll
-            for (int j = 0; j < 4; ++j) x[j] += real ? values[i][j] * weight : 0.0f;
+            for (int j = 0; j < 4; ++j) x[j] = real ? fmaf(values[i][j], weight, x[j]) : x[j];
         }
     }
     x *= 1.0f / sum;
