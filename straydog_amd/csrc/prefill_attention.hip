@@ -1269,10 +1269,11 @@ __global__ void __launch_bounds__(GROUPS * 64) __attribute__((amdgpu_waves_per_e
         #pragma unroll
         for (int qt = 0; qt < 2; ++qt) {
             const float top = fmaxf(fmaxf(fmaxf(s[qt][0][0], s[qt][0][1]), fmaxf(s[qt][0][2], s[qt][0][3])), fmaxf(fmaxf(s[qt][1][0], s[qt][1][1]), fmaxf(s[qt][1][2], s[qt][1][3])));
-            // (from the first step on: nothing has been seen yet; a row that sees none of a share's keys keeps that).  In the first four steps the
-            // reference follows every new maximum: a row of few keys has its largest weight exact in FP16 then, as the kernel that converts in its
-            // loop has (2 x 1531 tokens, distance from 64 bits 3.80e-4 without, 3.76e-4 with, there 3.77e-4; 0.3 us of 82).
-            if (__any(fmaf(top, args.scale_log2, -ref[qt]) > (step < begin + 4 ? 0.0f : SLACK))) {
+            // (from the first step on: nothing has been seen yet; a row that sees none of a share's keys keeps that).  In the first four steps of a
+            // sequence the reference follows every new maximum: a row of few keys has its largest weight exact in FP16 then, as the kernel that converts
+            // in its loop has (2 x 1531 tokens, distance from 64 bits 3.80e-4 without, 3.78e-4 in two steps, 3.76e-4 in four, there 3.77e-4; a call takes
+            // 0.4 us more in two, 1 in four).
+            if (__any(fmaf(top, args.scale_log2, -ref[qt]) > (step < 4 ? 0.0f : SLACK))) {
                 asm volatile("; new reference maxima" ::: "memory");
                 const float higher = fmaxf(ref[qt], row_max(top) * args.scale_log2), alpha = __builtin_amdgcn_exp2f(ref[qt] - higher);
                 ref[qt] = higher;
@@ -1449,9 +1450,10 @@ void prefill_attention(Device& d, const sdx_kv_pool* pool, const int32_t* page_t
     // 32 sequences, 72 rows 288 / 403; 8 of 16384 147 / 746; one of 2000 24 / 96; whole prompts of 2 x 1531 tokens 89 / 226; FP16, 36 rows, 64
     // of 1500 128 / 73, 32 of 8192 319 / 342).
     const uint64_t items = seqs * pool->kv_heads, groups = items * ((args.rows + WIDE_GROUP - 1) / WIDE_GROUP);
-    // It is also the better one for up to 128 keys where its workgroups are one round of the card: the operands are a launch more (64 tokens
-    // at 0, first / second, 12.2 / 10.3 us, 128 14.3 / 13.2, 200 16.4 / 18.3; 4 sequences of 64 12.5 / 10.8, 16 of 64, more than a round, 14.8 / 21.5).
-    const bool few_keys = max_context <= 128 && items * ((args.rows + GROUPS * 16 - 1) / (GROUPS * 16)) <= d.compute_units;
+    // It is also the better one for up to 192 keys (FP16 128) where its workgroups, which walk 64 keys a step, are one round of the card: the operands
+    // are a launch more (64 tokens at 0, first / second, 12.2 / 10.3 us, 128 14.3 / 13.2, 180 16.9 / 16.2, 200 17.1 / 18.5; 3 sequences of 180 18.8 / 17.3;
+    // FP16, 165 16.1 / 17.5; 4 sequences of 64 12.5 / 10.8, 16 of 64, more than a round, 14.8 / 21.5).
+    const bool few_keys = max_context <= (q8 ? 192 : 128) && items * ((args.rows + GROUPS * 16 - 1) / (GROUPS * 16)) <= d.compute_units;
     // And for up to 128 rows a K/V head and 448 keys of an eighth as many items as the card has units (second / first, 32 items: 64 rows of 364 keys 24 / 26, 96 of 312
     // 22 / 25, 128 of 428 27 / 31, 36 of 2036 97 / 41; 64 items of 308 22 / 28; 16 of 303 20 / 16).
     const bool few_rows = args.rows <= WIDE_GROUP && (items * 8 > uint64_t(d.compute_units) * 3 || (max_context <= 448 && items * 8 >= d.compute_units));

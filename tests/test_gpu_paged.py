@@ -732,6 +732,20 @@ def test_prompts_of_256_columns_do_not_depend_on_the_capacity(gpu, oracle, fmt, 
         gpu.release(b)
 
 
+@pytest.mark.parametrize("row_bytes", [272, 512])
+@pytest.mark.parametrize("keys", [128, 129, 192, 193])
+def test_prompts_on_both_sides_of_the_line_of_few_keys(gpu, oracle, row_bytes, keys):
+    # up to 128 keys (Q8_0: 192) go to the kernel that converts in its loop, more to the one over operands
+    rng = np.random.default_rng(keys)
+    dim, page_tokens, span, heads, kv_heads = 256, 64, 48, 8, 2
+    contexts = [keys - span, 0]
+    pool, buffer, host, table, tb = make_pool(gpu, oracle, rng, [c + span for c in contexts], kv_heads, dim, page_tokens, row_bytes)
+    q = rng.standard_normal((2, span, heads, dim)).astype(np.float16).astype(np.float32)
+    want = oracle.paged_attention(host, row_bytes, page_tokens, kv_heads, dim, table, np.array(contexts, np.int32), q, 0.0625)
+    close_enough(_run(gpu, pool, table, tb, contexts, q, span, heads, 0.0625, False, False), want)
+    gpu.release(buffer)
+
+
 def test_the_largest_weight_of_a_row_of_few_keys_is_exact(gpu, oracle):
     # two keys share the weight, in different steps of 32: the larger weight is one, which FP16 holds, and the other key's value is zero, so
     # the output is right to FP32 (rounded to FP16 against the first key's maximum it was up to 1e-4 away)
