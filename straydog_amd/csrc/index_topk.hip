@@ -431,11 +431,13 @@ __device__ __forceinline__ bool top_k_by_bound(ChoiceShared& sh, const uint32_t 
     for (int i = 1; i < KEYS; ++i) own[0] = max(own[0], keys[i]);
     const uint32_t bound = bound_by_maxima(sh, own, floor, uint32_t(k));
     if (!bound) return false;
+    unsigned t = threadIdx.x;
+    asm volatile("" : "+v"(t));                             // (places are formed again: kept from the loads on, 32 keys a thread spilled 28 registers)
     #pragma unroll
     for (int i = 0; i < KEYS; ++i)
         if (keys[i] >= bound) {
             const uint32_t at = atomicAdd(&sh.listed, 1u);
-            if (at < unsigned(CHOICE_LIST)) sh.list[at] = make_uint2(keys[i], i * TOPK_THREADS + threadIdx.x);
+            if (at < unsigned(CHOICE_LIST)) sh.list[at] = make_uint2(keys[i], i * TOPK_THREADS + t);
         }
     __syncthreads();
     const unsigned n = sh.listed;
@@ -446,7 +448,7 @@ __device__ __forceinline__ bool top_k_by_bound(ChoiceShared& sh, const uint32_t 
 // leaves few of them; else three passes of 11, 11 and 10 bits (the first digit takes in two bits of the mantissa: scores of one order of magnitude then meet
 // in a few bins instead of one, where their additions wait for each other), the ordered pass a ballot for each 64 neighbouring places and one scan over their
 // counts.  Bound by one workgroup's latency and instructions.  Measured (the call), by the passes over memory above / these / the bound: a row of 16250 normal
-// scores 35 / 13.4 / 8.4 us, of rectified ones - / 24 / 9; 32768 64 / 22 / 18.4; 1024 rows of 16250 - / 62 / 43; equal scores (no bound) one row of 16250 - / 51 / 52.
+// scores 35 / 13.4 / 8.4 us, of rectified ones - / 24 / 9; 32768 64 / 22 / 12.3 (256 such rows - / 23.3 / 14.0); 1024 rows of 16250 - / 62 / 43; equal scores (no bound) one row of 16250 - / 51 / 52.
 template<int KEYS, class Score, class Index>
 __device__ void top_k_held_row(Score score, Index index, size_t places, size_t k, int32_t* out) {
     constexpr int BINS = 2048, RUNS = KEYS * TOPK_WAVES;
@@ -506,13 +508,15 @@ __device__ void top_k_held_row(Score score, Index index, size_t places, size_t k
     const uint32_t ties_before = block_scan(t < RUNS ? run_ties[t] : 0u, wave_sums, all_ties);
     if (t < RUNS) { run_greater[t] = greater_before; run_ties[t] = ties_before; }
     __syncthreads();
+    unsigned again = t;
+    asm volatile("" : "+v"(again));
     #pragma unroll
     for (int i = 0; i < KEYS; ++i) {
         const bool greater = keys[i] > threshold, tie = !all && keys[i] == threshold;
         const uint64_t below = (uint64_t(1) << lane) - 1;
         const uint32_t ties = run_ties[i * TOPK_WAVES + wave] + __popcll(__ballot(tie) & below);
         const uint32_t slot = run_greater[i * TOPK_WAVES + wave] + __popcll(__ballot(greater) & below) + min(ties, need);
-        if (greater || (tie && ties < need)) out[slot] = index(t + size_t(i) * TOPK_THREADS);
+        if (greater || (tie && ties < need)) out[slot] = index(again + size_t(i) * TOPK_THREADS);
     }
     for (size_t i = kept + min(all_ties, need) + t; i < k; i += TOPK_THREADS) out[i] = -1;
 }

@@ -44,3 +44,19 @@ def make_pool(gpu, oracle, rng, lengths, kv_heads, dim, page_tokens, row_bytes, 
     gpu.write_buffer(buffer, 0, host)
     table_buffer = gpu.upload(table)
     return pool, buffer, host, table, table_buffer
+
+
+def call_us(gpu, call, calls=40):
+    """What a queued call takes, in us: the best of five averages."""
+    call()
+    gpu.synchronize()
+    taken = []
+    for _ in range(5):
+        begin = gpu.event()
+        for _ in range(calls):
+            call()
+        end = gpu.event()
+        gpu.synchronize()
+        taken.append(gpu.elapsed_ms(begin, end) * 1e3 / calls)
+    gpu.events_clear()
+    return min(taken)

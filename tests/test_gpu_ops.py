@@ -7,7 +7,7 @@ CPU oracle."""
 import numpy as np
 import pytest
 
-from gpu_util import backend, close_enough
+from gpu_util import backend, call_us, close_enough
 from test_oracle_attention import SHAPES, _attention_gpu_case
 from test_oracle_index_topk import Random, _adversarial
 
@@ -781,6 +781,19 @@ def test_top_k_by_the_threads_highest(gpu, oracle, kind, places, k):
     gpu.top_k(sb.base(), 2, places, k, ob.base())
     assert np.array_equal(_read(gpu, ob, np.int32, 2 * k).reshape(2, k), oracle.top_k(scores, k))
     gpu.release(sb); gpu.release(ob)
+
+
+def _top_k_us(gpu, scores, k):
+    sb, ob = gpu.upload(scores), gpu.buffer(scores.shape[0] * k * 4)
+    taken = call_us(gpu, lambda: gpu.top_k(sb.base(), scores.shape[0], scores.shape[1], k, ob.base()))
+    gpu.release(sb); gpu.release(ob)
+    return taken
+
+
+def test_top_k_of_twice_the_places_takes_no_more_than_twice_the_time(gpu):
+    # 256 rows, a compute unit each: 16384 places are sixteen keys a thread, 32768 thirty-two, which the registers have to hold
+    scores = np.random.default_rng(5).standard_normal((256, 32768)).astype(np.float32)
+    assert _top_k_us(gpu, scores, 512) <= 2.0 * _top_k_us(gpu, np.ascontiguousarray(scores[:, :16384]), 512)
 
 
 @pytest.mark.parametrize("rows,heads,kv_heads,dim,context,odd", [(65, 24, 2, 256, 333, False), (9, 16, 1, 256, 4000, False), (130, 16, 2, 256, 300, True), (128, 16, 4, 256, 1, False),
