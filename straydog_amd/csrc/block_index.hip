@@ -18,7 +18,7 @@
 // one ordered pass whose slots come from 64-wide ballots and a scan over (run, wave) counts.
 #include "kernels.hpp"
 #include "kv_codec.hpp"
-#include "list_choice.hpp"
+#include "bound_choice.hpp"
 #include "tree_sum.hpp"
 
 using namespace sd;
@@ -240,7 +240,7 @@ __global__ void __launch_bounds__(TILE_THREADS) scores_tiled_kernel(const float*
 }
 
 // ---- the selection ----------------------------------------------------------------------------------------------------------
-constexpr int SELECT_THREADS = CHOICE_THREADS, SELECT_WAVES = CHOICE_WAVES;
+constexpr int SELECT_THREADS = CHOICE_THREADS, SELECT_WAVES = CHOICE_WAVES, LDS_RUNS = 31, LIST_RUNS = 2, LIST = LIST_RUNS * SELECT_THREADS, SIXTEENS_MOST = 1024;
 
 // Exclusive prefix of `value` over the workgroup in thread order, and the workgroup's sum.
 __device__ __forceinline__ uint32_t group_scan(uint32_t value, uint32_t* wave_sums, uint32_t& total) {
@@ -265,9 +265,12 @@ struct SelectShared {
     union {
         struct {
             uint32_t bins[SELECT_WAVES * 256];              // a histogram per wave; at other times the (run, wave) counts or the sample's histogram
-            uint2 list[CHOICE_LIST];                        // (score bits, block) of the values that reach the guess
+            uint2 list[LIST_RUNS * SELECT_THREADS];         // (score bits, block) of the values that reach the guess
         };
-        ChoiceShared choice;
+        struct {
+            ChoiceShared choice;
+            uint32_t names[SIXTEENS_MOST];                  // of the sixteens that reach the bound
+        };
     };
     uint32_t wave_sums[SELECT_WAVES], threshold, remaining;
 };
@@ -355,26 +358,22 @@ __device__ __forceinline__ void choose_blocks(SelectShared& sh, Each each_run, B
 // scores, and little more (some 550 of 60K in no order), so it is a bound that only its own sixteens have to be read for.  Writes the row's entries; false, and
 // nothing written: too many reach the bound (many scores are equal), the row's workgroup sweeps the row itself.  (Thirty-two workgroups a row that each found
 // a bound from the same sample of it and listed their stretch took a launch of 10 us; a decode row's whole stage at 242K tokens 52.4 us with them, 38.7 now.)
-constexpr int SIXTEENS_MOST = CHOICE_MEMBERS, MAXIMA_EACH = (65536 / SIXTEENS + SELECT_THREADS) / SELECT_THREADS;
-__device__ __forceinline__ bool select_by_maxima(ChoiceShared& sh, const uint32_t (&top)[MAXIMA_EACH], const float* row, uint32_t complete, float* out) {
+constexpr int MAXIMA_EACH = (65536 / SIXTEENS + SELECT_THREADS) / SELECT_THREADS;
+__device__ __forceinline__ bool select_by_maxima(SelectShared& sh, const uint32_t (&top)[MAXIMA_EACH], const float* row, uint32_t complete, float* out) {
     const unsigned t = threadIdx.x, count = (complete + SIXTEENS - 1) / SIXTEENS;
     constexpr uint32_t NONE = 0xffffffffu;                  // (no score's bits)
     uint32_t valid[MAXIMA_EACH];
     #pragma unroll
     for (int i = 0; i < MAXIMA_EACH; ++i) valid[i] = i * SELECT_THREADS + t < count ? top[i] : NONE;
-    const uint32_t bound = bound_by_maxima(sh, valid, NONE, KEEP);
+    uint32_t high;
+    const uint32_t bound = bound_by_maxima(sh.choice, valid, NONE, KEEP, SIXTEENS_MOST, high);
     if (!bound) return false;
-    // the sixteens that reach it are named (in the room of the list's second half), then their scores that do are listed
-    uint32_t* const names = reinterpret_cast<uint32_t*>(sh.list + CHOICE_LIST / 2);
+    // the sixteens that reach it are named, then their scores that do are listed
     #pragma unroll
     for (int i = 0; i < MAXIMA_EACH; ++i)
-        if (valid[i] != NONE && valid[i] >= bound) {
-            const uint32_t at = atomicAdd(&sh.in_bin, 1u);
-            if (at < unsigned(SIXTEENS_MOST)) names[at] = i * SELECT_THREADS + t;
-        }
+        if (valid[i] != NONE && valid[i] >= bound) sh.names[atomicAdd(&sh.choice.named, 1u)] = i * SELECT_THREADS + t;
     __syncthreads();
-    const unsigned named = sh.in_bin;
-    if (named > unsigned(SIXTEENS_MOST)) return false;
+    const unsigned named = sh.choice.named;
     constexpr int AT_ONCE = 4;                              // reads in flight
     #pragma unroll 1
     for (unsigned base = 0; base < named; base += AT_ONCE * (SELECT_THREADS / SIXTEENS)) {
@@ -382,24 +381,26 @@ __device__ __forceinline__ bool select_by_maxima(ChoiceShared& sh, const uint32_
         #pragma unroll
         for (int i = 0; i < AT_ONCE; ++i) {
             const unsigned name = base + i * (SELECT_THREADS / SIXTEENS) + t / SIXTEENS;
-            block[i] = name < named ? names[name] * SIXTEENS + t % SIXTEENS : complete;
+            block[i] = name < named ? sh.names[name] * SIXTEENS + t % SIXTEENS : complete;
             bits[i] = __float_as_uint(row[min(block[i], complete - 1)]);
         }
         #pragma unroll
         for (int i = 0; i < AT_ONCE; ++i)
             if (block[i] < complete && bits[i] >= bound) {
-                const uint32_t at = atomicAdd(&sh.listed, 1u);
-                if (at < unsigned(CHOICE_LIST) / 2) sh.list[at] = make_uint2(bits[i], block[i]);
+                const uint32_t at = atomicAdd(&sh.choice.listed, 1u);
+                if (at < unsigned(CHOICE_LIST)) sh.choice.list[at] = make_uint2(bits[i], block[i]);
             }
     }
     __syncthreads();
-    const unsigned n = sh.listed;
-    if (n > unsigned(CHOICE_LIST) / 2) return false;
-    if (t == 0) sh.in_bin = 0u;                             // (the next barrier is the choice's first)
-    return choose_listed(sh, n, KEEP, [&](size_t slot, uint32_t block) {
+    const auto emit = [&](size_t slot, uint32_t block) {
         #pragma unroll
         for (size_t tap = 0; tap < 4; ++tap) out[slot * 4 + tap] = float(size_t(block) * 4 + tap);
-    });
+    };
+    const unsigned n = sh.choice.listed;
+    if (n > unsigned(CHOICE_LIST)) return false;
+    const uint2 own = sh.choice.list[t];
+    choose(sh.choice, KEEP, bound, high, [&](auto use) { if (t < n) use(own.x, own.y); }, emit);
+    return true;
 }
 
 // One workgroup per row; block i * 1024 + t is thread t's value i.  The row is read once and stays on the chip: its first
@@ -410,8 +411,7 @@ __device__ __forceinline__ bool select_by_maxima(ChoiceShared& sh, const uint32_
 // highest of a sample of four values a thread (spread over the runs in LDS; R: one and a half times the sample's share of 512, and
 // a margin), found to 24 bits by two 4096-bin histograms, is a guess below the 512th highest value of the row.  Two light sweeps count and list, in block order, the values that reach the guess; when they are
 // at least 512 and fit the list, the choice runs over the list alone, otherwise over the whole row.
-constexpr int LDS_RUNS = 31, LIST_RUNS = 2, LIST = LIST_RUNS * SELECT_THREADS;
-static_assert(LIST == CHOICE_LIST && sizeof(SelectShared) + LDS_RUNS * SELECT_THREADS * 4 <= 160 * 1024, "a compute unit's LDS");
+static_assert(sizeof(SelectShared) + LDS_RUNS * SELECT_THREADS * 4 <= 160 * 1024, "a compute unit's LDS");
 template<int REGS>
 __global__ void __launch_bounds__(SELECT_THREADS) select_kernel(const float* __restrict__ scores, size_t pool, size_t base, const uint32_t* dynamic,
                                                                 size_t selected, unsigned held_runs, float* __restrict__ indices,
@@ -446,7 +446,7 @@ __global__ void __launch_bounds__(SELECT_THREADS) select_kernel(const float* __r
     uint32_t list_count = 0;
     bool done = false;
     if (maxima && complete >= size_t(KEEP) * SIXTEENS) {
-        done = select_by_maxima(sh.choice, tops, row, uint32_t(complete), out);
+        done = select_by_maxima(sh, tops, row, uint32_t(complete), out);
         __syncthreads();
     }
     if (!done) {
@@ -474,9 +474,11 @@ __global__ void __launch_bounds__(SELECT_THREADS) select_kernel(const float* __r
         }
         for (; i < lds_runs; ++i) body(i, held[i * SELECT_THREADS + t], size_t(i) * SELECT_THREADS + t < complete);
         if constexpr (REGS > 0) {
+            unsigned again = t;
+            asm volatile("" : "+v"(again));                  // (the runs' places are formed again: kept from the loads on they are more registers than there are)
             #pragma unroll
             for (int j = 0; j < REGS; ++j)
-                if (unsigned(LDS_RUNS + j) < runs) body(unsigned(LDS_RUNS + j), values[j], size_t(LDS_RUNS + j) * SELECT_THREADS + t < complete);
+                if (unsigned(LDS_RUNS + j) < runs) body(unsigned(LDS_RUNS + j), values[j], size_t(LDS_RUNS + j) * SELECT_THREADS + again < complete);
         }
     };
     if (runs >= 8) {
@@ -531,7 +533,9 @@ __global__ void __launch_bounds__(SELECT_THREADS) select_kernel(const float* __r
             each_run([&](unsigned i, uint32_t bits, bool valid) {
                 const bool reaches = valid && bits >= guess;
                 const uint64_t reaching = __ballot(reaches);
-                if (reaches) sh.list[reach[i * SELECT_WAVES + wave] + uint32_t(__popcll(reaching & below))] = make_uint2(bits, i * SELECT_THREADS + t);
+                unsigned again = t;
+                asm volatile("" : "+v"(again));
+                if (reaches) sh.list[reach[i * SELECT_WAVES + wave] + uint32_t(__popcll(reaching & below))] = make_uint2(bits, i * SELECT_THREADS + again);
             });
         }
         __syncthreads();
@@ -547,7 +551,11 @@ __global__ void __launch_bounds__(SELECT_THREADS) select_kernel(const float* __r
                 if (unsigned(j) < list_runs) body(unsigned(j), mine[j].x, unsigned(j) * SELECT_THREADS + t < list_count);
         }, [&](unsigned j) { return size_t(j == 0 ? mine[0].y : mine[1].y); }, list_runs, LIST_RUNS, 0u, out);
     } else {
-        choose_blocks(sh, each_run, [&](unsigned i) { return size_t(i) * SELECT_THREADS + t; }, runs, LDS_RUNS + REGS, guess, out);
+        choose_blocks(sh, each_run, [&](unsigned i) {
+            unsigned again = t;
+            asm volatile("" : "+v"(again));
+            return size_t(i) * SELECT_THREADS + again;
+        }, runs, LDS_RUNS + REGS, guess, out);
     }
     }
     const size_t head = size_t(KEEP) * 4;

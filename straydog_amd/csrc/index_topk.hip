@@ -7,7 +7,7 @@
 // scale is applied last.  Top-k compares order-preserving integer keys, keeps the lowest indices among ties and
 // emits ascending indices.
 #include "device.hpp"
-#include "list_choice.hpp"
+#include "bound_choice.hpp"
 #include <hip/hip_fp16.h>
 #include "../../include/straydog_gpu.h"
 #include "../../include/straydog_gpu_ext.h"
@@ -421,34 +421,12 @@ __device__ void top_k_row(Score score, Index index, size_t places, size_t k, int
     for (size_t i = slot + t; i < k; i += TOPK_THREADS) out[i] = -1;
 }
 
-// (k at most half the threads) The k-th highest of the threads' own highest keys is a bound that k keys reach and little more (of 16250 scores some 700 for
-// k = 512); a key then costs a handful of instructions, where three passes over all of them cost fifty.  False, and nothing written: too few threads have a key,
-// or too many keys reach the bound (equal ones).
-template<int KEYS, class Index>
-__device__ __forceinline__ bool top_k_by_bound(ChoiceShared& sh, const uint32_t (&keys)[KEYS], uint32_t floor, Index index, size_t k, int32_t* out) {
-    uint32_t own[1] = {keys[0]};
-    #pragma unroll
-    for (int i = 1; i < KEYS; ++i) own[0] = max(own[0], keys[i]);
-    const uint32_t bound = bound_by_maxima(sh, own, floor, uint32_t(k));
-    if (!bound) return false;
-    unsigned t = threadIdx.x;
-    asm volatile("" : "+v"(t));                             // (places are formed again: kept from the loads on, 32 keys a thread spilled 28 registers)
-    #pragma unroll
-    for (int i = 0; i < KEYS; ++i)
-        if (keys[i] >= bound) {
-            const uint32_t at = atomicAdd(&sh.listed, 1u);
-            if (at < unsigned(CHOICE_LIST)) sh.list[at] = make_uint2(keys[i], i * TOPK_THREADS + t);
-        }
-    __syncthreads();
-    const unsigned n = sh.listed;
-    return n <= unsigned(CHOICE_LIST) && choose_listed(sh, n, uint32_t(k), [&](size_t slot, uint32_t place) { out[slot] = index(size_t(place)); });
-}
-
 // The same for rows of up to KEYS x 1024 places, which are read once and held: thread t has the places t, t + 1024, ...  By a bound where that
 // leaves few of them; else three passes of 11, 11 and 10 bits (the first digit takes in two bits of the mantissa: scores of one order of magnitude then meet
 // in a few bins instead of one, where their additions wait for each other), the ordered pass a ballot for each 64 neighbouring places and one scan over their
 // counts.  Bound by one workgroup's latency and instructions.  Measured (the call), by the passes over memory above / these / the bound: a row of 16250 normal
-// scores 35 / 13.4 / 8.4 us, of rectified ones - / 24 / 9; 32768 64 / 22 / 12.3 (256 such rows - / 23.3 / 14.0); 1024 rows of 16250 - / 62 / 43; equal scores (no bound) one row of 16250 - / 51 / 52.
+// scores 35 / 13.4 / 8.4 us, the same with an infinity among them, with nine tenths of them zeros, with all of them equal - / 13.3, 24, 51 / 8.4, 8.7, 8.0; 4096 - / 8.1 / 5.7;
+// 32768 64 / 22 / 13; 256 rows of 4096, 16250, 32768 - / 8.5, 16.2, 23.2 / 6.2, 11.1, 14.8.
 template<int KEYS, class Score, class Index>
 __device__ void top_k_held_row(Score score, Index index, size_t places, size_t k, int32_t* out) {
     constexpr int BINS = 2048, RUNS = KEYS * TOPK_WAVES;
@@ -465,15 +443,40 @@ __device__ void top_k_held_row(Score score, Index index, size_t places, size_t k
         keys[i] = place < places ? max(top_k_key(score(place)), floor) : floor;       // (what lies below minus infinity does not count either)
     }
     __shared__ ChoiceShared sh;
-    if (k <= TOPK_THREADS / 2 && places >= 2 * TOPK_THREADS) {
-        if (top_k_by_bound<KEYS>(sh, keys, floor, index, k, out)) return;
-        __syncthreads();
-    }
     uint32_t* const bins = sh.bins;
     uint32_t prefix = 0, rank = uint32_t(k);
-    bool all = false;
+    bool all = false, found = false;
+    // (The k-th highest of the threads' own highest keys is a bound that k keys reach and little more: of 16250 scores some 700 for k = 512.)
+    if (k <= TOPK_THREADS / 2 && places >= 2 * TOPK_THREADS) {
+        uint32_t own[1] = {keys[0]}, high;
+        #pragma unroll
+        for (int i = 1; i < KEYS; ++i) own[0] = max(own[0], keys[i]);
+        const uint32_t bound = bound_by_maxima(sh, own, floor, rank, TOPK_THREADS / 8 * 7, high);
+        const auto reaching = [&](auto use) {
+            unsigned again = t;
+            asm volatile("" : "+v"(again));                  // (places are formed again: kept from the loads on they are more registers than there are)
+            #pragma unroll
+            for (int i = 0; i < KEYS; ++i)
+                if (keys[i] >= bound) use(keys[i], i * TOPK_THREADS + again);
+        };
+        if (bound) {
+            choose(sh, rank, bound, high, reaching, [&](size_t slot, uint32_t place) { out[slot] = index(size_t(place)); });
+            return;
+        }
+        if (high) {                                   // as a rule it is the k-th highest key itself
+            uint32_t mine = 0, ties;
+            #pragma unroll
+            for (int i = 0; i < KEYS; ++i) mine += (keys[i] > high) + (keys[i] == high ? 1u << 16 : 0u);
+            block_scan(mine, wave_sums, ties);               // (at most 32768 of each)
+            const uint32_t more = ties & 0xffffu;
+            found = more < k && more + (ties >> 16) >= k;
+            if (found) { prefix = high; rank = uint32_t(k) - more; }
+        }
+        __syncthreads();
+    }
     #pragma unroll
     for (int level = 0; level < 3; ++level) {
+        if (found) break;
         const int shift = level == 0 ? 21 : level == 1 ? 10 : 0, above_digit = level == 1 ? 21 : 10;
         const uint32_t digits = level == 2 ? 1023u : 2047u;
         bins[t] = 0; bins[t + TOPK_THREADS] = 0;

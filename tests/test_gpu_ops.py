@@ -783,6 +783,45 @@ def test_top_k_by_the_threads_highest(gpu, oracle, kind, places, k):
     gpu.release(sb); gpu.release(ob)
 
 
+def _far_from_normal(kind, rng, rows, places):
+    s = rng.standard_normal((rows, places)).astype(np.float32)
+    thread, run = np.arange(places) % 1024, np.arange(places) // 1024
+    if kind == "infinity":
+        s[:, rng.integers(0, places)] = np.inf
+    if kind == "infinities":
+        s[:, rng.permutation(places)[:40]] = np.inf
+    if kind == "far":
+        s[:, rng.permutation(places)[:60]] *= 1e30
+    if kind == "lowest":                        # masked by the type's lowest value, not by -inf
+        s[:, rng.permutation(places)[:places * 2 // 5]] = np.finfo(np.float32).min
+    if kind == "equal":
+        s[:] = -3.0
+    if kind == "zeros":
+        s[rng.random(s.shape) < 0.95] = 0.0
+    if kind == "few threads":                   # the highest with a tenth of the threads
+        s[:, thread < 100] += 8.0
+    if kind == "equal highest":                 # more of the same than a bin's values are ranked among one another
+        s[:, thread < 60] = 9.0
+    if kind == "equal below":                   # nearly every thread's highest is the same, and more than k lie above it
+        s[:] = np.minimum(s, 0.5)
+        s[:, run == 0] = 0.5
+        s[:, (thread < 100) & (run < 12)] = 7.0 + rng.standard_normal(((thread < 100) & (run < 12)).sum())
+    if kind == "steps":
+        s = np.round(s * 16) / 16
+    return s.astype(np.float32)
+
+
+@pytest.mark.parametrize("kind", ["infinity", "infinities", "far", "lowest", "equal", "zeros", "few threads", "equal highest", "equal below", "steps"])
+@pytest.mark.parametrize("places,k", [(2048, 512), (4099, 100), (16384, 64), (16385, 512), (32768, 512)])
+def test_top_k_of_scores_far_from_normal(gpu, oracle, kind, places, k):
+    # the bins that a bound and the cut are found by: values that leave the others in one, more equal ones than are ranked, more than reach the bound as a rule
+    scores = _far_from_normal(kind, np.random.default_rng(places + k), 3, places)
+    sb, ob = gpu.upload(scores), gpu.buffer(3 * k * 4)
+    gpu.top_k(sb.base(), 3, places, k, ob.base())
+    assert np.array_equal(_read(gpu, ob, np.int32, 3 * k).reshape(3, k), oracle.top_k(scores, k))
+    gpu.release(sb); gpu.release(ob)
+
+
 def _top_k_us(gpu, scores, k):
     sb, ob = gpu.upload(scores), gpu.buffer(scores.shape[0] * k * 4)
     taken = call_us(gpu, lambda: gpu.top_k(sb.base(), scores.shape[0], scores.shape[1], k, ob.base()))
@@ -794,6 +833,16 @@ def test_top_k_of_twice_the_places_takes_no_more_than_twice_the_time(gpu):
     # 256 rows, a compute unit each: 16384 places are sixteen keys a thread, 32768 thirty-two, which the registers have to hold
     scores = np.random.default_rng(5).standard_normal((256, 32768)).astype(np.float32)
     assert _top_k_us(gpu, scores, 512) <= 2.0 * _top_k_us(gpu, np.ascontiguousarray(scores[:, :16384]), 512)
+
+
+@pytest.mark.parametrize("kind", ["infinity", "far", "equal", "zeros", "equal highest"])
+@pytest.mark.parametrize("rows,places", [(1, 4096), (256, 4096), (1, 16250)])
+def test_top_k_takes_as_long_whatever_the_scores(gpu, kind, rows, places):
+    # (the passes over all digits take 1.4 to three times as long, over equal scores six; hundreds of equal ones ranked among one
+    # another eleven: by their bits 2.4)
+    rng = np.random.default_rng(places)
+    normal = _top_k_us(gpu, rng.standard_normal((rows, places)).astype(np.float32), 512)
+    assert _top_k_us(gpu, _far_from_normal(kind, rng, rows, places), 512) <= (3.0 if kind == "equal highest" else 1.7) * normal
 
 
 @pytest.mark.parametrize("rows,heads,kv_heads,dim,context,odd", [(65, 24, 2, 256, 333, False), (9, 16, 1, 256, 4000, False), (130, 16, 2, 256, 300, True), (128, 16, 4, 256, 1, False),
