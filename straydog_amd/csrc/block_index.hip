@@ -355,8 +355,9 @@ __device__ __forceinline__ void choose_blocks(SelectShared& sh, Each each_run, B
 
 // A short span's rows (a decode step, a verification span) would leave all but a few compute units idle while one workgroup a row
 // sweeps 60K values.  Their scores' kernel leaves the highest score of each sixteen neighbouring blocks: the 512th highest of those is reached by 512
-// scores, and little more (some 550 of 60K in no order), so it is a bound that only its own sixteens have to be read for.  Writes the row's entries; false, and
-// nothing written: too many reach the bound (many scores are equal), the row's workgroup sweeps the row itself.  (Thirty-two workgroups a row that each found
+// scores, and little more (some 550 of 60K in no order), so it is a bound that only its own sixteens have to be read for.  Where neighbours are alike whole sixteens reach it, up to 16K scores: more
+// than the list holds, they are read again for each step of the choice (a row of 32768 blocks alike over sixteen 17.5 us; swept, with the attempt, 38; not alike 12.9).
+// Writes the row's entries; false, and nothing written: many scores are equal, the row's workgroup sweeps the row itself.  (Thirty-two workgroups a row that each found
 // a bound from the same sample of it and listed their stretch took a launch of 10 us; a decode row's whole stage at 242K tokens 52.4 us with them, 38.7 now.)
 constexpr int MAXIMA_EACH = (65536 / SIXTEENS + SELECT_THREADS) / SELECT_THREADS;
 __device__ __forceinline__ bool select_by_maxima(SelectShared& sh, const uint32_t (&top)[MAXIMA_EACH], const float* row, uint32_t complete, float* out) {
@@ -374,30 +375,37 @@ __device__ __forceinline__ bool select_by_maxima(SelectShared& sh, const uint32_
         if (valid[i] != NONE && valid[i] >= bound) sh.names[atomicAdd(&sh.choice.named, 1u)] = i * SELECT_THREADS + t;
     __syncthreads();
     const unsigned named = sh.choice.named;
-    constexpr int AT_ONCE = 4;                              // reads in flight
-    #pragma unroll 1
-    for (unsigned base = 0; base < named; base += AT_ONCE * (SELECT_THREADS / SIXTEENS)) {
-        uint32_t block[AT_ONCE], bits[AT_ONCE];
-        #pragma unroll
-        for (int i = 0; i < AT_ONCE; ++i) {
-            const unsigned name = base + i * (SELECT_THREADS / SIXTEENS) + t / SIXTEENS;
-            block[i] = name < named ? sh.names[name] * SIXTEENS + t % SIXTEENS : complete;
-            bits[i] = __float_as_uint(row[min(block[i], complete - 1)]);
-        }
-        #pragma unroll
-        for (int i = 0; i < AT_ONCE; ++i)
-            if (block[i] < complete && bits[i] >= bound) {
-                const uint32_t at = atomicAdd(&sh.choice.listed, 1u);
-                if (at < unsigned(CHOICE_LIST)) sh.choice.list[at] = make_uint2(bits[i], block[i]);
+    const auto read = [&](auto enough, auto use) {
+        constexpr int AT_ONCE = 4;                          // reads in flight
+        #pragma unroll 1
+        for (unsigned base = 0; base < named && !enough(); base += AT_ONCE * (SELECT_THREADS / SIXTEENS)) {
+            uint32_t block[AT_ONCE], bits[AT_ONCE];
+            #pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i) {
+                const unsigned name = base + i * (SELECT_THREADS / SIXTEENS) + t / SIXTEENS;
+                block[i] = name < named ? sh.names[name] * SIXTEENS + t % SIXTEENS : complete;
+                bits[i] = __float_as_uint(row[min(block[i], complete - 1)]);
             }
-    }
+            #pragma unroll
+            for (int i = 0; i < AT_ONCE; ++i)
+                if (block[i] < complete && bits[i] >= bound) use(bits[i], block[i]);
+        }
+    };
+    // (neighbours that are alike: most of what was named, which the list does not hold; a wave that sees it full adds no more)
+    read([&] { return *const_cast<volatile uint32_t*>(&sh.choice.listed) > unsigned(CHOICE_LIST); }, [&](uint32_t value, uint32_t name) {
+        const uint32_t at = atomicAdd(&sh.choice.listed, 1u);
+        if (at < unsigned(CHOICE_LIST)) sh.choice.list[at] = make_uint2(value, name);
+    });
     __syncthreads();
     const auto emit = [&](size_t slot, uint32_t block) {
         #pragma unroll
         for (size_t tap = 0; tap < 4; ++tap) out[slot * 4 + tap] = float(size_t(block) * 4 + tap);
     };
     const unsigned n = sh.choice.listed;
-    if (n > unsigned(CHOICE_LIST)) return false;
+    if (n > unsigned(CHOICE_LIST)) {
+        choose(sh.choice, KEEP, bound, high, [&](auto use) { read([] { return false; }, use); }, emit);
+        return true;
+    }
     const uint2 own = sh.choice.list[t];
     choose(sh.choice, KEEP, bound, high, [&](auto use) { if (t < n) use(own.x, own.y); }, emit);
     return true;

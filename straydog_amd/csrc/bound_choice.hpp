@@ -103,8 +103,8 @@ __device__ __forceinline__ bool range_refine(ChoiceShared& sh, uint32_t* bins, R
 
 // A bound by values that each are the highest of their own share of all: thread t's count of them (those that are not `none`).  The k-th highest of them, to
 // a bin of their range, rounded down, that no more than `most` of them reach; high: where the values that reach it are to be spread to.  0: there are fewer than k (high: 0), or
-// too many are equal (high: to what).  The range goes to the highest that four neighbouring waves all reach: an infinity, or a few scores far above the others, would leave those in a
-// handful of bins, whose additions wait for each other (a row of 4096 with an infinity 13.9 us, without 5.8; the passes alone 8.1).
+// too many are equal (high: to what).  The range ends at four times as far up as the highest that four neighbouring waves all reach: an infinity, or a few scores far above the others, would leave
+// those in a handful of bins, whose additions wait for each other (a row of 4096 with an infinity 13.9 us, without 5.8; the passes alone 8.1).
 template<int COUNT>
 __device__ __forceinline__ uint32_t bound_by_maxima(ChoiceShared& sh, const uint32_t (&top)[COUNT], uint32_t none, uint32_t k, uint32_t most, uint32_t& high) {
     uint32_t lowest = 0xffffffffu, highest = 0u;
@@ -122,7 +122,7 @@ __device__ __forceinline__ uint32_t bound_by_maxima(ChoiceShared& sh, const uint
     high = min(high, from_lane<LANE_XOR_1>(0u, high));
     high = min(high, from_lane<LANE_XOR_2>(0u, high));
     high = wave_most(high);
-    if (high <= lowest) high = highest;                     // (waves without a value)
+    high = high > lowest && high - lowest < (highest - lowest) / 4 ? high + 3 * (high - lowest) : highest;       // (0: waves without a value)
     Range range(lowest, high, highest);
     values([&](uint32_t value, uint32_t) { atomicAdd(&sh.bound_bins[range.bin(value)], 1u); });
     __syncthreads();

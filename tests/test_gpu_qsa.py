@@ -7,7 +7,7 @@ the blocks, in the order and with the ties, of the exact rule, and the block sco
 import numpy as np
 import pytest
 
-from gpu_util import backend
+from gpu_util import backend, call_us
 
 pytestmark = pytest.mark.gpu
 
@@ -113,6 +113,39 @@ def test_block_scores_and_selection(gpu, oracle, mode, base, steps, context, str
     selected = min(base + steps, 2052)
     queries, blocks = _case(oracle, mode, base, steps, pool, stride, seed=base + steps)
     _check(oracle, queries, blocks, base, selected, _run_index(gpu, queries, blocks, base, selected))
+
+
+def _alike(rng, pool, length, loud=0):
+    """Keys that are alike over `length` neighbouring blocks; the first `loud` are far from the others."""
+    noise = np.cumsum(rng.standard_normal((128, pool + length)), axis=1)
+    blocks = ((noise[:, length:] - noise[:, :pool]) / np.sqrt(length)).astype(np.float32)
+    blocks[:, :loud] *= 1e4
+    return blocks
+
+
+@pytest.mark.parametrize("length,loud,base,steps", [(16, 0, 40000, 3), (64, 0, 100001, 1), (300, 0, 240000, 8), (4, 0, 32767, 2), (16, 3, 66000, 4), (1, 700, 131070, 5),
+                                                    (1, 0, 4 * 8192 - 1, 1), (2000, 0, 36000, 2)])
+def test_selection_of_blocks_that_are_alike(gpu, oracle, length, loud, base, steps):
+    # more blocks reach the bound than its list holds, or a few lie far above all others
+    rng = np.random.default_rng(base)
+    pool = (base + steps) // 4 + 1
+    queries, blocks = rng.standard_normal((steps, 512)).astype(np.float32), _alike(rng, pool, length, loud)
+    _check(oracle, queries, blocks, base, 2052, _run_index(gpu, queries, blocks, base, 2052))
+
+
+def test_selection_takes_about_as_long_where_neighbours_are_alike(gpu):
+    rng = np.random.default_rng(3)
+    pool = 32768
+    queries = gpu.upload(rng.standard_normal((1, 512)).astype(np.float32))
+    scores, indices, counts = gpu.buffer(pool * 4), gpu.buffer(2052 * 4), gpu.buffer(16)
+    taken = []
+    for length in (1, 16):
+        blocks = gpu.upload(_alike(rng, pool, length))
+        taken.append(call_us(gpu, lambda: gpu.qsa_index(queries.base(), 512, blocks.base(), pool, 4 * pool - 1, 1, 2052, scores.base(), indices.base(), counts.base())))
+        gpu.release(blocks)
+    for b in (queries, scores, indices, counts):
+        gpu.release(b)
+    assert taken[1] <= 2.0 * taken[0]            # (three times as long where the row is swept after the list has run over)
 
 
 def _run_interval(gpu, queries, blocks, base, selected, state=None):
