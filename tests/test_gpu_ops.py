@@ -952,6 +952,47 @@ def test_dense_attention_of_scores_far_below_zero(gpu, rows, heads, kv_heads, di
         gpu.release(b)
 
 
+@pytest.mark.parametrize("kind", ["values", "subnormal values", "a column", "queries", "keys", "weights"])
+@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(8, 8, 2, 128), (40, 8, 2, 128), (160, 16, 2, 256)])
+def test_dense_attention_of_small_operands(gpu, oracle, rows, heads, kv_heads, dim, kind):
+    # operands near the lower end of FP32's range, times which something that makes up for it: as many bits as of any others
+    rng = np.random.default_rng(rows + dim)
+    context, scale = 200, np.float32(dim ** -0.5)
+    q = rng.standard_normal((rows, heads, dim)).astype(np.float32)
+    keys, values = (rng.standard_normal((context, kv_heads, dim)).astype(np.float32) for _ in range(2))
+    positions = rng.integers(0, context, size=rows).astype(np.int32)
+    positions[:8] = range(8)                    # (the bound grows with the keys)
+    small = np.float32(2.0 ** -122)
+    if kind == "values":
+        values *= small
+    if kind == "subnormal values":
+        values *= np.float32(2.0 ** -139)
+    if kind == "a column":
+        values[..., dim // 2 + 5] *= small
+        values[..., 3] = 0.0
+    if kind == "queries":
+        q, keys = q * small, keys / small
+    if kind == "keys":
+        q, keys = q / small, keys * small
+    if kind == "weights":                       # eight keys that weigh next to nothing, with values to make up for it
+        q[:], keys[:], positions[:], scale = 1.0, 0.0, context - 1, np.float32(1 / 16)
+        keys[40:48] = (-(86 + np.arange(8) / 8) * 16 / dim)[:, None, None]          # (every sum exact)
+        values[..., :8] = 0.0
+        values[range(40, 48), :, range(8)] = np.float32(2.0 ** 100)
+    qs, ks, vs, ps = (gpu.upload(x) for x in (q, keys, values, positions))
+    pairs = rows * heads
+    scratch, out = gpu.buffer(pairs * min(64, max(1, 256 // pairs)) * (dim + 2) * 4), gpu.buffer(q.size * 4)
+    gpu.attention(qs.base(), ks.base(), vs.base(), context, ps.base(), rows, heads, kv_heads, dim, float(scale), None, scratch, out.base())
+    got = _read(gpu, out, np.float32, q.size).reshape(q.shape)
+    want, bound = oracle.op_attention_f64(q, keys, values, positions, float(scale), None)
+    # (a sum of subnormal numbers is a whole number of 2^-149: one rounding a key, and the quotient's)
+    assert (np.abs(got - want) <= bound + (context + 1) * 2.0 ** -149).all()
+    if kind == "weights":                       # (a weight's exponent of 125, rounded three times to 24 bits)
+        assert (np.abs(got - want) <= 3 * 125 * 2.0 ** -24 * np.abs(want))[..., :8].all()
+    for b in (qs, ks, vs, ps, scratch, out):
+        gpu.release(b)
+
+
 def _plain_latent(q, raw, positions, window, table, selected, sinks, scale, pairs, frequencies):
     """Window rows and selected rows as keys and values, a sink, the last columns turned and turned back: sums in 64 bits, weights in FP32
     (those too small for it are zeros), infinities and NaNs as their own arithmetic has them."""
