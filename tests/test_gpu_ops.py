@@ -693,7 +693,8 @@ def test_latent_rows_on_the_matrix_cores(gpu, oracle, rows, heads, window, raw_r
 
 
 @pytest.mark.parametrize("rows,heads,kv_heads,dim,context", [(1, 16, 2, 256, 4200), (1, 4, 4, 128, 33), (2, 16, 1, 128, 1000), (5, 24, 2, 256, 96), (33, 16, 2, 128, 700),
-                                                             (70, 16, 2, 256, 300), (300, 16, 4, 128, 400), (1, 1, 1, 256, 1)])
+                                                             (70, 16, 2, 256, 300), (300, 16, 4, 128, 400), (1, 1, 1, 256, 1),
+                                                             (33, 1, 1, 128, 150), (5, 16, 2, 128, 900), (7, 9, 1, 128, 64), (4, 32, 2, 128, 333), (13, 10, 2, 128, 200)])
 def test_dense_attention_on_the_matrix_cores(gpu, oracle, rows, heads, kv_heads, dim, context):
     # 128 and 256 columns: one and two tiles of 32 query rows, runs of keys merged or one run finished in place, rows that see one key and
     # rows past the cache's end, what lies past every row's position never used; the scratch of the reference's contract, and graphs that
@@ -731,7 +732,8 @@ def test_dense_attention_on_the_matrix_cores(gpu, oracle, rows, heads, kv_heads,
         gpu.release(b)
 
 
-@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(40, 8, 2, 256), (40, 8, 2, 128), (3, 4, 2, 256), (3, 4, 2, 128)])
+@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(40, 8, 2, 256), (40, 8, 2, 128), (3, 4, 2, 256), (3, 4, 2, 128), (11, 6, 2, 128), (8, 16, 2, 128), (13, 10, 2, 128),
+                                                      (160, 16, 2, 256)])
 def test_dense_attention_keeps_to_the_keys_a_row_sees(gpu, oracle, rows, heads, kv_heads, dim):
     # keys and values that are no finite numbers: the rows before them have the results they have without them, the rows that see such a
     # value have no finite number in its column
@@ -893,7 +895,8 @@ def _plain_attention(q, keys, values, positions, scale):
     return out
 
 
-@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(1, 8, 2, 256), (1, 4, 4, 128), (40, 8, 2, 256), (40, 8, 2, 128)])
+@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(1, 8, 2, 256), (1, 4, 4, 128), (40, 8, 2, 256), (40, 8, 2, 128), (5, 16, 2, 128), (8, 8, 1, 128), (5, 13, 1, 128),
+                                                      (160, 16, 2, 256)])
 def test_dense_attention_of_odd_values_has_their_own_sums(gpu, rows, heads, kv_heads, dim):
     # values that are no finite numbers in steps of 32 keys that not every row sees whole: infinities of one sign stay that, of both signs
     # (or any sign and a weight of zero) are a NaN, a NaN stays one, and the other columns are as they were
@@ -931,7 +934,7 @@ def test_dense_attention_of_odd_values_has_their_own_sums(gpu, rows, heads, kv_h
         gpu.release(b)
 
 
-@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(1, 8, 2, 256), (40, 4, 2, 128), (40, 8, 2, 256)])
+@pytest.mark.parametrize("rows,heads,kv_heads,dim", [(1, 8, 2, 256), (40, 4, 2, 128), (40, 8, 2, 256), (33, 2, 2, 128), (9, 7, 1, 128), (13, 5, 1, 128), (160, 16, 2, 256)])
 def test_dense_attention_of_scores_far_below_zero(gpu, rows, heads, kv_heads, dim):
     # scores of -1e31 and beyond: the highest a row sees still takes all the weight (they lie a 200th apart, FP32 tells them apart)
     rng = np.random.default_rng(rows + dim)
