@@ -357,7 +357,8 @@ __device__ __forceinline__ void choose_blocks(SelectShared& sh, Each each_run, B
 // sweeps 60K values.  Their scores' kernel leaves the highest score of each sixteen neighbouring blocks: the 512th highest of those is reached by 512
 // scores, and little more (some 550 of 60K in no order), so it is a bound that only its own sixteens have to be read for.  Where neighbours are alike whole sixteens reach it, up to 16K scores: more
 // than the list holds, they are read again for each step of the choice (a row of 32768 blocks alike over sixteen 17.5 us; swept, with the attempt, 38; not alike 12.9).
-// Writes the row's entries; false, and nothing written: many scores are equal, the row's workgroup sweeps the row itself.  (Thirty-two workgroups a row that each found
+// Writes the row's entries; false, and nothing written: many scores are equal, the row's workgroup sweeps the row itself, as it does below 8192 blocks, whose sixteens are
+// fewer than the bound is asked of (a decode row's whole stage at 20K tokens 40.0 us, at 33K 34.4).  (Thirty-two workgroups a row that each found
 // a bound from the same sample of it and listed their stretch took a launch of 10 us; a decode row's whole stage at 242K tokens 52.4 us with them, 38.7 now.)
 constexpr int MAXIMA_EACH = (65536 / SIXTEENS + SELECT_THREADS) / SELECT_THREADS;
 __device__ __forceinline__ bool select_by_maxima(SelectShared& sh, const uint32_t (&top)[MAXIMA_EACH], const float* row, uint32_t complete, float* out) {
