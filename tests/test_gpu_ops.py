@@ -693,7 +693,7 @@ def test_latent_rows_on_the_matrix_cores(gpu, oracle, rows, heads, window, raw_r
 
 
 @pytest.mark.parametrize("rows,heads,kv_heads,dim,context", [(1, 16, 2, 256, 4200), (1, 4, 4, 128, 33), (2, 16, 1, 128, 1000), (5, 24, 2, 256, 96), (33, 16, 2, 128, 700),
-                                                             (70, 16, 2, 256, 300), (300, 16, 4, 128, 400), (1, 1, 1, 256, 1),
+                                                             (70, 16, 2, 256, 300), (140, 16, 2, 256, 300), (300, 16, 4, 128, 400), (1, 1, 1, 256, 1),
                                                              (33, 1, 1, 128, 150), (5, 16, 2, 128, 900), (7, 9, 1, 128, 64), (4, 32, 2, 128, 333), (13, 10, 2, 128, 200)])
 def test_dense_attention_on_the_matrix_cores(gpu, oracle, rows, heads, kv_heads, dim, context):
     # 128 and 256 columns: one and two tiles of 32 query rows, runs of keys merged or one run finished in place, rows that see one key and
